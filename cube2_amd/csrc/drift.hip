@@ -1,162 +1,213 @@
 // Drift of one image on the device (drift.f90:1-158, spine_image of
 // variables.f90:146-216): from the image with halo copies to the new
 // physical-only image.
-//   keys     a wavefront per extended cell of every tile moves each slot by
-//            dt_mid*vp (the reference's FP32/FP64 mix): target cell
-//            ceiling(xq + deltax), new int16 code xp + nint(dt_mid*vp /
-//            (x_resolution*ratio_cs)) (wrapping).  A slot whose target is a
-//            physical cell of the same tile gets the key (tile, cell, layer
-//            of its source z), the others a key past every valid one;
-//   sort     stable radix sort (sort.hip) of (key, slot): within a target cell the
+//   keys     every slot moves by dt_mid*vp (the reference's FP32/FP64 mix):
+//            target cell ceiling(xq + deltax), new int16 code xp +
+//            nint(dt_mid*vp / (x_resolution*ratio_cs)) (wrapping).  Of the
+//            slots (halo copies included) only those whose target is a
+//            physical cell of the same tile stay, a fifth of them at 256^3:
+//            a first pass counts them per block of 1024 slots (slots.h), a
+//            second one writes, in slot order, their key (tile, cell, layer
+//            of the source z), slot and new code;
+//   sort     stable radix sort (sort.hip) of (key, entry): within a target cell the
 //            particles come by source layer, then in slot order (source z,
 //            y, x, slot), the arrival order of the layered loop
 //            drift.f90:36-62, 90-122 (one source z per layer can reach a
 //            cell when |dz| <= (nlayer-2)/2, which the kernel checks);
 //   counts   run boundaries of the sorted cells give the new rhoc (halo
 //            cells 0), a row scan gives idx_b_r;
-//   gather   xp, vp of the kept slots in sorted order.
+//   gather   codes and velocities of the kept slots in sorted order.
+// At 256^3 (90 M slots, 16.7 M kept) the two key passes take 0.67 and 0.30 ms
+// (18 bytes a slot: 2.4 TB/s) and the sort 0.9 ms; a wavefront per cell that
+// wrote and sorted every slot took 5.9 and 3.3 ms.
+#include <algorithm>
 #include <cstring>
 
 #include "common.h"
 #include "engine.h"
 #include "profile.h"
 #include "scan.h"
+#include "slots.h"
 #include "sort.h"
 
 namespace cube2 {
 
 struct DriftState {
-    DevBuf key, key_sorted, val, val_sorted, xpn, sort_tmp, bounds, rows, scan_tmp, red;
+    DevBuf start, kept, key, key_sorted, val, val_sorted, slot, xpn, sort_tmp, bounds, rows,
+        scan_tmp, red;
     HostBuf h_red;
 };
 static DriftState g_dr;
 
 struct DriftArgs {
-    const int* rhoc;
+    SlotGeom G;
+    const int* start;  // running slot counts of the extended cells
     const int64_t* idx_b_r;
     const int16_t* xp;
     const float* vp;
     int64_t n_used;
-    int nt, ncb, nte, nnt, ratio_cs, nlayer;
+    int ratio_cs, nlayer;
     float dt_mid;
-    uint32_t key_none;  // key of a slot that leaves the tile
 };
 
-// red[0]: kept slots; red[1]: error bits (1: slot range, 2: moved beyond ncb
-// cells, 4: |dz| beyond the layer spacing).
-__global__ __launch_bounds__(256) void k_drift_keys(DriftArgs A, uint32_t* __restrict__ key,
-                                                    uint32_t* __restrict__ val,
-                                                    int16_t* __restrict__ xpn,
-                                                    unsigned long long* __restrict__ red) {
+// err bits: 1 slot range, 2 moved beyond ncb cells, 4 |dz| beyond the layer
+// spacing.  kEmit false: kept[block] = the block's kept slots, and the
+// checks.  kEmit true: kept[] holds the exclusive scan of those counts; the
+// kept slots' keys, entry numbers, slots and codes are written in slot order
+// (a wavefront takes 256 consecutive slots; blocks that keep none, most of
+// the halo, end at once).  kPow2: ratio_cs is a power of two, so that its
+// divisions are multiplications by the exact reciprocal (the same real
+// number, the same rounding).
+template <bool kEmit, bool kPow2>
+__global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
+    DriftArgs A, int* __restrict__ kept, uint32_t* __restrict__ key, uint32_t* __restrict__ val,
+    uint32_t* __restrict__ slot, int16_t* __restrict__ xpn, unsigned* __restrict__ err) {
 #pragma clang fp contract(off)
+    __shared__ int win[kSlotWin + 1];
+    __shared__ int wsum[kSlotThreads / 64];
+    const SlotGeom& G = A.G;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t q = (int64_t)blockIdx.x * 4 + wave;  // extended cell of the image
-    const int64_t te3 = (int64_t)A.nte * A.nte * A.nte;
-    if (q >= te3 * A.nnt * A.nnt * A.nnt) return;
-    const int t = (int)(q / te3);
-    const int r = (int)(q - (int64_t)t * te3);
-    const int i = r % A.nte, j = (r / A.nte) % A.nte, k = r / (A.nte * A.nte);
-    const int np = A.rhoc[q];
-    if (np <= 0) return;
-    // nzero = row end - sum(rhoc(i:)) of the row
-    const int64_t row = (int64_t)t * A.nte * A.nte + (int64_t)k * A.nte + j;
-    const int* rrow = A.rhoc + (q - i);
-    int64_t suf = 0;
-    for (int a = i; a < A.nte; a++) suf += rrow[a];
-    const int64_t nzero = A.idx_b_r[row] - suf;
-    if (nzero < 0 || nzero + np > A.n_used) {
-        if (lane == 0) atomicOr(&red[1], 1ull);
+    const int total = A.start[G.ncells];
+    if (total < 0 || total > A.n_used) {
+        if (!kEmit && threadIdx.x == 0) {
+            kept[blockIdx.x] = 0;
+            if (blockIdx.x == 0) atomicOr(err, 1u);
+        }
         return;
     }
-    const int src[3] = {i, j, k};
+    int out = 0;
+    if (kEmit) {
+        out = kept[blockIdx.x];
+        if (kept[blockIdx.x + 1] == out) return;
+    }
+    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
     const int dmax = (A.nlayer - 2) / 2;
-    unsigned long long bad = 0;
-    int kept = 0;
-    for (int l = lane; l < np; l += 64) {
-        const int64_t ip = nzero + l;
-        int ig[3];
-        int16_t code[3];
+    const float rf = (float)A.ratio_cs, irf = 1.0f / rf;
+    const double rd = 1.0 / 65536.0 * (double)A.ratio_cs, ird = 1.0 / rd;
+    unsigned bad = 0;
+    int mine = 0;  // kept slots of the wavefront's windows
+    constexpr int kIt = kSlotChunk / kSlotThreads;
+    walk_slots(A.start, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+        uint32_t kk[kIt], ss[kIt];
+        int16_t code[kIt][3];
+        uint64_t km[kIt];
+        int n = 0;
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const int16_t v = A.xp[3 * ip + d];
-            const double xq = (double)(src[d] - A.ncb) + frac16(v);  // (cell - 1) + frac
-            const float f = A.dt_mid * A.vp[3 * ip + d];              // FP32 product
-            const double deltax = (double)(f / (float)A.ratio_cs);    // FP32 quotient
-            const int c = (int)ceil(xq + deltax);                     // 1-based target cell
-            ig[d] = c - 1;                                            // 0-based physical index
-            const int moved = ig[d] - (src[d] - A.ncb);
-            if (moved > A.ncb || moved < -A.ncb) bad |= 2ull;
-            if (d == 2 && (moved > dmax || moved < -dmax)) bad |= 4ull;
-            const double sh = (double)f / (1.0 / 65536.0 * (double)A.ratio_cs);
-            const long long m = llround(sh);
-            code[d] = (int16_t)(uint16_t)(uint32_t)((long long)v + m);
-        }
-        const bool keep = ig[0] >= 0 && ig[0] < A.nt && ig[1] >= 0 && ig[1] < A.nt && ig[2] >= 0 &&
-                          ig[2] < A.nt;
-        uint32_t kk = A.key_none;
-        if (keep) {
-            const uint32_t cell = (uint32_t)(((int64_t)t * A.nt + ig[2]) * A.nt + ig[1]) * A.nt + ig[0];
-            kk = cell * (uint32_t)A.nlayer + (uint32_t)(k % A.nlayer);
-            kept++;
-        }
-        key[ip] = kk;
-        val[ip] = (uint32_t)ip;
+        for (int it = 0; it < kIt; it++) {
+            const int v = b + (wave * kIt + it) * 64 + lane;
+            bool keep = false;
+            if (v < e) {
+                int s0, s1;
+                const CellPos c = cell_pos(G, cell_of(v, s0, s1));
+                const int64_t sh = row_shift(A.start, A.idx_b_r, c.row, G.nte.d);
+                if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > A.n_used) {
+                    bad |= 1u;
+                } else {
+                    const int64_t ip = v + sh;
+                    const int src[3] = {c.i, c.j, c.k};
+                    int ig[3];
+                    float f[3];
+                    int16_t x[3];
 #pragma unroll
-        for (int d = 0; d < 3; d++) xpn[3 * ip + d] = code[d];
+                    for (int d = 0; d < 3; d++) {
+                        x[d] = A.xp[3 * ip + d];
+                        f[d] = A.dt_mid * A.vp[3 * ip + d];  // FP32 product
+                    }
+                    keep = true;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        const double xq = (double)(src[d] - G.ncb) + frac16(x[d]);  // (cell - 1) + frac
+                        const double deltax = (double)(kPow2 ? f[d] * irf : f[d] / rf);  // FP32 quotient
+                        ig[d] = (int)ceil(xq + deltax) - 1;  // 0-based physical target cell
+                        const int moved = ig[d] - (src[d] - G.ncb);
+                        if (moved > G.ncb || moved < -G.ncb) bad |= 2u;
+                        if (d == 2 && (moved > dmax || moved < -dmax)) bad |= 4u;
+                        keep &= ig[d] >= 0 && ig[d] < G.nt;
+                    }
+                    if (kEmit && keep) {
+                        const uint32_t cell =
+                            (uint32_t)(((int64_t)c.tile * G.nt + ig[2]) * G.nt + ig[1]) * G.nt + ig[0];
+                        kk[it] = cell * (uint32_t)A.nlayer + (uint32_t)(c.k % A.nlayer);
+                        ss[it] = (uint32_t)ip;
+#pragma unroll
+                        for (int d = 0; d < 3; d++) {
+                            const double m = kPow2 ? (double)f[d] * ird : (double)f[d] / rd;
+                            code[it][d] = (int16_t)(uint16_t)(uint32_t)((long long)x[d] + llround(m));
+                        }
+                    }
+                }
+            }
+            km[it] = __ballot(keep);
+            n += __popcll(km[it]);
+        }
+        if (!kEmit) {
+            mine += n;
+        } else {
+            if (lane == 0) wsum[wave] = n;
+            __syncthreads();
+            int o = out;
+            for (int w = 0; w < kSlotThreads / 64; w++) {
+                if (w < wave) o += wsum[w];
+                out += wsum[w];
+            }
+            const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+#pragma unroll
+            for (int it = 0; it < kIt; it++) {
+                if (km[it] >> lane & 1) {
+                    const int64_t p = o + __popcll(km[it] & lt);
+                    key[p] = kk[it];
+                    val[p] = (uint32_t)p;
+                    slot[p] = ss[it];
+#pragma unroll
+                    for (int d = 0; d < 3; d++) xpn[3 * p + d] = code[it][d];
+                }
+                o += __popcll(km[it]);
+            }
+        }
+    });
+    if (!kEmit) {
+        if (lane == 0) wsum[wave] = mine;
+        __syncthreads();
+        if (threadIdx.x == 0) kept[blockIdx.x] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        if (bad) atomicOr(err, bad);
     }
-    // wavefront sums: one atomic per wavefront
-    for (int o = 32; o > 0; o >>= 1) kept += __shfl_xor(kept, o, 64);
-    bad |= __shfl_xor(bad, 32, 64);
-    for (int o = 16; o > 0; o >>= 1) bad |= __shfl_xor(bad, o, 64);
-    if (lane == 0) {
-        if (kept) atomicAdd(&red[0], (unsigned long long)kept);
-        if (bad) atomicOr(&red[1], bad);
-    }
-}
-
-__global__ void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
 }
 
 // Positions (standard cells, FP64, wrapped into [0, ng)) of every slot of
-// the image: a wavefront per extended cell.
-__global__ __launch_bounds__(256) void k_slot_positions(const int* __restrict__ rhoc,
-                                                        const int64_t* __restrict__ idx_b_r,
-                                                        const int16_t* __restrict__ xp,
-                                                        int64_t n_used, int nt, int ncb, int nte,
-                                                        int nnt, int ratio_cs,
-                                                        double* __restrict__ pos,
-                                                        unsigned long long* __restrict__ err) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int64_t q = (int64_t)blockIdx.x * 4 + wave;
-    const int64_t te3 = (int64_t)nte * nte * nte;
-    if (q >= te3 * nnt * nnt * nnt) return;
-    const int np = rhoc[q];
-    if (np <= 0) return;
-    const int t = (int)(q / te3);
-    const int r = (int)(q - (int64_t)t * te3);
-    const int i = r % nte, j = (r / nte) % nte, k = r / (nte * nte);
-    const int64_t row = (int64_t)t * nte * nte + (int64_t)k * nte + j;
-    int64_t suf = 0;
-    for (int a = i; a < nte; a++) suf += rhoc[q - i + a];
-    const int64_t nzero = idx_b_r[row] - suf;
-    if (nzero < 0 || nzero + np > n_used) {
-        if (lane == 0) atomicOr(err, 1ull);
+// the image: a block per kSlotChunk slots (16.7 M slots without halo copies:
+// 0.18 ms; a wavefront per cell 1.85 ms).
+__global__ __launch_bounds__(kSlotThreads) void k_slot_positions(
+    SlotGeom G, const int* __restrict__ start, const int64_t* __restrict__ idx_b_r,
+    const int16_t* __restrict__ xp, int64_t n_used, int ratio_cs, double* __restrict__ pos,
+    unsigned* __restrict__ err) {
+    __shared__ int win[kSlotWin + 1];
+    const int total = start[G.ncells];
+    if (total < 0 || total > n_used) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1u);
         return;
     }
-    const int nc = nt * nnt;
-    const int tc[3] = {t % nnt, (t / nnt) % nnt, t / (nnt * nnt)};
-    const int cc[3] = {i, j, k};
-    int gc[3];
+    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
+    unsigned bad = 0;
+    walk_slots(start, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+        for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
+            int s0, s1;
+            const CellPos c = cell_pos(G, cell_of(v, s0, s1));
+            const int64_t sh = row_shift(start, idx_b_r, c.row, G.nte.d);
+            if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > n_used) {
+                bad = 1u;
+                continue;
+            }
+            const int64_t ip = v + sh;
+            int tx, ty, tz;
+            tile_pos(G, c.tile, tx, ty, tz);
+            const int gc[3] = {image_coord(G, tx, c.i), image_coord(G, ty, c.j),
+                               image_coord(G, tz, c.k)};
 #pragma unroll
-    for (int d = 0; d < 3; d++) gc[d] = ((tc[d] * nt + cc[d] - ncb) % nc + nc) % nc;
-    for (int l = lane; l < np; l += 64) {
-        const int64_t ip = nzero + l;
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            pos[3 * ip + d] = ((double)gc[d] + frac16(xp[3 * ip + d])) * (double)ratio_cs;
-    }
+            for (int d = 0; d < 3; d++)
+                pos[3 * ip + d] = ((double)gc[d] + frac16(xp[3 * ip + d])) * (double)ratio_cs;
+        }
+    });
+    if (bad) atomicOr(err, bad);
 }
 
 // bounds[2c] / bounds[2c+1]: first / past-last sorted position of cell c.
@@ -200,14 +251,15 @@ __global__ void k_drift_rows(const int* __restrict__ rows, int64_t nrows, int64_
 }
 
 __global__ void k_drift_gather(const uint32_t* __restrict__ vs, int64_t n_kept,
+                               const uint32_t* __restrict__ slot,
                                const int16_t* __restrict__ xpn, const float* __restrict__ vp,
                                int16_t* __restrict__ xp_out, float* __restrict__ vp_out) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n_kept) return;
-    const int64_t s = vs[p];
+    const int64_t e = vs[p], s = slot[e];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        xp_out[3 * p + d] = xpn[3 * s + d];
+        xp_out[3 * p + d] = xpn[3 * e + d];
         vp_out[3 * p + d] = vp[3 * s + d];
     }
 }
@@ -239,52 +291,47 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
     }
     C2_TRY(ensure_init());
     hipStream_t s = C.stream;
-    const int64_t te3 = (int64_t)g.nte * g.nte * g.nte;
-    const int64_t ncells = te3 * g.ntile;
+    const int64_t ncells = (int64_t)g.nte * g.nte * g.nte * g.ntile;
+    if (ncells >= ((int64_t)1 << 31) || n_used >= ((int64_t)1 << 31) - kSlotChunk) {
+        set_error("drift: image too large for 32-bit slots");
+        return CUBE2_ERR_CAPACITY;
+    }
     const int64_t nrows = (int64_t)g.ntile * g.nte * g.nte;
-    const size_t nn = (size_t)std::max<int64_t>(n_used, 1);
-    C2_TRY(g_dr.key.reserve(nn * 4));
-    C2_TRY(g_dr.key_sorted.reserve(nn * 4));
-    C2_TRY(g_dr.val.reserve(nn * 4));
-    C2_TRY(g_dr.val_sorted.reserve(nn * 4));
-    C2_TRY(g_dr.xpn.reserve(nn * 6));
+    const int64_t nblk = std::max<int64_t>(1, (n_used + kSlotChunk - 1) / kSlotChunk);
+    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(int)));
+    C2_TRY(g_dr.kept.reserve((size_t)(nblk + 1) * sizeof(int)));
     C2_TRY(g_dr.bounds.reserve((size_t)(2 * ncell_phys) * sizeof(int)));
     C2_TRY(g_dr.rows.reserve((size_t)(nrows + 1) * sizeof(int)));
-    C2_TRY(g_dr.scan_tmp.reserve(scan_tmp_ints(nrows) * sizeof(int)));
-    C2_TRY(g_dr.red.reserve(2 * sizeof(unsigned long long)));
-    C2_TRY(g_dr.h_red.reserve(2 * sizeof(unsigned long long)));
-    const uint32_t key_none = (uint32_t)(ncell_phys * nlayer);
+    C2_TRY(g_dr.red.reserve(sizeof(unsigned)));
+    C2_TRY(g_dr.h_red.reserve(2 * sizeof(int)));
+    const uint32_t key_none = (uint32_t)(ncell_phys * nlayer);  // past every key
     unsigned end_bit = 1;
-    while (end_bit < 32 && ((uint64_t)1 << end_bit) <= key_none) end_bit++;
-    unsigned long long* red = g_dr.red.as<unsigned long long>();
-    C2_TRY(fill_zero(red, 2 * sizeof(unsigned long long), s));
-    if (n_used) {  // slots no cell names (an inconsistent layout) sort last
-        k_fill_u32<<<ceil_div(n_used, 256), 256, 0, s>>>(g_dr.key.as<uint32_t>(), n_used, 0xffffffffu);
-        C2_HIP(hipGetLastError());
-    }
+    while (end_bit < 32 && ((uint64_t)1 << end_bit) < key_none) end_bit++;
+    unsigned* err = g_dr.red.as<unsigned>();
+    C2_TRY(fill_zero(err, sizeof(unsigned), s));
+    DriftArgs A;
+    A.G = make_slotgeom(g);
+    A.start = g_dr.start.as<int>();
+    A.idx_b_r = d_idx_b_r;
+    A.xp = d_xp;
+    A.vp = d_vp;
+    A.n_used = n_used;
+    A.ratio_cs = g.p.ratio_cs;
+    A.nlayer = nlayer;
+    A.dt_mid = dt_mid;
+    const bool pow2 = (g.p.ratio_cs & (g.p.ratio_cs - 1)) == 0;
+    int* kept = g_dr.kept.as<int>();
+    int* h = g_dr.h_red.as<int>();
     {
-        Stage st("drift_keys", (double)n_used * (6 + 12 + 4 + 4 + 6));
-        DriftArgs A;
-        A.rhoc = d_rhoc;
-        A.idx_b_r = d_idx_b_r;
-        A.xp = d_xp;
-        A.vp = d_vp;
-        A.n_used = n_used;
-        A.nt = g.nt;
-        A.ncb = g.ncb;
-        A.nte = g.nte;
-        A.nnt = g.p.nnt;
-        A.ratio_cs = g.p.ratio_cs;
-        A.nlayer = nlayer;
-        A.dt_mid = dt_mid;
-        A.key_none = key_none;
-        k_drift_keys<<<ceil_div(ncells, 4), 256, 0, s>>>(A, g_dr.key.as<uint32_t>(),
-                                                         g_dr.val.as<uint32_t>(),
-                                                         g_dr.xpn.as<int16_t>(), red);
+        Stage st("drift_keys", (double)n_used * (6 + 12));
+        C2_TRY(exclusive_scan_counts(d_rhoc, g_dr.start.as<int>(), ncells, g_dr.scan_tmp, s));
+        auto kern = pow2 ? k_drift_keys<false, true> : k_drift_keys<false, false>;
+        kern<<<(unsigned)nblk, kSlotThreads, 0, s>>>(A, kept, nullptr, nullptr, nullptr, nullptr, err);
         C2_HIP(hipGetLastError());
+        C2_TRY(exclusive_scan(kept, nblk, g_dr.scan_tmp, s));
+        C2_HIP(hipMemcpyAsync(h, kept + nblk, sizeof(int), hipMemcpyDeviceToHost, s));
+        C2_HIP(hipMemcpyAsync(h + 1, err, sizeof(int), hipMemcpyDeviceToHost, s));
     }
-    unsigned long long* h = g_dr.h_red.as<unsigned long long>();
-    C2_HIP(hipMemcpyAsync(h, red, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     C2_HIP(hipStreamSynchronize(s));
     if (h[1]) {
         set_error(h[1] & 1 ? "drift: rhoc and idx_b_r describe slots outside [0, n_used)"
@@ -298,11 +345,27 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
         set_error("drift: %lld particles kept, capacity %lld", (long long)n_kept, (long long)cap);
         return CUBE2_ERR_CAPACITY;
     }
+    const size_t nn = (size_t)std::max<int64_t>(n_kept, 1);
+    C2_TRY(g_dr.key.reserve(nn * 4));
+    C2_TRY(g_dr.key_sorted.reserve(nn * 4));
+    C2_TRY(g_dr.val.reserve(nn * 4));
+    C2_TRY(g_dr.val_sorted.reserve(nn * 4));
+    C2_TRY(g_dr.slot.reserve(nn * 4));
+    C2_TRY(g_dr.xpn.reserve(nn * 6));
+    if (n_kept) {
+        Stage st("drift_emit", (double)n_kept * (2 * (6 + 4) + 12 + 4));
+        auto kern = pow2 ? k_drift_keys<true, true> : k_drift_keys<true, false>;
+        kern<<<(unsigned)nblk, kSlotThreads, 0, s>>>(A, kept, g_dr.key.as<uint32_t>(),
+                                                     g_dr.val.as<uint32_t>(),
+                                                     g_dr.slot.as<uint32_t>(),
+                                                     g_dr.xpn.as<int16_t>(), err);
+        C2_HIP(hipGetLastError());
+    }
     {
-        Stage st("drift_sort", (double)n_used * 16);
+        Stage st("drift_sort", (double)n_kept * 16);
         C2_TRY(radix_sort_pairs_u32(g_dr.key.as<uint32_t>(), g_dr.key_sorted.as<uint32_t>(),
                                     g_dr.val.as<uint32_t>(), g_dr.val_sorted.as<uint32_t>(),
-                                    n_used, (int)end_bit, g_dr.sort_tmp, g_dr.scan_tmp, s));
+                                    n_kept, (int)end_bit, g_dr.sort_tmp, g_dr.scan_tmp, s));
     }
     {
         Stage st("drift_cells", (double)n_kept * 4 + (double)ncells * 8);
@@ -324,7 +387,8 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
     if (n_kept) {
         Stage st("drift_gather", (double)n_kept * (4 + 2 * (6 + 12)));
         k_drift_gather<<<ceil_div(n_kept, 256), 256, 0, s>>>(g_dr.val_sorted.as<uint32_t>(),
-                                                             n_kept, g_dr.xpn.as<int16_t>(), d_vp,
+                                                             n_kept, g_dr.slot.as<uint32_t>(),
+                                                             g_dr.xpn.as<int16_t>(), d_vp,
                                                              d_xp_out, d_vp_out);
         C2_HIP(hipGetLastError());
     }
@@ -342,17 +406,23 @@ int slot_positions(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d
     }
     C2_TRY(ensure_init());
     hipStream_t s = C.stream;
-    C2_TRY(g_dr.red.reserve(2 * sizeof(unsigned long long)));
-    C2_TRY(g_dr.h_red.reserve(2 * sizeof(unsigned long long)));
-    unsigned long long* red = g_dr.red.as<unsigned long long>();
-    C2_TRY(fill_zero(red, 2 * sizeof(unsigned long long), s));
     const int64_t ncells = (int64_t)g.nte * g.nte * g.nte * g.ntile;
-    k_slot_positions<<<ceil_div(ncells, 4), 256, 0, s>>>(d_rhoc, d_idx_b_r, d_xp, n_used, g.nt,
-                                                         g.ncb, g.nte, g.p.nnt, g.p.ratio_cs, d_pos,
-                                                         red);
+    if (ncells >= ((int64_t)1 << 31) || n_used >= ((int64_t)1 << 31) - kSlotChunk) {
+        set_error("positions: image too large for 32-bit slots");
+        return CUBE2_ERR_CAPACITY;
+    }
+    C2_TRY(g_dr.red.reserve(sizeof(unsigned)));
+    C2_TRY(g_dr.h_red.reserve(2 * sizeof(int)));
+    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(int)));
+    unsigned* err = g_dr.red.as<unsigned>();
+    C2_TRY(fill_zero(err, sizeof(unsigned), s));
+    int* start = g_dr.start.as<int>();
+    C2_TRY(exclusive_scan_counts(d_rhoc, start, ncells, g_dr.scan_tmp, s));
+    k_slot_positions<<<ceil_div((size_t)std::max<int64_t>(n_used, 1), kSlotChunk), kSlotThreads, 0, s>>>(
+        make_slotgeom(g), start, d_idx_b_r, d_xp, n_used, g.p.ratio_cs, d_pos, err);
     C2_HIP(hipGetLastError());
-    unsigned long long* h = g_dr.h_red.as<unsigned long long>();
-    C2_HIP(hipMemcpyAsync(h, red, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    int* h = g_dr.h_red.as<int>();
+    C2_HIP(hipMemcpyAsync(h, err, sizeof(int), hipMemcpyDeviceToHost, s));
     C2_TRY(sync_and_flush());
     if (h[0]) {
         set_error("positions: rhoc and idx_b_r describe slots outside [0, n_used)");
@@ -363,7 +433,7 @@ int slot_positions(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d
 
 void drift_release() {
     DriftState& D = g_dr;
-    for (DevBuf* b : {&D.key, &D.key_sorted, &D.val, &D.val_sorted, &D.xpn, &D.sort_tmp,
+    for (DevBuf* b : {&D.start, &D.kept, &D.slot, &D.key, &D.key_sorted, &D.val, &D.val_sorted, &D.xpn, &D.sort_tmp,
                       &D.bounds, &D.rows, &D.scan_tmp, &D.red})
         b->release();
     D.h_red.release();

@@ -1,4 +1,6 @@
 // Device-wide exclusive prefix sum of int32 counts (cell lists).
+#include <climits>
+
 #include "common.h"
 #include "scan.h"
 
@@ -37,28 +39,30 @@ __device__ inline int block_exclusive_scan(int v, int* total) {
     return off + inc - v;
 }
 
+// lo: values below it count as lo (0 for counts from a caller, INT_MIN for none)
 __global__ __launch_bounds__(kScanThreads) void k_block_sums(const int* __restrict__ d, int64_t n,
-                                                             int* __restrict__ sums) {
+                                                             int lo, int* __restrict__ sums) {
     int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     int s = 0;
 #pragma unroll
     for (int q = 0; q < kScanItems; q++)
-        if (base + q < n) s += d[base + q];
+        if (base + q < n) s += max(d[base + q], lo);
     int tot;
     (void)block_exclusive_scan(s, &tot);
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// Exclusive scan of each tile, offset by offs[blockIdx.x] (nullptr: 0);
-// writes the grand total to d[n] from the last block.
-__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int* __restrict__ d, int64_t n,
-                                                             const int* __restrict__ offs) {
+// Exclusive scan of each tile of src into d (may be src), offset by
+// offs[blockIdx.x] (nullptr: 0); writes the grand total to d[n] from the last
+// block.
+__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const int* src, int* d, int64_t n,
+                                                             int lo, const int* __restrict__ offs) {
     int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     int v[kScanItems];
     int s = 0;
 #pragma unroll
     for (int q = 0; q < kScanItems; q++) {
-        v[q] = base + q < n ? d[base + q] : 0;
+        v[q] = base + q < n ? max(src[base + q], lo) : 0;
         s += v[q];
     }
     int tot;
@@ -73,18 +77,18 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(int* __restrict__ d
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanThreads - 1) d[n] = o + tot;
 }
 
-static int scan_rec(int* d, int64_t n, int* tmp, hipStream_t s) {
+static int scan_rec(const int* src, int* d, int64_t n, int lo, int* tmp, hipStream_t s) {
     const int64_t nb = (n + kScanTile - 1) / kScanTile;
     if (nb <= 1) {
-        k_scan_tiles<<<1, kScanThreads, 0, s>>>(d, n, nullptr);
+        k_scan_tiles<<<1, kScanThreads, 0, s>>>(src, d, n, lo, nullptr);
         C2_HIP(hipGetLastError());
         return CUBE2_OK;
     }
     int* sums = tmp;
-    k_block_sums<<<(unsigned)nb, kScanThreads, 0, s>>>(d, n, sums);
+    k_block_sums<<<(unsigned)nb, kScanThreads, 0, s>>>(src, n, lo, sums);
     C2_HIP(hipGetLastError());
-    C2_TRY(scan_rec(sums, nb, tmp + nb + 1, s));
-    k_scan_tiles<<<(unsigned)nb, kScanThreads, 0, s>>>(d, n, sums);
+    C2_TRY(scan_rec(sums, sums, nb, INT_MIN, tmp + nb + 1, s));
+    k_scan_tiles<<<(unsigned)nb, kScanThreads, 0, s>>>(src, d, n, lo, sums);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }
@@ -117,7 +121,13 @@ int fill_zero(void* d, size_t bytes, hipStream_t s) {
 int exclusive_scan(int* d, int64_t n, DevBuf& tmp, hipStream_t s) {
     if (n <= 0) return fill_zero(d, sizeof(int), s);
     C2_TRY(tmp.reserve(scan_tmp_ints(n) * sizeof(int)));
-    return scan_rec(d, n, tmp.as<int>(), s);
+    return scan_rec(d, d, n, INT_MIN, tmp.as<int>(), s);
+}
+
+int exclusive_scan_counts(const int* counts, int* d, int64_t n, DevBuf& tmp, hipStream_t s) {
+    if (n <= 0) return fill_zero(d, sizeof(int), s);
+    C2_TRY(tmp.reserve(scan_tmp_ints(n) * sizeof(int)));
+    return scan_rec(counts, d, n, 0, tmp.as<int>(), s);
 }
 
 }  // namespace cube2

@@ -1,8 +1,7 @@
 // Stable LSD radix sort of 32-bit (key, value) pairs: ceil(end_bit / 11)
 // passes of equal digit widths (at most 11 bits, 2048 digits).
 //
-// A pass splits the n pairs into kSortBlocks contiguous segments, one per
-// block.  k_sort_hist counts each segment's digits in LDS and stores the
+// A pass splits the n pairs into contiguous segments, one per block.  k_sort_hist counts each segment's digits in LDS and stores the
 // counts digit-major ([digit][block]), so that one exclusive scan of them
 // gives every (digit, block) its first output position: all pairs of a
 // smaller digit first, and within a digit the segments in order.  The
@@ -26,10 +25,14 @@ namespace cube2 {
 constexpr int kSortThreads = 256;
 constexpr int kSortMaxBits = 11;
 constexpr int kSortMaxBins = 1 << kSortMaxBits;
-constexpr int kSortBlocks = 1024;
+// Segments (blocks) of a pass: one per 2048 pairs, at most 1024.  The digit
+// counts to scan are bins x blocks, so that a short sort with 1024 blocks
+// spends its time on them.
+constexpr int kSortMaxBlocks = 1024;
+constexpr int kSortSegment = 2048;
 
 __device__ inline void sort_segment(int n, int& beg, int& end) {
-    const int seg = (n + kSortBlocks - 1) / kSortBlocks;
+    const int seg = (n + (int)gridDim.x - 1) / (int)gridDim.x;
     beg = min(n, (int)blockIdx.x * seg);
     end = min(n, beg + seg);
 }
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_hist(const uint32_t* __re
         if (valid && __popcll(peers & lt) == 0) atomicAdd(&h[d], __popcll(peers));
     }
     __syncthreads();
-    for (int q = t; q < nbin; q += kSortThreads) hist[q * kSortBlocks + blockIdx.x] = h[q];
+    for (int q = t; q < nbin; q += kSortThreads) hist[q * gridDim.x + blockIdx.x] = h[q];
 }
 
 __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const uint32_t* __restrict__ kin,
@@ -80,7 +83,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const uint32_t* _
     const int t = threadIdx.x, wave = t >> 6, lane = t & 63, nbin = 1 << bits;
     const uint32_t mask = (uint32_t)nbin - 1u;
     for (int q = t; q < nbin; q += kSortThreads) {
-        base[q] = hist[q * kSortBlocks + blockIdx.x];
+        base[q] = hist[q * gridDim.x + blockIdx.x];
         wc[0][q] = wc[1][q] = wc[2][q] = wc[3][q] = 0;
     }
     __syncthreads();
@@ -125,7 +128,8 @@ int radix_sort_pairs_u32(const uint32_t* kin, uint32_t* kout, const uint32_t* vi
     }
     const int passes = std::max(1, (end_bit + kSortMaxBits - 1) / kSortMaxBits);
     const int width = std::max(1, (end_bit + passes - 1) / passes);
-    const size_t nh = (size_t)kSortMaxBins * kSortBlocks + 1;
+    const int blocks = (int)std::min<int64_t>(kSortMaxBlocks, (n + kSortSegment - 1) / kSortSegment);
+    const size_t nh = (size_t)(1 << width) * blocks + 1;
     const size_t pair_bytes = ((size_t)n * 4 + 255) / 256 * 256;
     C2_TRY(tmp.reserve(2 * pair_bytes + nh * sizeof(int)));
     uint32_t* kt = tmp.as<uint32_t>();
@@ -142,10 +146,10 @@ int radix_sort_pairs_u32(const uint32_t* kin, uint32_t* kout, const uint32_t* vi
         // above end_bit are ignored
         const int shift = p * width;
         const int bits = std::max(1, std::min(width, end_bit - shift));
-        k_sort_hist<<<kSortBlocks, kSortThreads, 0, s>>>(ks, (int)n, shift, bits, hist);
+        k_sort_hist<<<blocks, kSortThreads, 0, s>>>(ks, (int)n, shift, bits, hist);
         C2_HIP(hipGetLastError());
-        C2_TRY(exclusive_scan(hist, (int64_t)(1 << bits) * kSortBlocks, scan_tmp, s));
-        k_sort_scatter<<<kSortBlocks, kSortThreads, 0, s>>>(ks, vs, (int)n, shift, bits, hist, kd,
+        C2_TRY(exclusive_scan(hist, (int64_t)(1 << bits) * blocks, scan_tmp, s));
+        k_sort_scatter<<<blocks, kSortThreads, 0, s>>>(ks, vs, (int)n, shift, bits, hist, kd,
                                                             vd);
         C2_HIP(hipGetLastError());
         ks = kd;

@@ -88,18 +88,20 @@ def build_layout_device(pos, vel, geom: Geometry):
     rhoc = torch.empty((geom.ntile, geom.nte, geom.nte, geom.nte), dtype=torch.int32, device=dev)
     idx = torch.empty((geom.ntile, geom.nte, geom.nte), dtype=torch.int64, device=dev)
     n_used = C.c_int64(0)
-    L = _lib.lib()
-    rc = L.cube2_layout_build_dev(d_pos.data_ptr(), None if d_vel is None else d_vel.data_ptr(), n,
-                                  rhoc.data_ptr(), idx.data_ptr(), None, None, 0,
-                                  C.byref(n_used))
-    if rc not in (_lib.OK, _lib.ERR_CAPACITY):
-        _lib.check(rc)
-    m = max(n_used.value, 1)
-    xp = torch.empty((m, 3), dtype=torch.int16, device=dev)
-    vp = torch.empty((m, 3), dtype=torch.float32, device=dev)
-    _lib.check(L.cube2_layout_build_dev(d_pos.data_ptr(), None if d_vel is None else d_vel.data_ptr(),
-                                        n, rhoc.data_ptr(), idx.data_ptr(), xp.data_ptr(),
-                                        vp.data_ptr(), m, C.byref(n_used)))
+    # one call where the slots fit an eighth over the mean density's (the
+    # sort and the cell counts run once); a second, sized by the first, where
+    # clumps in the halos need more
+    m = n * geom.nte ** 3 // geom.nt ** 3 * 9 // 8 + 4096
+    for _ in range(2):
+        xp = torch.empty((m, 3), dtype=torch.int16, device=dev)
+        vp = torch.empty((m, 3), dtype=torch.float32, device=dev)
+        rc = _lib.lib().cube2_layout_build_dev(
+            d_pos.data_ptr(), None if d_vel is None else d_vel.data_ptr(), n, rhoc.data_ptr(),
+            idx.data_ptr(), xp.data_ptr(), vp.data_ptr(), m, C.byref(n_used))
+        if rc != _lib.ERR_CAPACITY or n_used.value <= m:
+            break
+        m = n_used.value
+    _lib.check(rc)
     k = n_used.value
     return rhoc, idx, xp[:k], vp[:k], k
 
