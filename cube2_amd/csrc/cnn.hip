@@ -10,6 +10,9 @@
 // 0..3; B column n0 + (lane % 16), the same K values; result lane holds rows
 // 4 (lane / 16) + 0..3 of column lane % 16.  Out-of-range operands are
 // zeros, so any M, N, K work.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "engine.h"
 
@@ -230,160 +233,352 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ out,
 // (channels-last), on v_mfma_f32_16x16x32_bf16 (BF16 operands, FP32
 // accumulation) with no materialised im2col.
 //
-// A workgroup (4 wavefronts) is persistent over output blocks of
-// 4 (x) x 4 (y) x 8 (z) positions.  For each block it stages the 6 x 6 x 10
-// input cells as BF16 in LDS; wavefront w computes the z-planes 2w and 2w+1
-// (two 16-row tiles, the 4 x 4 positions of a plane) against every output
-// column.  The packed weights Wp[tap][out][in] (BF16) are loaded into LDS
-// once per workgroup.  MFMA operands: lane l holds row (position) l % 16 of
-// A and column (output channel) l % 16 of B with K indices 8 (l / 16) + 0..7;
-// the result lane holds rows 4 (l / 16) + 0..3 of column l % 16.  K runs over
-// (tap, channel) with the channel fastest: for CIN = 32 one K step is one
-// tap; for CIN = 4 a step is 8 taps (taps 27..31 are zeros).
+// MFMA operands: lane l holds row (output channel) l % 16 of A and column
+// (position) l % 16 of B with K indices 8 (l / 16) + 0..7; the result lane
+// holds channels 4 (l / 16) + 0..3 of position l % 16, so that its store is
+// one 16-byte (BF16: 8-byte) access.  K runs over (tap, channel) with the
+// channel fastest: for CIN = 32 one K step is one tap; for CIN = 4 a step is
+// 8 taps (taps 27..31 are zeros).
+//
+// The 16 positions of a tile are tx (16, 8 or 4) consecutive x of 16 / tx
+// grids, whichever wastes the fewest positions (conv_tile): subtile grids of
+// 72^3 outputs divide by 8, training patches have 8^3, 6^3, 4^3 and 2^3.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
-constexpr int kConvBx = 4, kConvBy = 4, kConvBz = 8;
-constexpr int kConvIx = kConvBx + 2, kConvIy = kConvBy + 2, kConvIz = kConvBz + 2;
-constexpr int kConvCells = kConvIx * kConvIy * kConvIz;  // 360 staged input cells
+struct ConvTile {
+    int tx;   // consecutive x of a tile (16, 8, 4); 16 / tx grids side by side
+    int nx, ny, nz, nb;  // tiles along x, rows of tiles, z chunks, groups of grids
+    int zc;   // output planes of a z chunk
+};
 
-template <int CIN>
-constexpr int conv_taps_padded() { return CIN == 32 ? 27 : 32; }
-
-template <int CIN, int COUTP>
-constexpr size_t conv_lds_bytes() {
-    return (size_t)conv_taps_padded<CIN>() * COUTP * CIN * 2 + (size_t)kConvCells * CIN * 2;
+// 16 bytes of BF16 channels from 8 values of the input.
+__device__ inline v8bf load_bf16x8(const uint16_t* p) { return *reinterpret_cast<const v8bf*>(p); }
+__device__ inline v8bf load_bf16x8(const float* p) {
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    return v8bf{(__bf16)a.x, (__bf16)a.y, (__bf16)a.z, (__bf16)a.w,
+                (__bf16)b.x, (__bf16)b.y, (__bf16)b.z, (__bf16)b.w};
 }
 
-__device__ inline float bf16_to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
+// The output channel in MFMA row r (0..15) of row tile ct.  BF16 outputs: a
+// lane's two result tiles are then 8 consecutive channels, 16 bytes.
+template <class TOut>
+__device__ inline int conv_channel(int ct, int r) {
+    return sizeof(TOut) == 2 ? 8 * (r >> 2) + 4 * ct + (r & 3) : ct * 16 + r;
+}
 
-template <class T>
-__device__ inline float load_f32(const T* p);
-template <>
-__device__ inline float load_f32<float>(const float* p) { return *p; }
-template <>
-__device__ inline float load_f32<uint16_t>(const uint16_t* p) { return bf16_to_f32(*p); }
+// Stores a lane's two result tiles at its position's channels.
+__device__ inline void store32(uint16_t* row, int kq, const v4f& u, const v4f& v) {
+    *reinterpret_cast<v8bf*>(row + 8 * kq) =
+        v8bf{(__bf16)u[0], (__bf16)u[1], (__bf16)u[2], (__bf16)u[3],
+             (__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+}
+__device__ inline void store32(float* row, int kq, const v4f& u, const v4f& v) {
+    *reinterpret_cast<v4f*>(row + 4 * kq) = u;
+    *reinterpret_cast<v4f*>(row + 16 + 4 * kq) = v;
+}
 
-template <class T>
-__device__ inline void store_act(T* p, float v);
-template <>
-__device__ inline void store_act<float>(float* p, float v) { *p = v; }
-template <>
-__device__ inline void store_act<uint16_t>(uint16_t* p, float v) { *p = to_bf16(v); }
+// 32 input channels.  A wavefront owns 4 rows of tiles (4 y of tx x) and
+// marches along a chunk of z: the input plane's 6 rows are read into
+// registers once for the 27 taps and 4 output rows that use them, against
+// accumulators of the three output planes in progress.  Weights (55 KB) are in
+// LDS for the workgroup's life, a fragment read there feeds 4 MFMAs (half
+// of LDS's rate); the next plane's cells are fetched during this plane's
+// MFMAs, converted, and put into the wavefront's own LDS buffer, so that
+// wavefronts never wait for each other.  LDS rows of 64 bytes are swizzled
+// in 16-byte units by (row / 4) % 4: the 16 rows a quarter wavefront reads lie
+// in distinct banks.  Each accumulator takes its taps in the order 0..26.
+// 8 wavefronts of up to 256 VGPRs fill a CU.  8 grids of 72^3 FP32 inputs:
+// 235 and 205 us for the two 32 -> 32 layers (0.73 and 0.67 GB, 3.2 TB/s; 670
+// TFLOP/s) and 111 us for 32 -> 3; a workgroup with one staged block of 4 x 4 x
+// 8 outputs, every fragment read from LDS for each 2 MFMAs, took 666, 536 and
+// 318 us.
+constexpr int kConvWaves = 8;
+constexpr int kConvRows = 4;                   // output rows of a wavefront
+constexpr int kConvIn = kConvRows + 2;         // staged rows of a wavefront
+constexpr int kConvRow = 32 * 4;               // a staged row: 32 cells of 4 16-byte parts
+constexpr int kConvItems = kConvIn + 3;        // 16-byte items a lane stages
 
-template <int CIN, int COUTP, class TIn, class TOut>
-__global__ __launch_bounds__(256) void k_conv3(const TIn* __restrict__ X,
-                                               const uint16_t* __restrict__ Wp,
-                                               const float* __restrict__ bias,
-                                               TOut* __restrict__ Y, int B, int D, int cout,
-                                               int relu) {
-    extern __shared__ __align__(16) uint16_t conv_lds[];
-    constexpr int TAPS = conv_taps_padded<CIN>();
-    uint16_t* wl = conv_lds;                         // [TAPS][COUTP][CIN]
-    uint16_t* xl = conv_lds + TAPS * COUTP * CIN;    // [cell][CIN]
+// In 16-byte units: part kq of weight row (channel) r, and of cell x of grid
+// g of a staged row (16 / tx grids of tx + 2 cells; gs cells from one to the
+// next).
+__device__ inline int conv_w_addr(int r, int kq) { return r * 4 + (kq ^ ((r >> 2) & 3)); }
+__device__ inline int conv_x_addr(int tx, int g, int x, int kq) {
+    const int gs = tx == 8 ? 16 : 8, turn = tx == 8 ? 2 * g : g;  // (tx 16: g = 0)
+    return (g * gs + x) * 4 + (kq ^ (((x >> 2) + turn) & 3));
+}
+
+template <int NT>
+constexpr size_t conv_lds_bytes() {
+    return (size_t)27 * NT * 16 * 64 + (size_t)kConvWaves * kConvIn * kConvRow * 16;
+}
+
+template <int NT, class TIn, class TOut>
+__global__ __launch_bounds__(kConvWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_conv3(
+    const TIn* __restrict__ X, const uint16_t* __restrict__ Wp, const float* __restrict__ bias,
+    TOut* __restrict__ Y, int B, int D, int cout, int relu, ConvTile T) {
+    extern __shared__ __align__(16) uint4 conv_lds[];
+    uint4* wl = conv_lds;  // [tap][NT*16 channels][32], swizzled
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    {
-        const uint4* src = reinterpret_cast<const uint4*>(Wp);
-        uint4* dst = reinterpret_cast<uint4*>(wl);
-        for (int i = tid; i < TAPS * COUTP * CIN / 8; i += 256) dst[i] = src[i];
+    uint4* xl = conv_lds + 27 * NT * 64 + wave * kConvIn * kConvRow;
+    for (int i = tid; i < 27 * NT * 64; i += kConvWaves * 64) {
+        const int r = i >> 2, row = r % (NT * 16);
+        wl[conv_w_addr(r, i & 3)] = reinterpret_cast<const uint4*>(
+            Wp)[(r - row + conv_channel<TOut>(row >> 4, row & 15)) * 4 + (i & 3)];
     }
-    const int P = D - 2;
-    const int nbx = (P + kConvBx - 1) / kConvBx, nby = (P + kConvBy - 1) / kConvBy,
-              nbz = (P + kConvBz - 1) / kConvBz;
-    const int64_t per = (int64_t)nbx * nby * nbz, nblk = per * B;
-    const int r16 = lane & 15, kq = lane >> 4;
-    for (int64_t blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
-        const int b = (int)(blk / per);
-        const int64_t rr = blk - (int64_t)b * per;
-        const int bx = (int)(rr % nbx), by = (int)((rr / nbx) % nby), bz = (int)(rr / ((int64_t)nbx * nby));
-        const int x0 = bx * kConvBx, y0 = by * kConvBy, z0 = bz * kConvBz;
-        __syncthreads();  // the previous block's reads of xl are done (and wl is loaded)
-        // stage the input cells as BF16 (zeros outside the grid), 4 channels per item
-        for (int i = tid; i < kConvCells * (CIN / 4); i += 256) {
-            const int cell = i / (CIN / 4), q = i % (CIN / 4);
-            const int cx = cell % kConvIx, cy = (cell / kConvIx) % kConvIy, cz = cell / (kConvIx * kConvIy);
-            const int gx = x0 + cx, gy = y0 + cy, gz = z0 + cz;
-            uint16_t h[4] = {0, 0, 0, 0};
-            if (gx < D && gy < D && gz < D) {
-                const TIn* src = X + ((((int64_t)b * D + gz) * D + gy) * D + gx) * CIN + 4 * q;
+    __syncthreads();
+    const int P = D - 2, r16 = lane & 15, kq = lane >> 4;
+    const int ng = 16 / T.tx, rs = T.tx + 2;
+    const int xs = r16 % T.tx, gi = r16 / T.tx;  // the lane's position
+    int xa[3];                                   // its cells' addresses in a staged row
 #pragma unroll
-                for (int j = 0; j < 4; j++) h[j] = to_bf16(load_f32<TIn>(src + j));
-            }
-            uint2 v;
-            v.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
-            v.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
-            *reinterpret_cast<uint2*>(xl + cell * CIN + 4 * q) = v;
+    for (int dx = 0; dx < 3; dx++) xa[dx] = conv_x_addr(T.tx, gi, xs + dx, kq);
+    const int wa = conv_w_addr(r16, kq);
+    // A row is ng * rs * 4 items of 16 bytes (72, 80 or 96): the first 64 are
+    // one per lane, the rest of the 6 rows fill up to three more steps.
+    const int rest = ng * rs * 4 - 64;
+    int scell[4], srow[4], dst[4];  // [0]: the main step (row added per row)
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const int e = (m - 1) * 64 + lane;
+        srow[m] = m ? min(e / rest, kConvIn - 1) : 0;
+        const int i = m ? 64 + e % rest : lane;
+        const int g = (i >> 2) / rs, x = (i >> 2) - g * rs;
+        scell[m] = g * 64 + x;  // (x < 18)
+        dst[m] = srow[m] * kConvRow + conv_x_addr(T.tx, g, x, i & 3);
+    }
+    const uint32_t items = (uint32_t)T.nb * T.nx * T.ny * T.nz;
+    // (neighbouring items share input rows: one XCD takes a run of them)
+    for (uint32_t it = xcd_remap(blockIdx.x, gridDim.x) * kConvWaves + wave; it < items;
+         it += gridDim.x * kConvWaves) {
+        uint32_t q = it;
+        const int ix = (int)(q % T.nx);
+        q /= T.nx;
+        const int iy = (int)(q % T.ny);
+        q /= T.ny;
+        const int iz = (int)(q % T.nz), b0 = (int)(q / T.nz) * ng;
+        const int x0 = ix * T.tx, y0 = iy * kConvRows, z0 = iz * T.zc;
+        const int nz = min(T.zc, P - z0);  // output planes of the chunk
+        // staged items' places in the input plane (cells past the grid repeat
+        // its last ones; they reach only positions that are not stored)
+        int src[4];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const int gb = min(scell[m] >> 6, B - 1 - b0), gx = min(x0 + (scell[m] & 63), D - 1);
+            const int gy = m ? min(y0 + srow[m], D - 1) : 0;
+            src[m] = ((gb * D * D + gy) * D + gx) * 32 + (lane & 3) * 8;
         }
-        __syncthreads();
-        v4f acc[2][COUTP / 16];
+        const TIn* Xp = X + ((int64_t)b0 * D + z0) * D * D * 32;
+        auto item = [&](int k) {
+            if (k < kConvIn) return load_bf16x8(Xp + (int64_t)min(y0 + k, D - 1) * D * 32 + src[0]);
+            return load_bf16x8(Xp + src[k - kConvIn + 1]);
+        };
+        v4f acc[3][kConvRows][NT];
+        v8bf nxt[kConvItems];
+        auto stage = [&]() {
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int rt = 0; rt < 2; rt++)
+            for (int k = 0; k < kConvItems; k++)
+                *reinterpret_cast<v8bf*>(xl + (k < kConvIn ? k * kConvRow + dst[0] : dst[k - kConvIn + 1])) = nxt[k];
+            __builtin_amdgcn_wave_barrier();
+        };
 #pragma unroll
-            for (int ct = 0; ct < COUTP / 16; ct++) acc[rt][ct] = v4f{0.f, 0.f, 0.f, 0.f};
-        const int xr = r16 & 3, yr = r16 >> 2;
-        constexpr int STEPS = TAPS * CIN / 32;
-        for (int s = 0; s < STEPS; s++) {
-            v8bf a[2], bm[COUTP / 16];
-            if (CIN == 32) {
-                const int t = s, dz = t / 9, dy = (t / 3) % 3, dx = t % 3;
+        for (int k = 0; k < kConvItems; k++) nxt[k] = item(k);
+        stage();
+        // Input plane zz of the chunk (R = zz % 3): tap plane dz of output
+        // plane zz - dz, accumulated in slot (R - dz) mod 3.
+        auto plane = [&](auto r_c, int zz) {
+            constexpr int R = decltype(r_c)::value;
+            Xp += (int64_t)D * D * 32;
+            const bool more = zz + 1 < nz + 2;
 #pragma unroll
-                for (int rt = 0; rt < 2; rt++) {
-                    const int zl = 2 * wave + rt;
-                    const int cell = ((zl + dz) * kConvIy + yr + dy) * kConvIx + xr + dx;
-                    a[rt] = *reinterpret_cast<const v8bf*>(xl + cell * CIN + 8 * kq);
+            for (int y = 0; y < kConvRows; y++)
+#pragma unroll
+                for (int ct = 0; ct < NT; ct++) acc[R][y][ct] = v4f{0.f, 0.f, 0.f, 0.f};
+            v8bf a[kConvRows + 2][3];
+            auto row = [&](int y) {
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++)
+                    a[y][dx] = *reinterpret_cast<const v8bf*>(xl + y * kConvRow + xa[dx]);
+            };
+#pragma unroll
+            for (int y = 0; y < kConvRows - 1; y++) row(y);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++) {
+                row(kConvRows - 1 + dy);
+                if (more) {  // a third of the next plane's items
+#pragma unroll
+                    for (int k = dy * kConvItems / 3; k < (dy + 1) * kConvItems / 3; k++)
+                        nxt[k] = item(k);
                 }
 #pragma unroll
-                for (int ct = 0; ct < COUTP / 16; ct++)
-                    bm[ct] = *reinterpret_cast<const v8bf*>(wl + ((t * COUTP + ct * 16 + r16) * CIN + 8 * kq));
-            } else {  // CIN == 4: taps 8s + 2kq and 8s + 2kq + 1, four channels each
+                for (int dz = 0; dz < 3; dz++) {
+                    const int o = zz - dz;
+                    if (o < 0 || o >= nz) continue;
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const int t = 8 * s + 2 * kq + h;
-                    const bool tv = t < 27;
-                    const int tt = tv ? t : 0;
-                    const int dz = tt / 9, dy = (tt / 3) % 3, dx = tt % 3;
+                    for (int dx = 0; dx < 3; dx++) {
+                        const int t = dz * 9 + dy * 3 + dx;
+                        v8bf w[NT];
 #pragma unroll
-                    for (int rt = 0; rt < 2; rt++) {
-                        const int zl = 2 * wave + rt;
-                        const int cell = ((zl + dz) * kConvIy + yr + dy) * kConvIx + xr + dx;
-                        v4bf q = *reinterpret_cast<const v4bf*>(xl + cell * CIN);
-                        if (!tv) q = v4bf{};
+                        for (int ct = 0; ct < NT; ct++)
+                            w[ct] = *reinterpret_cast<const v8bf*>(
+                                wl + (t * NT + ct) * 64 + wa);
 #pragma unroll
-                        for (int j = 0; j < 4; j++) a[rt][4 * h + j] = q[j];
-                    }
+                        for (int y = 0; y < kConvRows; y++)
 #pragma unroll
-                    for (int ct = 0; ct < COUTP / 16; ct++) {
-                        const v4bf q = *reinterpret_cast<const v4bf*>(wl + (t * COUTP + ct * 16 + r16) * CIN);
-#pragma unroll
-                        for (int j = 0; j < 4; j++) bm[ct][4 * h + j] = q[j];
+                            for (int ct = 0; ct < NT; ct++)
+                                acc[(R - dz + 3) % 3][y][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    w[ct], a[y + dy][dx], acc[(R - dz + 3) % 3][y][ct], 0, 0, 0);
                     }
                 }
             }
+            // The next plane goes to LDS before this one's stores: a wavefront's
+            // loads and stores complete in one order, so that waiting for
+            // loads after the stores would wait for the stores too.
+            if (more) stage();
+            if (zz >= 2) {  // output plane zz - 2 is complete
+                const int gz = z0 + zz - 2, gx = x0 + xs;
+                if (gx < P && b0 + gi < B) {
 #pragma unroll
-            for (int rt = 0; rt < 2; rt++)
+                    for (int y = 0; y < kConvRows; y++) {
+                        if (y0 + y >= P) continue;
+                        if (NT == 1 && kq > 0) continue;  // 3 channels
+                        TOut* out = Y + ((((int64_t)(b0 + gi) * P + gz) * P + y0 + y) * P + gx) * cout;
+                        v4f v[NT];
 #pragma unroll
-                for (int ct = 0; ct < COUTP / 16; ct++)
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bm[ct], acc[rt][ct], 0, 0, 0);
+                        for (int ct = 0; ct < NT; ct++)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                const int o = conv_channel<TOut>(ct, 4 * kq + i);
+                                v[ct][i] = acc[(R + 1) % 3][y][ct][i];
+                                if (NT == 2 || i < 3) v[ct][i] += bias[o];
+                                if (relu) v[ct][i] = fmaxf(v[ct][i], 0.f);
+                            }
+                        if constexpr (NT == 2) {
+                            store32(out, kq, v[0], v[1]);
+                        } else {
+                            out[0] = v[0][0];
+                            out[1] = v[0][1];
+                            out[2] = v[0][2];
+                        }
+                    }
+                }
+            }
+        };
+        for (int zz = 0; zz < nz + 2; zz += 3) {
+            plane(std::integral_constant<int, 0>{}, zz);
+            if (zz + 1 < nz + 2) plane(std::integral_constant<int, 1>{}, zz + 1);
+            if (zz + 2 < nz + 2) plane(std::integral_constant<int, 2>{}, zz + 2);
         }
-        // epilogue: bias, activation, store the valid positions and channels
+    }
+}
+
+// 4 input channels (FP32): a wavefront takes tiles (one row of 16 positions,
+// all 32 channels: 8 MFMAs) along kC4Rows rows of y, its weights in
+// registers.  The 3 x (kC4Rows + 2) input rows of the item are fetched at
+// once, converted and kept in the wavefront's own LDS; a lane reads its two
+// taps of a K step from there.  Bound by the stores of the 32 output channels
+// and the loads that queue behind them: 8 grids of 72^3 outputs (FP32, 382 MB)
+// take 140 us, 79 without the stores and 85 without the loads.  Rows of 8 and
+// the next item's loads ahead of the stores (more registers, fewer
+// wavefronts): 150 and 174 us; taps straight from the grid, eight scattered
+// loads a tile: 172.
+constexpr int kC4Rows = 4;
+constexpr int kC4Row = 24;                                  // staged cells of a row, at most
+constexpr int kC4Items = (3 * (kC4Rows + 2) * kC4Row + 63) / 64;  // cells a lane stages
+
+template <class TOut>
+__global__ __launch_bounds__(256, 4) void k_conv3_c4(const float* __restrict__ X,
+                                                  const uint16_t* __restrict__ Wp,
+                                                  const float* __restrict__ bias,
+                                                  TOut* __restrict__ Y, int B, int D, int relu,
+                                                  ConvTile T) {
+    __shared__ v4bf lds[4][kC4Items * 64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    v4bf* xl = lds[wave];
+    const int P = D - 2, r16 = lane & 15, kq = lane >> 4;
+    const int xs = r16 % T.tx, gi = r16 / T.tx, ng = 16 / T.tx;
+    const int rs = T.tx + 2, rc = ng * rs;  // cells of a grid's row, of a staged row
+    v8bf w[4][2];
+    int off[4][2];  // the lane's taps in the staged rows [dz][y][grid][x]
 #pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
-            const int gz = z0 + 2 * wave + rt;
+    for (int s = 0; s < 4; s++) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = 4 * kq + i;
-                const int gx = x0 + (r & 3), gy = y0 + (r >> 2);
-                if (gx >= P || gy >= P || gz >= P) continue;
-                TOut* out = Y + ((((int64_t)b * P + gz) * P + gy) * P + gx) * cout;
+        for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-                for (int ct = 0; ct < COUTP / 16; ct++) {
-                    const int o = ct * 16 + r16;
-                    if (o >= cout) continue;
-                    float v = acc[rt][ct][i] + bias[o];
-                    if (relu) v = fmaxf(v, 0.f);
-                    store_act<TOut>(out + o, v);
-                }
+            for (int h = 0; h < 2; h++) {
+                const v4bf q = *reinterpret_cast<const v4bf*>(
+                    Wp + ((8 * s + 2 * kq + h) * 32 + conv_channel<TOut>(ct, r16)) * 4);
+#pragma unroll
+                for (int j = 0; j < 4; j++) w[s][ct][4 * h + j] = q[j];
             }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int t = min(8 * s + 2 * kq + h, 26);
+            off[s][h] = (t / 9 * (kC4Rows + 2) + t / 3 % 3) * rc + gi * rs + xs + t % 3;
+        }
+    }
+    float bs[2][4];
+#pragma unroll
+    for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) bs[ct][i] = bias[conv_channel<TOut>(ct, 4 * kq + i)];
+    int cell[kC4Items];  // staged cell: dz << 20 | y << 16 | grid << 8 | x
+#pragma unroll
+    for (int k = 0; k < kC4Items; k++) {
+        const int e = k * 64 + lane, row = min(e / rc, 3 * (kC4Rows + 2) - 1), c = e % rc;
+        const int dz = row / (kC4Rows + 2);
+        cell[k] = dz << 20 | (row - dz * (kC4Rows + 2)) << 16 | c / rs << 8 | c % rs;
+    }
+    // (an item is 128 output positions or more: the count fits 32 bits)
+    const uint32_t nyc = (uint32_t)(P + kC4Rows - 1) / kC4Rows;
+    const uint32_t items = (uint32_t)T.nb * P * T.nx * nyc;
+    for (uint32_t it = xcd_remap(blockIdx.x, gridDim.x) * 4 + wave; it < items; it += gridDim.x * 4) {
+        uint32_t q = it;
+        const int x0 = (int)(q % T.nx) * T.tx;
+        q /= T.nx;
+        const int y0 = (int)(q % nyc) * kC4Rows;
+        q /= nyc;
+        const int gz = (int)(q % P), b0 = (int)(q / P) * ng;
+        const float4* Xi = reinterpret_cast<const float4*>(X) + ((int64_t)b0 * D + gz) * D * D;
+        float4 v[kC4Items];
+#pragma unroll
+        for (int k = 0; k < kC4Items; k++) {
+            const int dz = cell[k] >> 20, y = min(y0 + (cell[k] >> 16 & 15), D - 1),
+                      g = min(cell[k] >> 8 & 255, B - 1 - b0), x = min(x0 + (cell[k] & 255), D - 1);
+            v[k] = Xi[((int64_t)(g * D + dz) * D + y) * D + x];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < kC4Items; k++)
+            xl[k * 64 + lane] = v4bf{(__bf16)v[k].x, (__bf16)v[k].y, (__bf16)v[k].z, (__bf16)v[k].w};
+        __builtin_amdgcn_wave_barrier();
+        const int gx = x0 + xs, gb = b0 + gi, ny = min(kC4Rows, P - y0);
+        TOut* out = Y + ((((int64_t)gb * P + gz) * P + y0) * P + gx) * 32;
+        const bool valid = gx < P && gb < B;
+        for (int y = 0; y < ny; y++, out += (int64_t)P * 32) {
+            v4f acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                v4bf e = xl[y * rc + off[s][0]], f = xl[y * rc + off[s][1]];
+                // taps 27..31: their weights are zeros, an infinity times one is not
+                if (s == 3 && kq > 1) e = v4bf{};
+                if (s == 3 && kq > 0) f = v4bf{};
+                const v8bf a = {e[0], e[1], e[2], e[3], f[0], f[1], f[2], f[3]};
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++)
+                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][ct], a, acc[ct], 0, 0, 0);
+            }
+            if (!valid) continue;
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    acc[ct][i] += bs[ct][i];
+                    if (relu) acc[ct][i] = fmaxf(acc[ct][i], 0.f);
+                }
+            store32(out, kq, acc[0], acc[1]);
         }
     }
 }
@@ -562,30 +757,79 @@ size_t cnn_conv_packed_count(int cin, int cout) {
     return (size_t)(cin == 32 ? 27 : 32) * (cout == 3 ? 16 : 32) * cin;
 }
 
-template <int CIN, int COUTP, class TIn, class TOut>
-static int conv_launch(const void* X, const uint16_t* Wp, const float* bias, void* Y, int B, int D,
-                       int cout, int relu, hipStream_t s) {
-    auto kern = k_conv3<CIN, COUTP, TIn, TOut>;
-    const size_t lds = conv_lds_bytes<CIN, COUTP>();
-    static int per_cu = 0;  // resident workgroups per CU (one value per instantiation)
-    if (!per_cu) {
-        C2_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)lds));
-        int per = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 256, lds) != hipSuccess || per < 1)
-            per = 1;
-        per_cu = per;
+// Tile shape of a convolution over B grids of P^3 outputs: the x width with
+// the fewest positions computed, counting padding in x and in the groups of
+// 16 / tx grids (the wider one where equal), and as many z chunks as fill the
+// given wavefronts evenly.  A chunk costs its planes and about one more (the
+// halo planes' loads and the start of the pipeline).
+static ConvTile conv_tile(int B, int P, int64_t waves) {
+    ConvTile T{};
+    int64_t best = -1;
+    for (int tx : {16, 8, 4}) {
+        const int g = 16 / tx;
+        const int64_t n = (int64_t)((P + tx - 1) / tx) * ((B + g - 1) / g);
+        // (offsets within a group of grids are 32-bit)
+        const bool fits = g == 1 || (int64_t)g * (P + 2) * (P + 2) * (P + 2) * 32 < ((int64_t)1 << 31);
+        if (best < 0 || (fits && n < best)) {
+            best = n;
+            T.tx = tx;
+            T.nx = (P + tx - 1) / tx;
+            T.nb = (B + g - 1) / g;
+        }
     }
+    T.ny = (P + kConvRows - 1) / kConvRows;
+    const int64_t cols = (int64_t)T.nx * T.ny * T.nb;
+    double cost = 0.0;
+    for (int zc = P; zc >= 1; zc--) {
+        const int nz = (P + zc - 1) / zc;
+        const double c = (double)((cols * nz + waves - 1) / waves) * (zc + 1.0);
+        if (T.nz == 0 || c < cost) {
+            cost = c;
+            T.nz = nz;
+            T.zc = zc;
+        }
+    }
+    return T;
+}
+
+static int device_cus() {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         ncu = 256;
-    const int P = D - 2;
-    const int64_t nblk = (int64_t)B * ((P + kConvBx - 1) / kConvBx) * ((P + kConvBy - 1) / kConvBy) *
-                         ((P + kConvBz - 1) / kConvBz);
-    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(nblk, (int64_t)ncu * per_cu));
-    kern<<<grid, 256, lds, s>>>(static_cast<const TIn*>(X), Wp, bias, static_cast<TOut*>(Y), B, D,
-                                cout, relu);
+    return std::max(1, ncu);
+}
+
+template <int NT, class TIn, class TOut>
+static int conv_launch(const void* X, const uint16_t* Wp, const float* bias, void* Y, int B, int D,
+                       int cout, int relu, hipStream_t s) {
+    auto kern = k_conv3<NT, TIn, TOut>;
+    const size_t lds = conv_lds_bytes<NT>();
+    static bool attr = false;  // (one value per instantiation)
+    if (!attr) {
+        C2_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)lds));
+        attr = true;
+    }
+    const int ncu = device_cus();
+    const ConvTile T = conv_tile(B, D - 2, (int64_t)ncu * kConvWaves);
+    const int64_t items = (int64_t)T.nb * T.nx * T.ny * T.nz;
+    const unsigned grid = (unsigned)std::min<int64_t>((items + kConvWaves - 1) / kConvWaves, ncu);
+    kern<<<grid, kConvWaves * 64, lds, s>>>(static_cast<const TIn*>(X), Wp, bias,
+                                            static_cast<TOut*>(Y), B, D, cout, relu, T);
+    C2_HIP(hipGetLastError());
+    return CUBE2_OK;
+}
+
+template <class TOut>
+static int conv_c4_launch(const void* X, const uint16_t* Wp, const float* bias, void* Y, int B,
+                          int D, int relu, hipStream_t s) {
+    const int ncu = device_cus();
+    const ConvTile T = conv_tile(B, D - 2, (int64_t)ncu * 16);
+    const int64_t items = (int64_t)T.nb * T.nx * (D - 2) * ((D - 2 + kC4Rows - 1) / kC4Rows);
+    const unsigned grid = (unsigned)std::min<int64_t>((items + 3) / 4, (int64_t)ncu * 16);
+    k_conv3_c4<TOut><<<grid, 256, 0, s>>>(static_cast<const float*>(X), Wp, bias,
+                                          static_cast<TOut*>(Y), B, D, relu, T);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }
@@ -596,16 +840,16 @@ int cnn_conv3(const void* X, int x_bf16, const uint16_t* Wp, const float* bias, 
     C2_TRY(cnn_check(X && Wp && bias && Y && B >= 0 && D >= 3, "conv3"));
     if (B == 0) return CUBE2_OK;
     if (cin == 4 && cout == 32 && !x_bf16)
-        return y_bf16 ? conv_launch<4, 32, float, uint16_t>(X, Wp, bias, Y, B, D, cout, relu, s)
-                      : conv_launch<4, 32, float, float>(X, Wp, bias, Y, B, D, cout, relu, s);
+        return y_bf16 ? conv_c4_launch<uint16_t>(X, Wp, bias, Y, B, D, relu, s)
+                      : conv_c4_launch<float>(X, Wp, bias, Y, B, D, relu, s);
     if (cin == 32 && cout == 32)
-        return x_bf16 ? (y_bf16 ? conv_launch<32, 32, uint16_t, uint16_t>(X, Wp, bias, Y, B, D, cout, relu, s)
-                                : conv_launch<32, 32, uint16_t, float>(X, Wp, bias, Y, B, D, cout, relu, s))
-                      : (y_bf16 ? conv_launch<32, 32, float, uint16_t>(X, Wp, bias, Y, B, D, cout, relu, s)
-                                : conv_launch<32, 32, float, float>(X, Wp, bias, Y, B, D, cout, relu, s));
+        return x_bf16 ? (y_bf16 ? conv_launch<2, uint16_t, uint16_t>(X, Wp, bias, Y, B, D, cout, relu, s)
+                                : conv_launch<2, uint16_t, float>(X, Wp, bias, Y, B, D, cout, relu, s))
+                      : (y_bf16 ? conv_launch<2, float, uint16_t>(X, Wp, bias, Y, B, D, cout, relu, s)
+                                : conv_launch<2, float, float>(X, Wp, bias, Y, B, D, cout, relu, s));
     if (cin == 32 && cout == 3 && !y_bf16)
-        return x_bf16 ? conv_launch<32, 16, uint16_t, float>(X, Wp, bias, Y, B, D, cout, relu, s)
-                      : conv_launch<32, 16, float, float>(X, Wp, bias, Y, B, D, cout, relu, s);
+        return x_bf16 ? conv_launch<1, uint16_t, float>(X, Wp, bias, Y, B, D, cout, relu, s)
+                      : conv_launch<1, float, float>(X, Wp, bias, Y, B, D, cout, relu, s);
     set_error("conv3: no kernel for %d -> %d channels (x %s, y %s)", cin, cout,
               x_bf16 ? "bf16" : "f32", y_bf16 ? "bf16" : "f32");
     return CUBE2_ERR_ARG;
