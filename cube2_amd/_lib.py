@@ -76,6 +76,9 @@ SIGNATURES = {
                                               vp_, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int]),
     "cube2_cnn_conv_pack_dev": (C.c_int, [vp_, vp_, C.c_int, C.c_int]),
     "cube2_cnn_conv3_dev": (C.c_int, [vp_, C.c_int, vp_, vp_, vp_, C.c_int] + [C.c_int] * 5),
+    "cube2_cnn_net_forward_dev": (C.c_int, [vp_] * 4 + [C.c_int] * 2),
+    "cube2_cnn_net_backward_dev": (C.c_int, [vp_] * 3 + [C.c_int] * 2 + [vp_] * 2),
+    "cube2_cnn_net_adam_dev": (C.c_int, [vp_] * 6 + [C.c_float] * 4 + [C.c_int]),
     "cube2_learned_set": (C.c_int, [vp_, vp_, C.c_float, C.c_int]),
     "cube2_learned_clear": (C.c_int, []),
     "cube2_learned_inputs_dev": (C.c_int, [vp_, C.c_int, vp_, vp_]),

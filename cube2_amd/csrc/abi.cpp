@@ -406,6 +406,7 @@ void c_gpu_velocity_finalize(void) {
     layout_release();
     drift_release();
     cnn_release();
+    cnn_bwd_release();
     learned_release();
     Context& C = ctx();
     C.dv64.release();
@@ -485,6 +486,55 @@ int cube2_cnn_conv3_dev(const void* X, int x_bf16, const uint16_t* Wp, const flo
     return cnn_call([&] {
         C2_TRY(ensure_init());
         return cnn_conv3(X, x_bf16, Wp, bias, Y, y_bf16, B, D, cin, cout, relu, ctx().stream);
+    });
+}
+int cube2_cnn_net_forward_dev(const float* x, const uint16_t* const* Wp, const float* const* b,
+                              float* const* y, int B, int D) {
+    return cnn_call([&] {
+        C2_TRY(ensure_init());
+        bool ok = x && Wp && b && y && B >= 0 && D >= 9;
+        for (int l = 0; ok && l < 4; l++) ok = Wp[l] && b[l] && y[l];
+        if (!ok) {
+            set_error("cnn: bad arguments to net_forward");
+            return (int)CUBE2_ERR_ARG;
+        }
+        const int c[5] = {4, 32, 32, 32, 3};
+        for (int l = 0; l < 4; l++)
+            C2_TRY(cnn_conv3(l ? y[l - 1] : x, 0, Wp[l], b[l], y[l], 0, B, D - 2 * l, c[l], c[l + 1],
+                             l < 3, ctx().stream));
+        return (int)CUBE2_OK;
+    });
+}
+int cube2_cnn_net_backward_dev(const float* const* acts, const uint16_t* const* Wb,
+                               const float* dout, int B, int D, float* const* dW,
+                               float* const* db) {
+    return cnn_call([&] {
+        C2_TRY(ensure_init());
+        bool ok = acts && Wb && dout && dW && db && B >= 1 && acts[4];
+        for (int l = 0; ok && l < 4; l++) ok = acts[l] && Wb[l] && dW[l] && db[l];
+        if (!ok) {
+            set_error("cnn: bad arguments to net_backward");
+            return (int)CUBE2_ERR_ARG;
+        }
+        if (!cnn_net_backward_fits(D)) {
+            set_error("net_backward: patches of %d cells a side (9 or 10)", D);
+            return (int)CUBE2_ERR_CAPACITY;
+        }
+        return cnn_net_backward(acts, Wb, dout, B, D, dW, db, ctx().stream);
+    });
+}
+int cube2_cnn_net_adam_dev(float* const* w, const float* const* g, float* const* m,
+                           float* const* v, uint16_t* const* wb, uint16_t* const* wp, float lr,
+                           float b1, float b2, float eps, int t) {
+    return cnn_call([&] {
+        C2_TRY(ensure_init());
+        bool ok = w && g && m && v && wb && wp && t >= 1;
+        for (int l = 0; ok && l < 8; l++) ok = w[l] && g[l] && m[l] && v[l] && (l >= 4 || (wb[l] && wp[l]));
+        if (!ok) {
+            set_error("cnn: bad arguments to net_adam");
+            return (int)CUBE2_ERR_ARG;
+        }
+        return cnn_net_adam(w, g, m, v, wb, wp, lr, b1, b2, eps, t, ctx().stream);
     });
 }
 int cube2_learned_set(const float* const* W, const float* const* b, float y_scale, int occupancy) {

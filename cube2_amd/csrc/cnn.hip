@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "adam.h"
 #include "common.h"
 #include "engine.h"
 
@@ -197,11 +198,10 @@ __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float
                        float b1, float b2, float eps, float c1, float c2) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const float gi = g[e];
-    const float mi = b1 * m[e] + (1.f - b1) * gi, vi = b2 * v[e] + (1.f - b2) * gi * gi;
+    float mi = m[e], vi = v[e];
+    const float wi = adam_update(w[e], g[e], mi, vi, lr, b1, b2, eps, c1, c2);
     m[e] = mi;
     v[e] = vi;
-    const float wi = w[e] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     w[e] = wi;
     if (wb) wb[e] = to_bf16(wi);
 }

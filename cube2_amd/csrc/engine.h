@@ -134,6 +134,14 @@ int cnn_gemm(const uint16_t* A, int64_t sam, int64_t sak, const uint16_t* B, int
 int cnn_gemm_noalloc(const uint16_t* A, int64_t sam, int64_t sak, const uint16_t* B, int64_t sbk,
                      int64_t sbn, float* C, int64_t ldc, int M, int N, int K, int acc);
 void cnn_release();
+// Backward and Adam step of the whole network on training patches (cnn_bwd.hip).
+bool cnn_net_backward_fits(int D);
+int cnn_net_backward(const float* const* acts, const uint16_t* const* Wb, const float* dout, int B,
+                     int D, float* const* dW, float* const* db, hipStream_t s);
+int cnn_net_adam(float* const* w, const float* const* g, float* const* m, float* const* v,
+                 uint16_t* const* wb, uint16_t* const* wp, float lr, float b1, float b2, float eps,
+                 int t, hipStream_t s);
+void cnn_bwd_release();
 // 3^3 valid convolution on the matrix cores (cin 4 or 32; cout 32, or 3
 // from 32); Wp packed by cnn_conv_pack (cnn_conv_packed_count entries).
 int cnn_conv_pack(const float* W, uint16_t* Wp, int cin, int cout, hipStream_t s);

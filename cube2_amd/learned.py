@@ -39,6 +39,11 @@ def _p(t):
     return t.data_ptr()
 
 
+def _ps(ts):
+    """A host array of the tensors' addresses."""
+    return (C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
+
+
 class LearnedPP:
     def __init__(self, params=None, seed: int = 0, device: str = "cuda:0"):
         """params: [(W [27*c_in][c_out], b [c_out])] (numpy), or He-uniform
@@ -84,25 +89,27 @@ class LearnedPP:
         """x [B][D][D][D][4] float32 on the device -> out [B][D-8][D-8][D-8][3]
         (the matrix-core convolution per layer, FP32 activations kept for
         the backward pass)."""
-        torch, L = self.torch, _lib.lib()
+        torch = self.torch
         B, D = x.shape[0], x.shape[1]
         h = x.contiguous()
-        self.acts = [h]
-        for l in range(4):
-            cin, cout = CHANNELS[l], CHANNELS[l + 1]
-            P = D - 2
-            y = torch.empty((B, P, P, P, cout), dtype=torch.float32, device=self.dev)
-            _lib.check(L.cube2_cnn_conv3_dev(_p(h), 0, _p(self.Wp[l]), _p(self.b[l]), _p(y), 0, B,
-                                             D, cin, cout, int(l < 3)))
-            h = y
-            self.acts.append(h)
-            D = P
-        return h
+        ys = [torch.empty((B, D - 2 * l, D - 2 * l, D - 2 * l, CHANNELS[l]), dtype=torch.float32,
+                          device=self.dev) for l in range(1, 5)]
+        _lib.check(_lib.lib().cube2_cnn_net_forward_dev(_p(h), _ps(self.Wp), _ps(self.b), _ps(ys),
+                                                         B, D))
+        self.acts = [h] + ys
+        return ys[3]
 
     def backward(self, dout):
         """Gradients [(dW, db)] of sum(dout * out) for the last forward."""
         torch, L = self.torch, _lib.lib()
-        B = dout.shape[0]
+        B, D = dout.shape[0], self.acts[0].shape[1]
+        if D <= PATCH and B:  # training patches: no im2col
+            grads = [(torch.empty_like(w), torch.empty_like(b)) for w, b in zip(self.W, self.b)]
+            dout = dout.contiguous()  # held until the call returns
+            _lib.check(L.cube2_cnn_net_backward_dev(_ps(self.acts), _ps(self.Wb), _p(dout), B, D,
+                                                    _ps([g[0] for g in grads]),
+                                                    _ps([g[1] for g in grads])))
+            return grads
         g = dout.contiguous().clone()
         grads = [None] * 4
         for l in range(3, -1, -1):
@@ -135,13 +142,10 @@ class LearnedPP:
     def step(self, grads, lr: float = 1e-3, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8):
         L = _lib.lib()
         self.t += 1
-        for l, (dW, db) in enumerate(grads):
-            _lib.check(L.cube2_cnn_adam_dev(_p(self.W[l]), _p(dW), _p(self.mW[l]), _p(self.vW[l]),
-                                            _p(self.Wb[l]), self.W[l].numel(), lr, b1, b2, eps,
-                                            self.t))
-            _lib.check(L.cube2_cnn_adam_dev(_p(self.b[l]), _p(db), _p(self.mb[l]), _p(self.vb[l]),
-                                            None, self.b[l].numel(), lr, b1, b2, eps, self.t))
-        self._refresh(bf16=False)
+        gs = [dW.contiguous() for dW, _ in grads] + [db.contiguous() for _, db in grads]
+        _lib.check(L.cube2_cnn_net_adam_dev(_ps(self.W + self.b), _ps(gs), _ps(self.mW + self.mb),
+                                            _ps(self.vW + self.vb), _ps(self.Wb), _ps(self.Wp),
+                                            lr, b1, b2, eps, self.t))
 
     def cic_mse(self, out, frac, target):
         """(loss, dloss/dout, predictions) of the CIC combination of out

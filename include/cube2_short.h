@@ -249,6 +249,23 @@ int cube2_cnn_conv_pack_dev(const float* W, uint16_t* Wp, int cin, int cout);
  * 32 -> 32, 32 -> 3 (Y FP32). */
 int cube2_cnn_conv3_dev(const void* X, int x_bf16, const uint16_t* Wp, const float* bias, void* Y,
                         int y_bf16, int B, int D, int cin, int cout, int relu);
+/* The whole network (4 -> 32 -> 32 -> 32 -> 3 channels, ReLU after the first
+ * three layers) in one call each; arrays of device pointers are host arrays.
+ * net_forward: y[l] [B][(D-2-2l)^3][c_{l+1}] FP32 from x [B][D^3][4], Wp as
+ * packed by cube2_cnn_conv_pack_dev.  net_backward: the gradients dW[l]
+ * [27 c_l][c_{l+1}] and db[l] of sum(dout * y[3]) from acts[0..4] = x, y[0..3]
+ * and the BF16 weights Wb[l] [27 c_l][c_{l+1}]; D = 9 or 10 (training patches),
+ * else CUBE2_ERR_CAPACITY.  net_adam: one Adam step (cube2_cnn_adam_dev) of W
+ * of the four layers and then their b (w, g, m, v: 8 pointers), refreshing
+ * the layers' BF16 copies wb and the weights of their packed forms wp. */
+int cube2_cnn_net_forward_dev(const float* x, const uint16_t* const* Wp, const float* const* b,
+                              float* const* y, int B, int D);
+int cube2_cnn_net_backward_dev(const float* const* acts, const uint16_t* const* Wb,
+                               const float* dout, int B, int D, float* const* dW,
+                               float* const* db);
+int cube2_cnn_net_adam_dev(float* const* w, const float* const* g, float* const* m,
+                           float* const* v, uint16_t* const* wb, uint16_t* const* wp, float lr,
+                           float b1, float b2, float eps, int t);
 /* Learned stand-in in the kick (CUBE2_KICK_LEARNED).  The network: four
  * valid 3^3 convolutions 4 -> 32 -> 32 -> 32 -> 3 channels, ReLU after the
  * first three, over fine cells of the level-2 mesh; input channels
