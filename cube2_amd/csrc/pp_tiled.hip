@@ -44,191 +44,11 @@
 #include <type_traits>
 
 #include "pp_kernels.h"
+#include "pp_law.h"
 #include "profile.h"
 #include "reduce.h"
 
 namespace cube2 {
-
-constexpr int kQ = 128;  // queue entries per wavefront
-// A position farther from every particle than any range: its squared distance
-// overflows to +inf, so a pair test with it fails without a bounds check.
-constexpr float kFar = 1e30f;
-
-// 1/x from an approximation y0: with e = 1 - x*y0 (one FMA, rounded once),
-// 1/x = y0/(1-e) = y0 (1 + e + e^2 + e^3/(1-e)), so y0 + y0 (e + e^2) is
-// within |e|^3 + 3*2^-53 (relative) of 1/x.  For |e| <= 2^-18 that is below
-// 2^-51.
-__device__ inline double recip_refine(double x, double y0) {
-    const double e = fma(-x, y0, 1.0);
-    return fma(fma(e, e, e), y0, y0);
-}
-
-// FP64 reciprocal of a float: v_rcp_f64 and one cubic refinement.  The
-// self-test checks |1 - x*y| <= 2^-51 for every float x with exponent in
-// [-40, 40].
-__device__ inline double recip64(double x) { return recip_refine(x, __builtin_amdgcn_rcp(x)); }
-
-__device__ inline float div_by(float a, double y) { return (float)((double)a * y); }
-
-// RN(sqrt(x)) for normal positive finite x (pair distances: r^2 >= 2^-28,
-// the positions being multiples of ratio_cs * 2^-16 apart).  v_sqrt_f32 is
-// within one ulp; of s and its neighbours s-, s+ the rounding test keeps s-
-// if x <= s- * s and s+ if x > s * s+ (FMA residuals, exact in sign: the
-// residuals are integer multiples of ulp^2 and midpoints squared are not).
-// No scaling or special-value fix-ups, which only zero, infinities, NaNs and
-// tiny inputs need.  The self-test checks it against IEEE sqrtf for every
-// float with exponent in [-40, 40].
-__device__ inline float sqrt_rn(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float lo = __int_as_float(__float_as_int(s) - 1);
-    const float hi = __int_as_float(__float_as_int(s) + 1);
-    float r = fmaf(-lo, s, x) <= 0.0f ? lo : s;
-    r = fmaf(-hi, s, x) > 0.0f ? hi : r;
-    return r;
-}
-
-struct FraK {
-    float a;        // softening diameter
-    double inv_a;   // 1/a in FP64
-    double half_a2;  // (a/2)^2 in FP64
-    float c;        // (1/35)/(a*a), as basic_functions.f08:103 rounds it
-    float r2max;    // a^2 (1 + 2^-17): for r^2 above it, RN(2r/a) > 2 for certain
-};
-
-__device__ inline FraK make_frak(float a) {
-    FraK K;
-    K.a = a;
-    K.inv_a = a > 0.0f ? 1.0 / (double)a : 0.0;
-    K.half_a2 = 0.25 * (double)a * (double)a;
-    K.r2max = (float)((double)a * a * (1.0 + 0x1p-17));
-    {
-#pragma clang fp contract(off)
-        K.c = 1.0f / 35.0f / (a * a);
-    }
-    return K;
-}
-
-// F_ra(r, a) of basic_functions.f08:95-109 with the reference's rounding, for
-// ep = RN(2r/a) <= 2 (the caller handles a = 0 and ep > 2, where F_ra is
-// 1/(r*r)).  Evaluated without divergence: the powers are shared, both
-// polynomials are formed in the reference's operation order, and one is
-// selected.  RN(12/e2) is 12 * (FP64 reciprocal), rounded once to float;
-// the reciprocal refines y0 = (a/2)^2 (1/r)^2, which is within a few float
-// roundings of 1/e2 (ep = RN(2r/a), e2 = RN(ep*ep)).
-__device__ inline float fra_ref_poly(float ep, const FraK& K, double inv_r2) {
-#pragma clang fp contract(off)
-    const float e2 = ep * ep, e3 = e2 * ep, e4 = e3 * ep, e5 = e4 * ep, e6 = e5 * ep;
-    const float t12 = (float)(12.0 * recip_refine((double)e2, K.half_a2 * inv_r2));
-    const float hi = K.c * (t12 - 224.0f + 896.0f * ep - 840.0f * e2 + 224.0f * e3 + 70.0f * e4 -
-                            48.0f * e5 + 7.0f * e6);
-    const float lo = K.c * (224.0f * ep - 224.0f * e3 + 70.0f * e4 + 48.0f * e5 - 21.0f * e6);
-    // (the reference's F_ra is 0 at ep = 0; pairs here have r^2 >= 2^-28, so
-    // ep > 0)
-    return ep > 1.0f ? hi : lo;
-}
-
-__device__ inline float fra_fast2(float ep, float ir2, float c) {
-    if (ep > 2.0f) return ir2;
-    const float hi = fmaf(3.0f / 35.0f, ir2,
-                          c * fmaf(ep, fmaf(ep, fmaf(ep, fmaf(ep, fmaf(ep, fmaf(ep, 7.0f, -48.0f),
-                                                                         70.0f), 224.0f), -840.0f),
-                                            896.0f), -224.0f));
-    const float e2 = ep * ep;
-    const float lo = c * ep * fmaf(e2, fmaf(ep, fmaf(ep, fmaf(ep, -21.0f, 48.0f), 70.0f), -224.0f), 224.0f);
-    return ep > 1.0f ? hi : lo;
-}
-
-enum { kModeRef = 0, kModeFast = 1, kModePrecise = 2, kModePlummer = 3 };
-
-// 1/r^2 - F_ra(r, a) for r < a (ep = 2r/a in (0, 2]), cancellation-free.
-__device__ inline float short_term(float ep, float ir2, float c) {
-    const float t = 2.0f - ep, t2 = t * t;
-    const float q = fmaf(ep, fmaf(ep, fmaf(ep, 7.0f, 22.0f), 10.0f), 4.0f);
-    const float hi = t2 * t2 * t * q * ir2 * (1.0f / 140.0f);
-    const float e2 = ep * ep;
-    const float lo =
-        ir2 - c * ep * fmaf(e2, fmaf(ep, fmaf(ep, fmaf(ep, -21.0f, 48.0f), 70.0f), -224.0f), 224.0f);
-    return ep > 1.0f ? hi : lo;
-}
-
-// 1/r^2 - r / (r^2 + eps^2)^(3/2) (Plummer softening), cancellation-free:
-// with u = eps^2/r^2 and w = (1 + u)^(-1/2) it is (1 - w^3)/r^2, and
-// 1 - w = u w^2 / (1 + w), so (1/r^2) u w^2 (1 + w + w^2) / (1 + w).
-__device__ inline float plummer_term(float ir2, float eps2) {
-    const float u = eps2 * ir2;
-    const float w = __frsqrt_rn(1.0f + u);
-    const float w2 = w * w;
-    return ir2 * u * w2 * (1.0f + w + w2) / (1.0f + w);
-}
-
-template <int kMode>
-__device__ inline void pair_force(float4 e, const FraK& Ka, const FraK& Kr, float& fx, float& fy,
-                                  float& fz) {
-    if (kMode == kModeRef) {
-#pragma clang fp contract(off)
-        const float rm = sqrt_rn(e.w);
-        const double inv_rm = recip64((double)rm);
-        // RN(1/(r*r)): the reciprocal of RN(r*r) refined from (1/r)^2
-        const double inv_rm2 = inv_rm * inv_rm;
-        const float frr = (float)recip_refine((double)(rm * rm), inv_rm2);
-        // range term: r < range, so ep <= 2 except by rounding at the cutoff
-        const float epr = div_by(2.0f * rm, Kr.inv_a);
-        const float fr = epr > 2.0f ? frr : fra_ref_poly(epr, Kr, inv_rm2);
-        // softening term: 1/(r*r) unless r is within app; the polynomial runs
-        // only when some lane of the wavefront needs it
-        float fa = frr;
-        if (Ka.a != 0.0f && __ballot(e.w <= Ka.r2max)) {
-            const float epa = div_by(2.0f * rm, Ka.inv_a);
-            if (__ballot(epa <= 2.0f)) {
-                const float pa = fra_ref_poly(epa, Ka, inv_rm2);
-                if (epa <= 2.0f) fa = pa;
-            }
-        }
-        const float fpp = fa - fr;
-        fx = div_by(fpp * e.x, inv_rm);
-        fy = div_by(fpp * e.y, inv_rm);
-        fz = div_by(fpp * e.z, inv_rm);
-    } else if (kMode == kModeFast) {
-        const float ir = __frsqrt_rn(e.w);
-        const float ir2 = ir * ir;
-        const float r = e.w * ir;
-        float fa = ir2;
-        if (r <= Ka.a) fa = fra_fast2(r * (float)(2.0 * Ka.inv_a), ir2, Ka.c);
-        const float f = (fa - fra_fast2(r * (float)(2.0 * Kr.inv_a), ir2, Kr.c)) * ir;
-        fx = f * e.x;
-        fy = f * e.y;
-        fz = f * e.z;
-    } else if (kMode == kModePlummer) {
-        // pair = (1/r^2 - F_ra(r, range)) - (1/r^2 - r/(r^2 + app^2)^(3/2)),
-        // each piece cancellation-free (softening length eps = app)
-        const float r = sqrtf(e.w);
-        const float ir = 1.0f / r;
-        const float ir2 = ir * ir;
-        float f = short_term(r * (float)(2.0 * Kr.inv_a), ir2, Kr.c);
-        if (Ka.a > 0.0f) f -= plummer_term(ir2, Ka.a * Ka.a);
-        f *= ir;
-        fx = f * e.x;
-        fy = f * e.y;
-        fz = f * e.z;
-    } else {
-        // pair = (1/r^2 - F_ra(r, range)) - (1/r^2 - F_ra(r, app)), the second
-        // term zero for r > app; each piece cancellation-free.
-        const float r = sqrtf(e.w);
-        const float ir = 1.0f / r;
-        const float ir2 = ir * ir;
-        float f = short_term(r * (float)(2.0 * Kr.inv_a), ir2, Kr.c);
-        if (Ka.a > 0.0f && r < Ka.a) f -= short_term(r * (float)(2.0 * Ka.inv_a), ir2, Ka.c);
-        f *= ir;
-        fx = f * e.x;
-        fy = f * e.y;
-        fz = f * e.z;
-    }
-}
-
-// Orders LDS accesses of the lanes of one wavefront.  LDS operations of a
-// wavefront are performed in issue order, so a compiler barrier suffices (no
-// block barrier: the wavefronts of a block run independent trip counts).
-__device__ inline void wave_lds_sync() { __builtin_amdgcn_wave_barrier(); }
 
 template <int kMode, int kJB = 64, bool kNewton = false>
 struct WaveLDS {
@@ -237,41 +57,17 @@ struct WaveLDS {
     float4 q[kQ];           // queued chunks: accepted pairs (dx, dy, dz, r^2)
     unsigned char qi[kQ];   // and their i slot
     Acc acc[64][3];         // per-i force sums
-    float4 jb[kJB + 64];    // current batch of j positions, then J far-away ones
+    // current batch of j positions, then J far-away ones; pairs once: two
+    // blocks of 64 j, the first 32 of each repeated after it
+    float4 jb[kNewton ? 192 : kJB + 64];
     int rs[64], rp[64];     // row group: j = v + rs[k] for rp[k-1] <= v < rp[k]
-    // pairs-once pass: per batch slot, the sum over the chunk's i of the
-    // pair forces on i from that slot's j (j's reaction, negated; one
-    // 16-byte LDS store per slot)
-    float4 jr[kNewton ? kJB : 1];
 };
 
-// Sums over groups of 2^LG consecutive lanes (LG <= 6), left in each
-// group's last lane: DPP row shifts within the 16-lane rows (shift 1, 2, 4,
-// 8), then row broadcasts across them (lane 15 to the next row, lane 31 to
-// the upper half).  Every lane must be active.
-template <int K>
-__device__ inline float dpp_add(float x) {
-    constexpr int ctrl = K < 4 ? 0x110 + (1 << K) : (K == 4 ? 0x142 : 0x143);
-    constexpr int rows = K < 4 ? 0xf : (K == 4 ? 0xa : 0xc);
-    return x + __int_as_float(
-                   __builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, rows, 0xf, K < 4));
-}
-
-template <int LG>
-__device__ inline void group_sum3(float& x, float& y, float& z) {
-    if constexpr (LG > 0) {
-        group_sum3<LG - 1>(x, y, z);
-        x = dpp_add<LG - 1>(x);
-        y = dpp_add<LG - 1>(y);
-        z = dpp_add<LG - 1>(z);
-    }
-}
-
-// Signed fixed point (value * scale, rounded to nearest) of a pairs-once
-// partial sum, added to a particle's 64-bit accumulator: integer adds
-// commute, so the totals do not depend on the order of the atomics.
-__device__ inline void fixed_add(unsigned long long* dst, float v, float scale) {
-    if (v != 0.0f) atomicAdd(dst, (unsigned long long)__double2ll_rn((double)v * (double)scale));
+constexpr int kJBlock = 96;  // a block of 64 j and the repeats
+// x from the next higher lane, lane 63 from lane 0 (DPP, folded into the add
+// that uses it).  Every lane must be active.
+__device__ inline float wave_rol1(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x134, 0xf, 0xf, true));
 }
 
 template <int kMode, int kJB, bool kN>
@@ -289,12 +85,6 @@ __device__ inline void flush(WaveLDS<kMode, kJB, kN>& L, int lane, int begin, in
         atomicAdd(&L.acc[ii][2], (Acc)fz);
     }
     wave_lds_sync();
-}
-
-// Wavefront-uniform copies (scalar registers) of values every lane holds.
-__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline float uni(float v) {
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
 __device__ inline int find_tile2(const PPTile* __restrict__ T, int ntile, uint32_t c) {
@@ -362,7 +152,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             R = (int)ceilf(range * (float)T.rcp / (float)A.ratio_cs);
             pp2 = range * range;
         }
-        const FraK Ka = make_frak(A.app), Kr = make_frak(range);
+        const FraK Ka = uni(make_frak(A.app)), Kr = uni(make_frak(range));
         for (int q = lane; q < 64 * 3; q += 64) (&L.acc[0][0])[q] = 0;
         wave_lds_sync();
         const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
@@ -393,6 +183,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         }
         Acc dax = 0, day = 0, daz = 0;
         unsigned npa = 0;
+        int jhead = 0, jtail = 0;  // pairs once: kept j taken and staged
         // direct chunks: bounding box of the chunk's i; a j farther than the
         // range from the box cannot pair with any of them (the 1e-4 relative
         // margin keeps every j the per-pair test could accept)
@@ -476,26 +267,113 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             // one: rp of the rows past the group is M > v, so the walk stops
             // inside the group
             int frow = 0;
-            auto fetch = [&](int vb) {
+            auto fetch = [&](int vb, int& jx) {
                 const int v = vb + lane;
                 float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (v < M) {
                     while (L.rp[frow] <= v) frow++;
-                    const int jx = v + L.rs[frow];
+                    jx = v + L.rs[frow];
                     q4 = A.pos4[jx];
-                    // pairs once: w = the sorted index of a j of the chunk's
-                    // range, INT_MAX for a j that acts on i alone
-                    if (kNewton) q4.w = __int_as_float(q4.w == range ? jx : INT_MAX);
                 }
                 return q4;
             };
             // a batch is kJB candidates, kH fetches of 64; the next batch's
             // fetches are issued before this batch's pairs run
             float4 qcur[kH];
+            int jcur[kH] = {};
 #pragma unroll
-            for (int h = 0; h < kH; h++) qcur[h] = fetch(64 * h);
-            for (int vb = 0; vb < M; vb += kJB) {
+            for (int h = 0; h < kH; h++) qcur[h] = fetch(64 * h, jcur[h]);
+            // (pairs once: a last step without candidates for the j left over)
+            const bool last = nwc && rg + 64 >= nrows;
+            const int vend = last ? (M + kJB - 1) / kJB * kJB + kJB : M;
+            for (int vb = 0; vb < vend; vb += kJB) {
                 int nb = 0;
+                if (nwc) {
+                    // Keep the j near the chunk's box that no chunk before this
+                    // one's evaluates (a j of the chunk's range before its
+                    // first i does) and collect 64 of them.  Then, at step s,
+                    // lane l takes j (l + s) mod 64: over the I steps each j
+                    // meets I consecutive lanes, every i once, and its
+                    // reaction moves along with it (rotated one lane per step
+                    // by the DPP operand of the add that sums it), so that 64
+                    // j cost I steps of one pair per lane and three additions.
+                    // (Summing a j's reaction over the lanes of one step
+                    // instead took 18 instructions more per step.)
+#pragma unroll
+                    for (int h = 0; h < kH; h++) {
+                        float4 qh = qcur[h];
+                        // w = the sorted index of a j of the chunk's range,
+                        // INT_MAX for a j that acts on i alone
+                        const int jx = qh.w == range ? jcur[h] : INT_MAX;
+                        qh.w = __int_as_float(jx);
+                        const float ex = fmaxf(fmaxf(bx0 - qh.x, qh.x - bx1), 0.0f);
+                        const float ey = fmaxf(fmaxf(by0 - qh.y, qh.y - by1), 0.0f);
+                        const float ez = fmaxf(fmaxf(bz0 - qh.z, qh.z - bz1), 0.0f);
+                        const bool keep = (vb + 64 * h + lane < M) & (jx >= a0) &
+                                          (ex * ex + ey * ey + ez * ez < pp2m);
+                        const uint64_t km = __ballot(keep);
+                        if (keep) {
+                            const int t = jtail + __popcll(km & lt);
+                            const int at = (t >> 6 & 1) * kJBlock + (t & 63);
+                            L.jb[at] = qh;
+                            if ((t & 63) < 32) L.jb[at + 64] = qh;
+                        }
+                        jtail += __popcll(km);
+                        if (h == kH - 1) {
+#pragma unroll
+                            for (int k = 0; k < kH; k++)
+                                if (vb + kJB + 64 * k < M) qcur[k] = fetch(vb + kJB + 64 * k, jcur[k]);
+                        }
+                        const bool rest = last && vb + kJB >= vend && h == kH - 1;
+                        if (jtail - jhead < 64 && !(rest && jtail > jhead)) continue;
+                        const int bb = (jhead >> 6 & 1) * kJBlock;
+                        if (rest && lane >= jtail - jhead) {  // far-away j to the block's end
+                            const float4 far4 = make_float4(kFar, kFar, kFar, __int_as_float(INT_MAX));
+                            L.jb[bb + lane] = far4;
+                            if (lane < 32) L.jb[bb + lane + 64] = far4;
+                        }
+                        wave_lds_sync();
+                        float rx = 0.0f, ry = 0.0f, rz = 0.0f;
+                        for (int s0 = 0; s0 < I; s0 += 32) {
+                            const float4* jp = &L.jb[bb + ((lane + s0) & 63)];
+                            const int ns = uni(min(32, I - s0));
+                            for (int s = 0; s < ns; s++, jp++) {
+#pragma clang fp contract(off)
+                                const float4 qj = *jp;
+                                const int jw = __float_as_int(qj.w);
+                                float4 e;
+                                e.x = qj.x - pix;
+                                e.y = qj.y - piy;
+                                e.z = qj.z - piz;
+                                e.w = e.x * e.x + e.y * e.y + e.z * e.z;
+                                const bool ok = (e.w > 0.0f) & (e.w < pp2) & (jw > ia);
+                                const uint64_t okm = __ballot(ok);
+                                npa += 2 * __popcll(okm) - __popcll(okm & __ballot(jw == INT_MAX));
+                                float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+                                if (ok) {
+                                    pair_force<kMode>(e, Ka, Kr, fx, fy, fz);
+                                    dax += (Acc)fx;
+                                    day += (Acc)fy;
+                                    daz += (Acc)fz;
+                                }
+                                rx = wave_rol1(rx) + fx;
+                                ry = wave_rol1(ry) + fy;
+                                rz = wave_rol1(rz) + fz;
+                            }
+                        }
+                        // lane l now holds the reaction of j (l + I - 1) mod 64
+                        const int jw = __float_as_int(L.jb[bb + ((lane + I - 1) & 63)].w);
+                        if (jw != INT_MAX) {
+                            unsigned long long* d = A.react + 3 * (size_t)jw;
+                            fixed_add(d, -rx, A.react_scale);
+                            fixed_add(d + 1, -ry, A.react_scale);
+                            fixed_add(d + 2, -rz, A.react_scale);
+                        }
+                        jhead += 64;
+                        wave_lds_sync();
+                    }
+                    continue;
+                }
                 if (direct) {  // keep the j near the chunk's box, compacted
 #pragma unroll
                     for (int h = 0; h < kH; h++) {
@@ -503,11 +381,8 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                         const float ex = fmaxf(fmaxf(bx0 - qh.x, qh.x - bx1), 0.0f);
                         const float ey = fmaxf(fmaxf(by0 - qh.y, qh.y - by1), 0.0f);
                         const float ez = fmaxf(fmaxf(bz0 - qh.z, qh.z - bz1), 0.0f);
-                        // (pairs once: a j of the chunk's range before its first
-                        // i evaluates the pair itself)
                         const bool keep = vb + 64 * h + lane < M &&
-                                          ex * ex + ey * ey + ez * ez < pp2m &&
-                                          (!nwc || __float_as_int(qh.w) >= a0);
+                                          ex * ex + ey * ey + ez * ez < pp2m;
                         const uint64_t km = __ballot(keep);
                         if (keep) L.jb[nb + __popcll(km & lt)] = qh;
                         nb += __popcll(km);
@@ -523,7 +398,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                 wave_lds_sync();
 #pragma unroll
                 for (int h = 0; h < kH; h++)
-                    if (vb + kJB + 64 * h < M) qcur[h] = fetch(vb + kJB + 64 * h);
+                    if (vb + kJB + 64 * h < M) qcur[h] = fetch(vb + kJB + 64 * h, jcur[h]);
                 // (i, j) of slot t: the difference vector and whether it pairs
                 // (branch-free: slots past the batch hold far-away j, and an
                 // i slot past the chunk tests from a far-away i)
@@ -539,61 +414,6 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                         e.w = e.x * e.x + e.y * e.y + e.z * e.z;
                     return (e.w > 0.0f) & (e.w < pp2);
                 };
-                if (nwc) {
-                    // Lane (i, s) takes slot t + s at step t, as below; the I
-                    // lanes of slot t + s then hold the forces on all the
-                    // chunk's i from that j, and their sum (a DPP reduction,
-                    // no LDS traffic) is j's reaction for the batch, which
-                    // the group's last lane stores.  (LDS float atomics cost
-                    // ~190 cycles per wavefront instruction on gfx950.)
-                    // (one loop per chunk size: the reduction's DPP steps
-                    // and the group shape are then constants)
-                    auto pairs = [&](auto lg_c) {
-                        constexpr int LG = decltype(lg_c)::value;
-                        constexpr int IC = 1 << LG, JC = 64 >> LG;
-                        for (int t = 0; t < nb; t += JC) {
-                            float4 e;
-                            const int jw = __float_as_int(L.jb[t + jslot].w);
-                            float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-                            if (test(t + jslot, e) & (jw > ia)) {
-#pragma clang fp contract(off)
-                                pair_force<kMode>(e, Ka, Kr, fx, fy, fz);
-                                dax += (Acc)fx;
-                                day += (Acc)fy;
-                                daz += (Acc)fz;
-                                npa += jw != INT_MAX ? 2u : 1u;
-                            }
-                            group_sum3<LG>(fx, fy, fz);
-                            if ((lane & (IC - 1)) == IC - 1 && t + jslot < nb)
-                                L.jr[t + jslot] = make_float4(fx, fy, fz, 0.0f);
-                        }
-                    };
-                    switch (lgI) {
-                        case 0: pairs(std::integral_constant<int, 0>{}); break;
-                        case 1: pairs(std::integral_constant<int, 1>{}); break;
-                        case 2: pairs(std::integral_constant<int, 2>{}); break;
-                        case 3: pairs(std::integral_constant<int, 3>{}); break;
-                        case 4: pairs(std::integral_constant<int, 4>{}); break;
-                        case 5: pairs(std::integral_constant<int, 5>{}); break;
-                        default: pairs(std::integral_constant<int, 6>{}); break;
-                    }
-                    wave_lds_sync();
-                    // the reactions of the batch's j of the chunk's range
-#pragma unroll
-                    for (int h = 0; h < kH; h++) {
-                        const int l = 64 * h + lane;
-                        if (l < nb) {
-                            const int jw = __float_as_int(L.jb[l].w);
-                            if (jw != INT_MAX) {
-                                const float4 r = L.jr[l];
-                                unsigned long long* d = A.react + 3 * (size_t)jw;
-                                fixed_add(d, -r.x, A.react_scale);
-                                fixed_add(d + 1, -r.y, A.react_scale);
-                                fixed_add(d + 2, -r.z, A.react_scale);
-                            }
-                        }
-                    }
-                } else
                 // two loops on the chunk-uniform branch, so that the direct
                 // loop carries only its accumulators
                 if (direct) {
@@ -638,7 +458,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                 atomicAdd(&L.acc[islot][1], day);
                 atomicAdd(&L.acc[islot][2], daz);
             }
-            pa += npa;
+            if (!nwc || lane == 0) pa += npa;  // (pairs once: the wavefront's count)
             wave_lds_sync();
         }
         if (qtail > qhead) flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr);
@@ -843,7 +663,7 @@ int pair_forces_debug(int mode, const float* pairs, int n, float app, float* for
 // [-40, 40] (n = 81 * 2^23) as b and r, with a = l = 1.  Checked: a/b,
 // 12/b, |1 - b*recip64(b)| <= 2^-51, 1/RN(r*r) refined from (1/r)^2, and
 // 12/e2 for ep = RN(2r/l), e2 = RN(ep*ep) refined from (l/2)^2 (1/r)^2, and
-// sqrt_rn(b) against IEEE sqrtf.
+// sqrt_rn(b) and sqrt_recip(b) against IEEE sqrtf, and the latter's reciprocal.
 __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
@@ -883,6 +703,10 @@ __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
     const float mine = div_by(a, yb);
     const float twelve = (float)(12.0 * yb);
     const bool resid = fabs(fma(-(double)b, yb, 1.0)) <= 0x1p-51;
+    double inv_s;
+    const float root = sqrt_recip(b, inv_s);
+    const bool root_ok = __float_as_uint(root) == __float_as_uint(ieee_sqrt) &&
+                         fabs(fma(-(double)root, inv_s, 1.0)) <= 0x1p-51;
     const double inv_r = recip64((double)r);
     const float rr = (float)recip_refine((double)p, inv_r * inv_r);
     const float ep2 = div_by(2.0f * r, 1.0 / (double)l);
@@ -892,7 +716,7 @@ __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
         __float_as_uint(ieee12) != __float_as_uint(twelve) || !resid ||
         __float_as_uint(ieee_rr) != __float_as_uint(rr) || __float_as_uint(ep) != __float_as_uint(ep2) ||
         __float_as_uint(ieee_t12) != __float_as_uint(t12) ||
-        __float_as_uint(ieee_sqrt) != __float_as_uint(sqrt_rn(b)))
+        __float_as_uint(ieee_sqrt) != __float_as_uint(sqrt_rn(b)) || !root_ok)
         atomicAdd(bad, 1ull);
 }
 
