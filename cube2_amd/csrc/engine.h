@@ -36,6 +36,7 @@ struct PPPlan {
     bool all_active = false;   // every subtile has a PP range (apm3 > 0 at its level)
     bool newton = false;       // pairs of one range evaluated once (split pass)
     float react_scale = 0.0f;  // its fixed-point scale, a power of two
+    int small = 0;             // cells of at most this many particles are k_pp_sparse's
     LearnedPlan lp;
     std::array<int, 7> ratio_sf{};
     std::array<float, 7> apm3{};

@@ -392,10 +392,10 @@ __global__ void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb, int n
 // n <= a < cap, and for every a if the call has failed.
 // Reads the scatter's output (rpos, rslot) and copies every particle not in
 // an active cell of >= 64 particles to pos4 / slot (k_pp_subsort places the
-// others).  Pairs-once pass (small > 0): the particles of active cells of at
-// most `small` particles, whose chunks evaluate their pairs one-sidedly, are
-// marked by a negative range (w = -range); every reader of w then takes |w|
-// as the range and w != 0 as active.
+// others).  small > 0 (pairs-once pass): the particles of active cells of at
+// most `small` particles are k_pp_sparse's: they get no chunks and are marked
+// by a negative range (w = -range); every reader of w then takes |w| as the
+// range and w != 0 as active.
 __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
                               const int* __restrict__ cell_start, const int* __restrict__ n_sorted,
@@ -417,7 +417,10 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
             const int mask = dense ? (1 << dense_lg) - 1 : 63;
             f = ((a - c0) & mask) == 0;
             if (dense && a == c0) dense_list[atomicAdd(ndense, 1)] = (int)c;
-            if (cn <= small) p.w = -p.w;
+            if (cn <= small) {
+                p.w = -p.w;
+                f = 0;
+            }
         }
         if (!dense) {
             pos4[a] = p;
@@ -798,6 +801,25 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
             P.react_scale = std::ldexp(1.0f, k);
         }
     }
+    // Small cells apart where a tile's grid is finer than its sparse subtiles
+    // need: from rcp 4 on (a stencil of 5^3 cells; at rcp 2 a cell holds 8
+    // particles at the mean density).  There the pass depends on it: a chunk
+    // per small cell would add its every reaction by an atomic of its own.
+    P.small = 0;
+    if (P.newton) {
+        bool fine = false, fits = true;
+        for (int t = 0; t < P.ntile; t++) {
+            fine = fine || T[t].rcp >= 4;
+            for (int q = 0; q < P.nsub3; q++) {
+                const int lv = P.iloc[t * P.nsub3 + q];
+                if (lv >= 1 && lv <= 7)
+                    fits = fits && pp_sparse_fits(T[t].rcp, apm3[lv - 1], g.p.ratio_cs);
+            }
+        }
+        // (cells of 64 and more are subsorted)
+        if (fine && fits) P.small = std::min((1 << pp_direct_lg()) / 2, 63);
+        P.newton = !fine || fits;
+    }
     if (split || P.newton) {
         C2_TRY(g_pp.term.reserve(P.cap * 3 * sizeof(float)));
         const int64_t rows = (int64_t)g.ntile * g.nt * g.nt;
@@ -1056,7 +1078,7 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
             k_chunk_flags<<<ceil_div(P.cap, 256), 256, 0, s>>>(
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cellid, A.cell_start,
                 n_sorted, &red->err, (int)P.cap, pp_dense_lg(P.newton),
-                P.newton ? (1 << pp_direct_lg()) / 2 : 0, flags, g_pp.dense.as<int>(),
+                P.small, flags, g_pp.dense.as<int>(),
                 &red->ndense, g_pp.pos4.as<float4>(), g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(flags, (int64_t)P.cap, g_pp.scan_tmp, s));
@@ -1092,7 +1114,13 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
             k_react_zero<<<2048, 256, 0, s>>>(A.react, n_sorted, (int)P.cap, &red->err);
             C2_HIP(hipGetLastError());
         }
-        C2_TRY(launch_pp_tiled(A, chunks, flags + P.cap, P.grid_pairs, P.mode, s));
+        if (P.small)
+            C2_TRY(launch_pp_sparse(A, d_rhoc, g.nt, g.ncb, (int)((int64_t)P.ntile * g.nt * g.nt * g.nt),
+                                    P.small, P.mode, s));
+        if (P.newton)
+            C2_TRY(launch_pp_newton(A, chunks, flags + P.cap, P.grid_pairs, P.small, P.mode, s));
+        else
+            C2_TRY(launch_pp_tiled(A, chunks, flags + P.cap, P.grid_pairs, P.mode, s));
         if (P.learned) C2_TRY(learned_enqueue(P.lp, A, g_pp.tile_first.as<int>(), s));
         if (P.newton) {
             Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));

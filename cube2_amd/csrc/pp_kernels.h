@@ -79,6 +79,17 @@ struct PPArgs {
 
 int launch_pp_pairs(const PPArgs& a, int mode, hipStream_t s);
 
+// Pairs-once pair kernel (pp_newton.hip) over the chunks; cells of at most
+// `small` particles are k_pp_sparse's (0: none).
+int launch_pp_newton(const PPArgs& a, const int* chunks, const int* nchunks, int grid, int small,
+                     int mode, hipStream_t s);
+
+// The small cells' particles of a pairs-once pass (pp_sparse.hip): nt coarse
+// cells per tile side and ncb halo ones, ncoarse physical coarse cells in all.
+bool pp_sparse_fits(int rcp, float range, int ratio_cs);
+int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int small,
+                     int mode, hipStream_t s);
+
 // Whether the pair kernel has a pairs-once variant for this PP mode.
 bool pp_newton_mode(int mode);
 
@@ -87,8 +98,8 @@ bool& pp_count_tiles();
 
 // log2 of the pair kernel's chunk size in PP cells of >= 64 particles: 16
 // built in, 32 with pairs once (half the reaction atomics, which share HBM
-// with the mesh kernels in the overlapped kick: at 256^3 the kick 112.3 ->
-// 111.4 ms, the pair kernel alone 64.5 -> 67.2 ms)
+// with the mesh kernels in the overlapped kick; at 256^3 16 and 64 are both
+// slower)
 inline int pp_dense_lg(bool newton) {
     const int v = ctx().tune[CUBE2_TUNE_PP_DENSE_LG];
     return v ? v : (newton ? 5 : 4);

@@ -223,11 +223,11 @@ __device__ inline void wave_lds_sync() { __builtin_amdgcn_wave_barrier(); }
 // Signed fixed point (value * scale, rounded to nearest) of a pairs-once
 // partial sum, added to a particle's 64-bit accumulator: integer adds
 // commute, so the totals do not depend on the order of the atomics.
-__device__ inline unsigned long long to_fixed(float v, float scale) {
-    return (unsigned long long)__double2ll_rn((double)v * (double)scale);
+__device__ inline unsigned long long to_fixed(double v, float scale) {
+    return (unsigned long long)__double2ll_rn(v * (double)scale);
 }
-__device__ inline void fixed_add(unsigned long long* dst, float v, float scale) {
-    if (v != 0.0f) atomicAdd(dst, to_fixed(v, scale));
+__device__ inline void fixed_add(unsigned long long* dst, double v, float scale) {
+    if (v != 0.0) atomicAdd(dst, to_fixed(v, scale));
 }
 
 }  // namespace cube2

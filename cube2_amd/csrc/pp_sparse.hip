@@ -1,0 +1,332 @@
+// Pairs-once pass: the particles of PP cells of at most `small` particles.
+//
+// The PP grid of a tile follows its densest subtile, so that in the sparse
+// subtiles beside a clump a PP cell holds one particle or none while its
+// stencil has up to 13^2 rows.  Taken as chunks of the pair kernel, a chunk
+// per cell, these particles (64% of C1's, 2.5% of its accepted pairs) cost
+// 11.1 M chunks of 25 to 169 rows each: half of that kernel's instructions
+// and most of its memory traffic (cell starts, and registers spilled around
+// each chunk).
+//
+// Here a wavefront takes a coarse cell: it lists the particles of its small
+// cells, up to 64 at a time, and walks the cells within R of any of them once
+// for all, each row of cells being read once instead of once per particle.  Every j of that
+// region is tested against every i (lane (i, s) takes j slot t + s); whether
+// j's cell lies in i's stencil, for the count of candidates, is one packed
+// comparison of cell coordinates.  Accepted pairs are queued in LDS and their
+// forces evaluated 64 at a time, summed per i as 64-bit fixed point (integer
+// LDS atomics; float ones cost ~190 cycles an instruction on gfx950).  These
+// particles evaluate all their pairs themselves and nothing else adds to
+// them (k_chunk_flags marks them), so their sums are stored, not added.
+// Bound by VALU issue: the region's tests.  The particles beside a clump cost
+// the most by far, one batch of them up to 1 ms; kParts wavefronts share a
+// coarse cell, so that such batches run side by side.  REF, clustered: 7.9 ms
+// at 256^3 (kParts 1: 12.1, 4: 7.9, 16: 11.7, empty parts counting), 2.0 ms
+// at 128^3 (3.8, 2.1, 1.9); the pair kernel falls from 57.8 to 32.4 and from
+// 7.8 to 3.9 ms.
+#include <algorithm>
+
+#include "common.h"
+#include "engine.h"
+#include "pp_kernels.h"
+#include "pp_law.h"
+#include "profile.h"
+#include "reduce.h"
+
+namespace cube2 {
+
+constexpr unsigned kOnes = 1u | 1u << 10 | 1u << 20;  // one in each packed coordinate
+constexpr unsigned kTop = 512u * kOnes;
+
+struct SparseLDS {
+    float4 q[kQ];             // accepted pairs (dx, dy, dz, r^2)
+    unsigned char qi[kQ];     // and their i slot
+    unsigned long long acc[64][3];
+    float4 jb[128];           // a batch of j (w: packed cell), then far-away ones
+    int list[128];            // sorted indices of small cells' particles
+    unsigned lcell[128];      // their cells (packed, in the coarse cell) and
+    unsigned short lblk[128]; // blocks
+    int rs[64], rp[64];       // row group: j = v + rs[k] for rp[k-1] <= v < rp[k]
+    unsigned rc[64];          // packed cell of a j of row k, less its cell id
+};
+
+template <int kMode>
+__device__ inline void sparse_flush(SparseLDS& L, int lane, int begin, int count, const FraK& Ka,
+                                    const FraK& Kr, float scale) {
+    if (lane < count) {
+        const int s = (begin + lane) & (kQ - 1);
+        const float4 e = L.q[s];
+        const int ii = L.qi[s];
+        float f[3];
+        pair_force<kMode>(e, Ka, Kr, f[0], f[1], f[2]);
+#pragma unroll
+        for (int c = 0; c < 3; c++) atomicAdd(&L.acc[ii][c], to_fixed(f[c], scale));
+    }
+    wave_lds_sync();
+}
+
+// n / d as the high word of n * recip(d), exact for n d < 2^32.
+__device__ inline unsigned recip_u32(unsigned d) { return 0xffffffffu / d + 1u; }
+__device__ inline int quot(int n, unsigned recip) { return (int)__umulhi((unsigned)n, recip); }
+
+// Mean particles of a block (below): small blocks walk less that only one of
+// their particles needs, large ones read rows less often (at 256^3 with one
+// wavefront per coarse cell 4: 17.1 ms, 8: 13.0, 16: 12.1, 32: 13.2).
+constexpr float kBlockCount = 16.0f;
+// Wavefronts that share a coarse cell's blocks.
+constexpr int kParts = 8;
+
+template <int kMode>
+__global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __restrict__ rhoc, int nt,
+                                                      int ncb, int ncoarse, int small) {
+    __shared__ SparseLDS lds[4];
+    const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    SparseLDS& L = lds[wave];
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const FraK Ka = uni(make_frak(A.app));
+    unsigned long long pc = 0, pa = 0;  // (wavefront-uniform)
+    const int nw = A.red->err == 0 ? ncoarse * kParts : 0;
+    // neighbouring coarse cells share most of their j: one XCD takes a run
+    for (int w = (int)xcd_remap(blockIdx.x, gridDim.x) * 4 + wave; w < nw; w += gridDim.x * 4) {
+        const int cw = w / kParts, part = w % kParts;
+        const int t = cw / (nt * nt * nt), wr = cw - t * nt * nt * nt;
+        const PPTile T = A.tiles[t];
+        const int S = T.S, rcp = T.rcp;
+        const int bx = (wr % nt + 1) * rcp, by = (wr / nt % nt + 1) * rcp, bz = (wr / (nt * nt) + 1) * rcp;
+        const unsigned off = (unsigned)T.cell_off;
+        // mean count of the 27 coarse cells around -> side of a block
+        float mean = 0.0f;
+        {
+            const int nte = nt + 2 * ncb, l = min(lane, 26);
+            const size_t cc = (((size_t)t * nte + wr / (nt * nt) + ncb - 1 + l / 9) * nte + wr / nt % nt +
+                               ncb - 1 + l / 3 % 3) * nte + wr % nt + ncb - 1 + l % 3;
+            int c = lane < 27 ? rhoc[cc] : 0;
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+            mean = (float)uni(c) * (1.0f / 27.0f);
+        }
+        const int nb1 = min(rcp, max(1, (int)ceilf(cbrtf(mean * (1.0f / kBlockCount)))));
+        const int Bs = uni((rcp + nb1 - 1) / nb1), nbl = (rcp + Bs - 1) / Bs;  // blocks of Bs^3 cells
+        const int nblk = nbl * nbl * nbl, cblk = Bs * Bs * Bs;  // blocks, cells of one
+        const int ncell = nblk * (part + 1) / kParts * cblk;
+        const unsigned i1 = recip_u32(Bs), i2 = recip_u32(Bs * Bs), i3 = recip_u32(Bs * Bs * Bs);
+        const unsigned k1 = recip_u32(nbl), k2 = recip_u32(nbl * nbl);
+        const unsigned long long pc0 = pc, pa0 = pa;
+        int c0 = nblk * part / kParts * cblk, depth = 0, n = 0, first = 0, blk = 0, head = 0, tail = 0;
+        unsigned cpk = 0;
+        float range = 0.0f;
+        FraK Kr = Ka;
+        int R = 0;
+        float pp2 = 0.0f;
+        for (;;) {
+            // list the small cells' particles, the depth-th of 64 cells at a time
+            while (tail - head < 64 && c0 < ncell) {
+                if (depth == 0) {
+                    n = 0;
+                    const int c = c0 + lane;
+                    if (c < ncell) {
+                        // (block, cell in it) -> cell of the coarse cell
+                        blk = Bs > 1 ? quot(c, i3) : c;
+                        const int r = c - blk * Bs * Bs * Bs;
+                        const int kz = nbl > 1 ? quot(blk, k2) : blk, kzy = nbl > 1 ? quot(blk, k1) : blk;
+                        const int rz = Bs > 1 ? quot(r, i2) : r, rzy = Bs > 1 ? quot(r, i1) : r;
+                        const int z = kz * Bs + rz, y = (kzy - kz * nbl) * Bs + rzy - rz * Bs,
+                                  x = (blk - kzy * nbl) * Bs + r - rzy * Bs;
+                        if (z < rcp && y < rcp && x < rcp) {
+                            const unsigned cell = off + ((unsigned)(bz + z) * S + by + y) * S + bx + x;
+                            first = A.cell_start[cell];
+                            n = A.cell_start[cell + 1] - first;
+                            if (n > small) n = 0;
+                            cpk = (unsigned)z << 20 | (unsigned)y << 10 | (unsigned)x;
+                        }
+                    }
+                }
+                const uint64_t m = __ballot(n > depth);
+                if (n > depth) {
+                    const int at = (tail + __popcll(m & lt)) & 127;
+                    L.list[at] = first + depth;
+                    L.lcell[at] = cpk;
+                    L.lblk[at] = (unsigned short)blk;
+                }
+                tail += __popcll(m);
+                depth++;
+                if (!__ballot(n > depth)) {
+                    depth = 0;
+                    c0 += 64;
+                }
+            }
+            wave_lds_sync();
+            if (tail == head) break;
+            // the batch: the listed particles of the first one's block
+            const int b0 = uni((int)L.lblk[head & 127]);
+            const uint64_t same = __ballot(head + lane < tail && L.lblk[(head + lane) & 127] == b0);
+            const int ni = ~same ? __ffsll((unsigned long long)~same) - 1 : 64;
+            int lgI = 0;
+            while ((1 << lgI) < ni) lgI++;
+            const int I = 1 << lgI, J = 64 >> lgI;
+            const int islot = lane & (I - 1), jslot = lane >> lgI;
+            const bool vi = islot < ni;
+            const int at = (head + (vi ? islot : 0)) & 127, ia = L.list[at];
+            const unsigned cell = L.lcell[at];
+            head += ni;
+            const float4 p = A.pos4[ia];
+            if (range == 0.0f) {  // one subtile per coarse cell: one range
+                range = fabsf(uni(p.w));
+                if (range == 0.0f || (A.learned_occ && range == A.learned_range)) break;
+                R = (int)ceilf(__fmul_rn(range, (float)rcp) / (float)A.ratio_cs);
+                pp2 = __fmul_rn(range, range);
+                Kr = uni(make_frak(range));
+            }
+            // cells relative to the origin (bx, by, bz) - R; j's cell is in i's
+            // stencil iff each coordinate of (j - i + R) and of (i - j + R) is
+            // not negative: with 512 added to each, iff its top bit stays
+            // (|j - i| + R < 512)
+            const int X0 = bx - R, Y0 = by - R, Z0 = bz - R;
+            const unsigned lo = cell - kTop, hi = cell + 2u * (unsigned)R * kOnes + kTop;
+            // the region: the block's cells and R around them
+            const int kz = b0 / (nbl * nbl), ky = b0 / nbl % nbl, kx = b0 % nbl;
+            const int xa = max(X0 + kx * Bs, 0), xb = min(bx + min(kx * Bs + Bs, rcp) - 1 + R, S - 1);
+            const int ya = max(Y0 + ky * Bs, 0), yb = min(by + min(ky * Bs + Bs, rcp) - 1 + R, S - 1);
+            const int za = max(Z0 + kz * Bs, 0), zb = min(bz + min(kz * Bs + Bs, rcp) - 1 + R, S - 1);
+            const int ny = yb - ya + 1, nrows = ny * (zb - za + 1);
+            const unsigned inv_ny = recip_u32(ny);
+            const uint64_t vim = __ballot(vi);
+            const float pix = vi ? p.x : -kFar, piy = vi ? p.y : -kFar, piz = vi ? p.z : -kFar;
+            for (int q = lane; q < 64 * 3; q += 64) (&L.acc[0][0])[q] = 0ull;
+            int qhead = 0, qtail = 0;
+            for (int rg = 0; rg < nrows; rg += 64) {
+                int js = 0, cnt = 0;
+                const int r = rg + lane;
+                if (r < nrows) {
+                    const int rz = ny > 1 ? quot(r, inv_ny) : r;
+                    const int zz = za + rz, yy = ya + r - rz * ny;
+                    const unsigned row = off + ((unsigned)zz * S + yy) * S;
+                    js = A.cell_start[row + xa];
+                    cnt = A.cell_start[row + xb + 1] - js;
+                    L.rc[lane] = ((unsigned)(zz - Z0) << 20 | (unsigned)(yy - Y0) << 10) - row - (unsigned)X0;
+                }
+                int inc = cnt;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int u = __shfl_up(inc, o, 64);
+                    if (lane >= o) inc += u;
+                }
+                const int M = uni(__shfl(inc, 63, 64));
+                L.rs[lane] = js - (inc - cnt);
+                L.rp[lane] = inc;
+                wave_lds_sync();
+                int frow = 0;  // (a lane's candidates only grow: its row walks forward)
+                unsigned rc = 0, jc = 0;
+                auto fetch = [&](int vb) {
+                    const int v = vb + lane;
+                    float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (v < M) {
+                        while (L.rp[frow] <= v) frow++;
+                        const int jx = v + L.rs[frow];
+                        q4 = A.pos4[jx];
+                        jc = A.cellid[jx];
+                        rc = L.rc[frow];
+                    }
+                    return q4;
+                };
+                float4 qc = fetch(0);
+                for (int vb = 0; vb < M; vb += 64) {
+                    const int nb = min(64, M - vb);
+                    qc.w = __uint_as_float(rc + jc);
+                    L.jb[lane] = qc;
+                    wave_lds_sync();
+                    // past the batch: far away and in no stencil
+                    L.jb[nb + lane] = make_float4(kFar, kFar, kFar, __uint_as_float(511u * kOnes));
+                    wave_lds_sync();
+                    if (vb + 64 < M) qc = fetch(vb + 64);
+                    // lane's pair with the j at slot u: its vector, r^2, whether
+                    // it pairs; candidates counted
+                    auto test = [&](const float4& qj, float4& e) {
+#pragma clang fp contract(off)
+                        e.x = qj.x - pix;
+                        e.y = qj.y - piy;
+                        e.z = qj.z - piz;
+                        e.w = e.x * e.x + e.y * e.y + e.z * e.z;
+                        const unsigned jk = __float_as_uint(qj.w);
+                        pc += __popcll(__ballot(((jk - lo) & (hi - jk) & kTop) == kTop) & vim);
+                        return (e.w > 0.0f) & (e.w < pp2);
+                    };
+                    auto append = [&](bool ok, const float4& e) {
+                        const uint64_t m = __ballot(ok);
+                        if (!m) return;
+                        if (ok) {
+                            const int s = (qtail + __popcll(m & lt)) & (kQ - 1);
+                            L.q[s] = e;
+                            L.qi[s] = (unsigned char)islot;
+                        }
+                        qtail += __popcll(m);
+                        if (qtail - qhead >= 64) {
+                            wave_lds_sync();
+                            sparse_flush<kMode>(L, lane, qhead, 64, Ka, Kr, A.react_scale);
+                            qhead += 64;
+                        }
+                    };
+                    if (J <= 16) {  // (4 J slots past the batch's last are set)
+                        for (int u = 0; u < nb; u += 4 * J) {
+                            float4 qj[4], e[4];
+                            bool ok[4];
+#pragma unroll
+                            for (int k = 0; k < 4; k++) qj[k] = L.jb[u + k * J + jslot];
+#pragma unroll
+                            for (int k = 0; k < 4; k++) ok[k] = test(qj[k], e[k]);
+#pragma unroll
+                            for (int k = 0; k < 4; k++) append(ok[k], e[k]);
+                        }
+                    } else {
+                        for (int u = 0; u < nb; u += J) {
+                            float4 e;
+                            const bool ok = test(L.jb[u + jslot], e);
+                            append(ok, e);
+                        }
+                    }
+                    wave_lds_sync();  // jb is rewritten by the next batch
+                }
+            }
+            wave_lds_sync();
+            if (qtail > qhead) sparse_flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr, A.react_scale);
+            pa += (unsigned)qtail;
+            pc -= (unsigned)ni;  // the particles themselves
+            if (vi && jslot == 0)
+#pragma unroll
+                for (int c = 0; c < 3; c++) A.react[3 * (size_t)ia + c] = L.acc[islot][c];
+            wave_lds_sync();  // acc, the queue and the list are reused
+        }
+        if (A.tile_pairs && lane == 0) {  // per-tile counts (on request only)
+            atomicAdd(&A.tile_pairs[2 * t], pc - pc0);
+            atomicAdd(&A.tile_pairs[2 * t + 1], pa - pa0);
+        }
+    }
+    const unsigned long long sm[2] = {lane == 0 ? pc : 0ull, lane == 0 ? pa : 0ull};
+    block_sum_to<2>(&A.red->p_cand, sm);
+}
+
+// Largest stencil radius and PP cells per coarse cell whose packed cell
+// coordinates fit (rcp + 3 R < 512); beyond it the pass is not pairs-once.
+bool pp_sparse_fits(int rcp, float range, int ratio_cs) {
+    const double R = std::ceil((double)range * rcp / ratio_cs) + 1.0;
+    return R < 512.0 && rcp + 3.0 * R < 512.0;
+}
+
+int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int small,
+                     int mode, hipStream_t s) {
+    if (ncoarse <= 0) return CUBE2_OK;
+    Stage st("pp_pairs_sparse");
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        ncu = 256;
+    // as the pair kernel's: far more blocks than are resident, so that the
+    // hardware balances their uneven costs
+    const unsigned blocks = (unsigned)std::min(ceil_div((size_t)ncoarse * kParts, 4), (unsigned)std::max(1, ncu) * 64u);
+    if (mode == CUBE2_PP_REF) k_pp_sparse<kModeRef><<<blocks, 256, 0, s>>>(a, rhoc, nt, ncb, ncoarse, small);
+    else k_pp_sparse<kModeFast><<<blocks, 256, 0, s>>>(a, rhoc, nt, ncb, ncoarse, small);
+    C2_HIP(hipGetLastError());
+    return CUBE2_OK;
+}
+
+}  // namespace cube2

@@ -1,11 +1,12 @@
-// PP pair kernel.
+// PP pair kernel of the ordered passes (every i sums all its pairs; the
+// pairs-once pass is pp_newton.hip).
 //
 // Wavefronts take chunks of physical particles of one PP cell by a static
 // stride (a grid of 64 blocks per CU, far more than are resident, so that
 // the hardware balances the chunks' uneven costs): the whole cell if it
-// holds fewer than 64, else 2^dense_lg at a time (16 built in, 32 with pairs
-// once).  The lanes are split into I i-slots x J j-slots (I the chunk
-// size rounded up to a power of two, I*J = 64).  The j of the (2R+1)^2
+// holds fewer than 64, else 2^dense_lg at a time (16 built in).  The lanes
+// are split into I i-slots x J j-slots (I the chunk size rounded up to a
+// power of two, I*J = 64).  The j of the (2R+1)^2
 // neighbour rows are contiguous runs of the sorted particle stream; a
 // wavefront concatenates them into one candidate list and fetches it 64 at
 // a time (one coalesced load, prefetched a batch ahead, staged in LDS).
@@ -28,9 +29,7 @@
 //   representable or at least 2^-49 (relative) away from every rounding
 //   midpoint, so this equals IEEE a/b.  The pair forces are bit-identical to
 //   the reference; only the order of the per-i sums differs (<= ~4e-7
-//   relative RMS), and with pairs once (kNewton, below) a pair of one range
-//   is evaluated once and its force summed for both particles in 64-bit
-//   fixed point.
+//   relative RMS).
 // FAST: FMA/rsqrt arithmetic with F_ra in Horner form.
 // PLUMMER: Plummer softening r/(r^2 + app^2)^(3/2) in place of F_ra(r, app)
 //   (no counterpart in the reference), in PRECISE's arithmetic.
@@ -50,28 +49,19 @@
 
 namespace cube2 {
 
-template <int kMode, int kJB = 64, bool kNewton = false>
+template <int kMode, int kJB = 64>
 struct WaveLDS {
     using Acc = typename std::conditional<kMode == kModePrecise || kMode == kModePlummer, double,
                                           float>::type;
     float4 q[kQ];           // queued chunks: accepted pairs (dx, dy, dz, r^2)
     unsigned char qi[kQ];   // and their i slot
     Acc acc[64][3];         // per-i force sums
-    // current batch of j positions, then J far-away ones; pairs once: two
-    // blocks of 64 j, the first 32 of each repeated after it
-    float4 jb[kNewton ? 192 : kJB + 64];
+    float4 jb[kJB + 64];    // current batch of j positions, then J far-away ones
     int rs[64], rp[64];     // row group: j = v + rs[k] for rp[k-1] <= v < rp[k]
 };
 
-constexpr int kJBlock = 96;  // a block of 64 j and the repeats
-// x from the next higher lane, lane 63 from lane 0 (DPP, folded into the add
-// that uses it).  Every lane must be active.
-__device__ inline float wave_rol1(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x134, 0xf, 0xf, true));
-}
-
-template <int kMode, int kJB, bool kN>
-__device__ inline void flush(WaveLDS<kMode, kJB, kN>& L, int lane, int begin, int count,
+template <int kMode, int kJB>
+__device__ inline void flush(WaveLDS<kMode, kJB>& L, int lane, int begin, int count,
                              const FraK& Ka, const FraK& Kr) {
     if (lane < count) {
         const int s = (begin + lane) & (kQ - 1);
@@ -79,7 +69,7 @@ __device__ inline void flush(WaveLDS<kMode, kJB, kN>& L, int lane, int begin, in
         const int ii = L.qi[s];
         float fx, fy, fz;
         pair_force<kMode>(e, Ka, Kr, fx, fy, fz);
-        using Acc = typename WaveLDS<kMode, kJB, kN>::Acc;
+        using Acc = typename WaveLDS<kMode, kJB>::Acc;
         atomicAdd(&L.acc[ii][0], (Acc)fx);
         atomicAdd(&L.acc[ii][1], (Acc)fy);
         atomicAdd(&L.acc[ii][2], (Acc)fz);
@@ -104,15 +94,15 @@ __device__ inline int find_tile2(const PPTile* __restrict__ T, int ntile, uint32
 // budgets for 5 and 7 wavefronts 89.2 and 86.0 ms; 4 blocks per CU instead
 // of 6: 105 ms).  The REF variant spills a few registers outside its inner
 // loops.
-template <int kMode, int kJB, bool kNewton>
+template <int kMode, int kJB>
 __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __restrict__ chunks,
                                                   const int* __restrict__ nchunks_dev,
                                                   int direct_lg, int dense_lg) {
     static_assert(kJB == 64 || kJB == 128, "j batch of 64 or 128");
     constexpr int kH = kJB / 64;  // fetched float4 per lane per batch
-    __shared__ WaveLDS<kMode, kJB, kNewton> lds[4];
+    __shared__ WaveLDS<kMode, kJB> lds[4];
     const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    WaveLDS<kMode, kJB, kNewton>& L = lds[wave];
+    WaveLDS<kMode, kJB>& L = lds[wave];
     const int nchunks = uni(*nchunks_dev);
 
     float f2 = 0.f, v0 = 0.f, v1 = 0.f, v2 = 0.f;
@@ -140,9 +130,8 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         const long long key = (long long)cid - T.cell_off;
         const int S = T.S;
         const int x = (int)(key % S), y = (int)((key / S) % S), z = (int)(key / ((long long)S * S));
-        // one subtile per PP cell: same range for the chunk (w < 0 marks the
-        // pairs-once pass's small cells)
-        const float range = fabsf(uni(p.w));
+        // one subtile per PP cell: same range for the chunk
+        const float range = uni(p.w);
         // learned kick: the network stands in for the sparse level-2 cells
         if (A.learned_occ && range == A.learned_range && cend - cbeg < A.learned_occ) continue;
         int R;
@@ -157,33 +146,10 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         wave_lds_sync();
         const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
         int qhead = 0, qtail = 0;
-        // pairs once: chunks of cells of more than 2^(direct_lg-1) particles
-        // (each such cell's chunks alike, k_chunk_flags marks the others)
-        const bool direct = kNewton ? cend - cbeg > (1 << direct_lg) / 2 : lgI >= direct_lg;
-        const bool nwc = kNewton && direct;
-        using Acc = typename WaveLDS<kMode, kJB, kNewton>::Acc;
-        // Pairs once (kNewton): a j of the chunk's own range in a cell of
-        // more than 2^(direct_lg-1) particles is an active particle of the
-        // same tile and level, an i of a chunk of this kind whose stencil
-        // holds this chunk's cell; of the two, the one with the lower sorted
-        // index evaluates the pair and adds the force to both (the pair force
-        // is exactly antisymmetric: RN(a - b) = -RN(b - a)).  Other j (halo
-        // copies, other levels, small cells) act on i alone, and the chunks
-        // of small cells evaluate all their pairs themselves.  A chunk whose
-        // stencil lies inside its own subtile meets only j of its own range,
-        // so it skips the rows and cells before its own.
-        bool interior = false;
-        if (nwc) {
-            const int cps = A.ntt * T.rcp, span = S - 2 * T.rcp;
-            auto inside = [&](int c) {
-                const int lo = c - R - T.rcp, hi = c + R - T.rcp;
-                return lo >= 0 && hi < span && lo / cps == hi / cps;
-            };
-            interior = inside(x) && inside(y) && inside(z);
-        }
+        const bool direct = lgI >= direct_lg;
+        using Acc = typename WaveLDS<kMode, kJB>::Acc;
         Acc dax = 0, day = 0, daz = 0;
         unsigned npa = 0;
-        int jhead = 0, jtail = 0;  // pairs once: kept j taken and staged
         // direct chunks: bounding box of the chunk's i; a j farther than the
         // range from the box cannot pair with any of them (the 1e-4 relative
         // margin keeps every j the per-pair test could accept)
@@ -214,7 +180,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         // the group's runs form one virtual list of M candidates, fetched 64
         // at a time with one coalesced load, prefetched a batch ahead.
         for (int rg = 0; rg < nrows; rg += 64) {
-            int js = 0, cnt = 0, cfull = 0;
+            int js = 0, cnt = 0;
             const int r = rg + lane;
             if (r < nrows) {
                 const int zz = z + r / W - R, yy = y + r % W - R;
@@ -222,26 +188,6 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                     const long long row = T.cell_off + ((long long)zz * S + yy) * S;
                     js = A.cell_start[row + xlo];
                     cnt = A.cell_start[row + xhi + 1] - js;
-                    cfull = cnt;
-                    if (kNewton && interior && zz * S + yy <= z * S + y) {
-                        // rows before the chunk's: none; its own row: from its
-                        // first i -- unless a small cell lies there, whose j
-                        // act on this chunk's i only from here
-                        const bool own = zz * S + yy == z * S + y;
-                        const int xe = own ? x : xhi + 1, small = (1 << direct_lg) / 2;
-                        bool has_small = false;
-                        int c0 = js;
-                        for (int xc = xlo; xc < xe; xc++) {
-                            const int c1 = A.cell_start[row + xc + 1];
-                            has_small |= c1 - c0 > 0 && c1 - c0 <= small;
-                            c0 = c1;
-                        }
-                        if (!has_small) {
-                            const int j0 = own ? a0 : js + cnt;
-                            cnt -= j0 - js;
-                            js = j0;
-                        }
-                    }
                 }
             }
             int inc = cnt;
@@ -254,126 +200,28 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             L.rs[lane] = js - (inc - cnt);
             L.rp[lane] = inc;
             wave_lds_sync();
-            if (kNewton && interior) {  // the candidates counted: the whole stencil
-                int sf = cfull;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) sf += __shfl_xor(sf, o, 64);
-                if (vi && jslot == 0) pc += (unsigned long long)sf;
-            } else if (vi && jslot == 0) {
-                pc += (unsigned long long)M;
-            }
+            if (vi && jslot == 0) pc += (unsigned long long)M;
             // a lane's candidates v = vb + lane only grow, so its row (the
             // first with rp > v) is found by walking forward from the last
             // one: rp of the rows past the group is M > v, so the walk stops
             // inside the group
             int frow = 0;
-            auto fetch = [&](int vb, int& jx) {
+            auto fetch = [&](int vb) {
                 const int v = vb + lane;
                 float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (v < M) {
                     while (L.rp[frow] <= v) frow++;
-                    jx = v + L.rs[frow];
-                    q4 = A.pos4[jx];
+                    q4 = A.pos4[v + L.rs[frow]];
                 }
                 return q4;
             };
             // a batch is kJB candidates, kH fetches of 64; the next batch's
             // fetches are issued before this batch's pairs run
             float4 qcur[kH];
-            int jcur[kH] = {};
 #pragma unroll
-            for (int h = 0; h < kH; h++) qcur[h] = fetch(64 * h, jcur[h]);
-            // (pairs once: a last step without candidates for the j left over)
-            const bool last = nwc && rg + 64 >= nrows;
-            const int vend = last ? (M + kJB - 1) / kJB * kJB + kJB : M;
-            for (int vb = 0; vb < vend; vb += kJB) {
+            for (int h = 0; h < kH; h++) qcur[h] = fetch(64 * h);
+            for (int vb = 0; vb < M; vb += kJB) {
                 int nb = 0;
-                if (nwc) {
-                    // Keep the j near the chunk's box that no chunk before this
-                    // one's evaluates (a j of the chunk's range before its
-                    // first i does) and collect 64 of them.  Then, at step s,
-                    // lane l takes j (l + s) mod 64: over the I steps each j
-                    // meets I consecutive lanes, every i once, and its
-                    // reaction moves along with it (rotated one lane per step
-                    // by the DPP operand of the add that sums it), so that 64
-                    // j cost I steps of one pair per lane and three additions.
-                    // (Summing a j's reaction over the lanes of one step
-                    // instead took 18 instructions more per step.)
-#pragma unroll
-                    for (int h = 0; h < kH; h++) {
-                        float4 qh = qcur[h];
-                        // w = the sorted index of a j of the chunk's range,
-                        // INT_MAX for a j that acts on i alone
-                        const int jx = qh.w == range ? jcur[h] : INT_MAX;
-                        qh.w = __int_as_float(jx);
-                        const float ex = fmaxf(fmaxf(bx0 - qh.x, qh.x - bx1), 0.0f);
-                        const float ey = fmaxf(fmaxf(by0 - qh.y, qh.y - by1), 0.0f);
-                        const float ez = fmaxf(fmaxf(bz0 - qh.z, qh.z - bz1), 0.0f);
-                        const bool keep = (vb + 64 * h + lane < M) & (jx >= a0) &
-                                          (ex * ex + ey * ey + ez * ez < pp2m);
-                        const uint64_t km = __ballot(keep);
-                        if (keep) {
-                            const int t = jtail + __popcll(km & lt);
-                            const int at = (t >> 6 & 1) * kJBlock + (t & 63);
-                            L.jb[at] = qh;
-                            if ((t & 63) < 32) L.jb[at + 64] = qh;
-                        }
-                        jtail += __popcll(km);
-                        if (h == kH - 1) {
-#pragma unroll
-                            for (int k = 0; k < kH; k++)
-                                if (vb + kJB + 64 * k < M) qcur[k] = fetch(vb + kJB + 64 * k, jcur[k]);
-                        }
-                        const bool rest = last && vb + kJB >= vend && h == kH - 1;
-                        if (jtail - jhead < 64 && !(rest && jtail > jhead)) continue;
-                        const int bb = (jhead >> 6 & 1) * kJBlock;
-                        if (rest && lane >= jtail - jhead) {  // far-away j to the block's end
-                            const float4 far4 = make_float4(kFar, kFar, kFar, __int_as_float(INT_MAX));
-                            L.jb[bb + lane] = far4;
-                            if (lane < 32) L.jb[bb + lane + 64] = far4;
-                        }
-                        wave_lds_sync();
-                        float rx = 0.0f, ry = 0.0f, rz = 0.0f;
-                        for (int s0 = 0; s0 < I; s0 += 32) {
-                            const float4* jp = &L.jb[bb + ((lane + s0) & 63)];
-                            const int ns = uni(min(32, I - s0));
-                            for (int s = 0; s < ns; s++, jp++) {
-#pragma clang fp contract(off)
-                                const float4 qj = *jp;
-                                const int jw = __float_as_int(qj.w);
-                                float4 e;
-                                e.x = qj.x - pix;
-                                e.y = qj.y - piy;
-                                e.z = qj.z - piz;
-                                e.w = e.x * e.x + e.y * e.y + e.z * e.z;
-                                const bool ok = (e.w > 0.0f) & (e.w < pp2) & (jw > ia);
-                                const uint64_t okm = __ballot(ok);
-                                npa += 2 * __popcll(okm) - __popcll(okm & __ballot(jw == INT_MAX));
-                                float fx = 0.0f, fy = 0.0f, fz = 0.0f;
-                                if (ok) {
-                                    pair_force<kMode>(e, Ka, Kr, fx, fy, fz);
-                                    dax += (Acc)fx;
-                                    day += (Acc)fy;
-                                    daz += (Acc)fz;
-                                }
-                                rx = wave_rol1(rx) + fx;
-                                ry = wave_rol1(ry) + fy;
-                                rz = wave_rol1(rz) + fz;
-                            }
-                        }
-                        // lane l now holds the reaction of j (l + I - 1) mod 64
-                        const int jw = __float_as_int(L.jb[bb + ((lane + I - 1) & 63)].w);
-                        if (jw != INT_MAX) {
-                            unsigned long long* d = A.react + 3 * (size_t)jw;
-                            fixed_add(d, -rx, A.react_scale);
-                            fixed_add(d + 1, -ry, A.react_scale);
-                            fixed_add(d + 2, -rz, A.react_scale);
-                        }
-                        jhead += 64;
-                        wave_lds_sync();
-                    }
-                    continue;
-                }
                 if (direct) {  // keep the j near the chunk's box, compacted
 #pragma unroll
                     for (int h = 0; h < kH; h++) {
@@ -398,7 +246,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                 wave_lds_sync();
 #pragma unroll
                 for (int h = 0; h < kH; h++)
-                    if (vb + kJB + 64 * h < M) qcur[h] = fetch(vb + kJB + 64 * h, jcur[h]);
+                    if (vb + kJB + 64 * h < M) qcur[h] = fetch(vb + kJB + 64 * h);
                 // (i, j) of slot t: the difference vector and whether it pairs
                 // (branch-free: slots past the batch hold far-away j, and an
                 // i slot past the chunk tests from a far-away i)
@@ -458,19 +306,12 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                 atomicAdd(&L.acc[islot][1], day);
                 atomicAdd(&L.acc[islot][2], daz);
             }
-            if (!nwc || lane == 0) pa += npa;  // (pairs once: the wavefront's count)
+            pa += npa;
             wave_lds_sync();
         }
         if (qtail > qhead) flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr);
         if (lane == 0) pa += (unsigned long long)qtail;
-        if (kNewton && vi && jslot == 0) {
-            pc -= 1;  // the particle itself
-            // the i's own sums join its reactions; k_pp_newton_terms forms
-            // the velocity term once every chunk has added to it
-#pragma unroll
-            for (int c = 0; c < 3; c++)
-                fixed_add(A.react + 3 * (size_t)ia + c, (float)L.acc[islot][c], A.react_scale);
-        } else if (vi && jslot == 0) {
+        if (vi && jslot == 0) {
 #pragma clang fp contract(off)
             pc -= 1;  // the particle itself
             const int a = ia;
@@ -546,18 +387,14 @@ static void launch_pp_tiled_jb(const PPArgs& a, const int* chunks, const int* nc
                                unsigned blocks, int mode, int direct_lg, int dense_lg,
                                hipStream_t s) {
     const int dl = direct_lg, gl = dense_lg;
-    if (a.react && mode == CUBE2_PP_REF)
-        k_pp_tiled<kModeRef, kJB, true><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
-    else if (a.react && mode == CUBE2_PP_FAST)
-        k_pp_tiled<kModeFast, kJB, true><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
-    else if (mode == CUBE2_PP_REF)
-        k_pp_tiled<kModeRef, kJB, false><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
+    if (mode == CUBE2_PP_REF)
+        k_pp_tiled<kModeRef, kJB><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
     else if (mode == CUBE2_PP_FAST)
-        k_pp_tiled<kModeFast, kJB, false><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
+        k_pp_tiled<kModeFast, kJB><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
     else if (mode == CUBE2_PP_PLUMMER)
-        k_pp_tiled<kModePlummer, kJB, false><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
+        k_pp_tiled<kModePlummer, kJB><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
     else
-        k_pp_tiled<kModePrecise, kJB, false><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
+        k_pp_tiled<kModePrecise, kJB><<<blocks, 256, 0, s>>>(a, chunks, nchunks, dl, gl);
 }
 
 int launch_pp_tiled(const PPArgs& a, const int* chunks, const int* nchunks, int grid, int mode,
@@ -570,7 +407,7 @@ int launch_pp_tiled(const PPArgs& a, const int* chunks, const int* nchunks, int 
     const unsigned blocks = (unsigned)std::max(1, grid);
     // chunks of more than 2 particles sum directly unless tuned otherwise
     const int direct_lg = pp_direct_lg();
-    const int dense_lg = pp_dense_lg(a.react != nullptr);
+    const int dense_lg = pp_dense_lg(false);
     if (pp_jbatch() == 128)
         launch_pp_tiled_jb<128>(a, chunks, nchunks, blocks, mode, direct_lg, dense_lg, s);
     else

@@ -123,6 +123,8 @@ int cube2_set_pp_mode(int mode);
  *                     balances the chunks' uneven costs);
  *   PP_DIRECT_LG      1..7, chunks of > 2^(v-1) particles (lanes for >= 2^v
  *                     i slots) sum directly, smaller ones queue pairs (2);
+ *                     where PP_NEWTON evaluates pairs once, cells of at most
+ *                     2^(v-1) particles are taken by coarse cells instead;
  *   FFT_MIN_LGC       1..6, minimum log2 column-tile width of the y/z FFT
  *                     passes (built-in: ~2048 LDS elements per tile);
  *   INTERP_SEG        1..32, particles per wavefront work item of the mesh
