@@ -392,14 +392,16 @@ __global__ void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb, int n
 // n <= a < cap, and for every a if the call has failed.
 // Reads the scatter's output (rpos, rslot) and copies every particle not in
 // an active cell of >= 64 particles to pos4 / slot (k_pp_subsort places the
-// others).  small > 0 (pairs-once pass): the particles of active cells of at
-// most `small` particles are k_pp_sparse's: they get no chunks and are marked
-// by a negative range (w = -range); every reader of w then takes |w| as the
-// range and w != 0 as active.
+// others).  No chunks for the particles of active cells of at most `small`
+// particles (k_pp_sparse's) or, in the learned kick, of fewer than occ in
+// subtiles of range occ_range (the network's).  A pairs-once pass (newton)
+// marks both by a negative range (w = -range): to other i they are one-sided
+// sources; every reader of w then takes |w| as the range and w != 0 as active.
 __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
                               const int* __restrict__ cell_start, const int* __restrict__ n_sorted,
-                              const int* __restrict__ err, int cap, int dense_lg, int small,
+                              const int* __restrict__ err, int cap, int dense_lg, int small, int occ,
+                              float occ_range, int newton,
                               int* __restrict__ flags, int* __restrict__ dense_list,
                               int* __restrict__ ndense, float4* __restrict__ pos4,
                               uint32_t* __restrict__ slot) {
@@ -417,9 +419,9 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
             const int mask = dense ? (1 << dense_lg) - 1 : 63;
             f = ((a - c0) & mask) == 0;
             if (dense && a == c0) dense_list[atomicAdd(ndense, 1)] = (int)c;
-            if (cn <= small) {
-                p.w = -p.w;
+            if (cn <= small || (cn < occ && p.w == occ_range)) {
                 f = 0;
+                if (newton) p.w = -p.w;
             }
         }
         if (!dense) {
@@ -793,7 +795,7 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
     // below 2^62 for 2^k <= 2^62 / (10 / app^2 * cap); at 256^3 (app 0.06)
     // k = 24, a resolution of 6e-8 against forces of order 1 to 1e3.
     P.newton = false;
-    if (pp_newton_on() && pp_newton_mode(P.mode) && !learned && g.p.app > 0.0) {
+    if (pp_newton_on() && pp_newton_mode(P.mode) && g.p.app > 0.0) {
         const double bound = 10.0 / (g.p.app * g.p.app) * (double)P.cap;
         const int k = std::min(40, (int)std::floor(62.0 - std::log2(bound)));
         if (k >= 12) {
@@ -819,6 +821,13 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
         // (cells of 64 and more are subsorted)
         if (fine && fits) P.small = std::min((1 << pp_direct_lg()) / 2, 63);
         P.newton = !fine || fits;
+        // learned: the network's cells hold more than `small` and are not
+        // subsorted, so that k_chunk_flags can mark them
+        const int occ = learned_model_occupancy();
+        if (learned && (occ <= P.small || occ > 64)) {
+            P.newton = false;
+            P.small = 0;
+        }
     }
     if (split || P.newton) {
         C2_TRY(g_pp.term.reserve(P.cap * 3 * sizeof(float)));
@@ -1078,7 +1087,7 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
             k_chunk_flags<<<ceil_div(P.cap, 256), 256, 0, s>>>(
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cellid, A.cell_start,
                 n_sorted, &red->err, (int)P.cap, pp_dense_lg(P.newton),
-                P.small, flags, g_pp.dense.as<int>(),
+                P.small, A.learned_occ, A.learned_range, P.newton, flags, g_pp.dense.as<int>(),
                 &red->ndense, g_pp.pos4.as<float4>(), g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(flags, (int64_t)P.cap, g_pp.scan_tmp, s));
@@ -1121,7 +1130,6 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
             C2_TRY(launch_pp_newton(A, chunks, flags + P.cap, P.grid_pairs, P.small, P.mode, s));
         else
             C2_TRY(launch_pp_tiled(A, chunks, flags + P.cap, P.grid_pairs, P.mode, s));
-        if (P.learned) C2_TRY(learned_enqueue(P.lp, A, g_pp.tile_first.as<int>(), s));
         if (P.newton) {
             Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));
             k_pp_newton_terms<<<4096, 256, 0, s>>>(A.pos4, A.slot, A.react, n_sorted, (int)P.cap,
@@ -1129,6 +1137,8 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                                                     red);
             C2_HIP(hipGetLastError());
         }
+        // (after the pairs-once terms, which are 0 for the network's particles)
+        if (P.learned) C2_TRY(learned_enqueue(P.lp, A, g_pp.tile_first.as<int>(), s));
     }
     if (P.split) return CUBE2_OK;  // pp_enqueue_apply updates vp and copies the results
     if (P.newton) C2_TRY(pp_apply_kernels(P, d_vp, dv64, s));

@@ -155,16 +155,18 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
                     cfull = cnt;
                     if (interior && zz * S + yy <= z * S + y) {
                         // rows before the chunk's: none; its own row: from its
-                        // first i -- unless a small cell lies there, whose j
-                        // act on this chunk's i only from here
+                        // first i -- unless a small cell (in the learned kick
+                        // one of the network's) lies there, whose j act on
+                        // this chunk's i only from here
                         const bool own = zz * S + yy == z * S + y;
                         const int xe = own ? x : xhi + 1;
                         bool has_small = false;
-                        if (small) {
+                        const int marked = range == A.learned_range ? max(small, A.learned_occ - 1) : small;
+                        if (marked > 0) {
                             int c0 = js;
                             for (int xc = xlo; xc < xe; xc++) {
                                 const int c1 = A.cell_start[row + xc + 1];
-                                has_small |= c1 - c0 > 0 && c1 - c0 <= small;
+                                has_small |= c1 - c0 > 0 && c1 - c0 <= marked;
                                 c0 = c1;
                             }
                         }

@@ -132,8 +132,6 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         const int x = (int)(key % S), y = (int)((key / S) % S), z = (int)(key / ((long long)S * S));
         // one subtile per PP cell: same range for the chunk
         const float range = uni(p.w);
-        // learned kick: the network stands in for the sparse level-2 cells
-        if (A.learned_occ && range == A.learned_range && cend - cbeg < A.learned_occ) continue;
         int R;
         float pp2;
         {
