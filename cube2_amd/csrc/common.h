@@ -89,7 +89,7 @@ struct Context {
     hipStream_t stream = nullptr;
     // second library stream: PP's pass beside PM3 in an overlapped kick
     hipStream_t stream2 = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_pairs = nullptr;
     // stream the stage profiler records on (nullptr: stream)
     hipStream_t stage_stream = nullptr;
     // set while one kick's PM3 and PP share a cell-base table computed up front

@@ -153,6 +153,7 @@ int ensure_init() {
         C2_HIP(hipStreamCreateWithFlags(&c.stream2, hipStreamDefault));
         C2_HIP(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
         C2_HIP(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
+        C2_HIP(hipEventCreateWithFlags(&c.ev_pairs, hipEventDisableTiming));
     }
     return CUBE2_OK;
 }

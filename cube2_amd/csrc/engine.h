@@ -35,6 +35,7 @@ struct PPPlan {
     bool learned = false;      // the network stands in for PP in sparse level-2 cells
     bool all_active = false;   // every subtile has a PP range (apm3 > 0 at its level)
     bool newton = false;       // pairs of one range evaluated once (split pass)
+    bool help = false;         // the other stream joins its pair kernel at the end
     float react_scale = 0.0f;  // its fixed-point scale, a power of two
     int small = 0;             // cells of at most this many particles are k_pp_sparse's
     LearnedPlan lp;
@@ -48,7 +49,13 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                float* d_vp, const float* d_scal, const double* dv64, hipStream_t s);
 // After a split pp_enqueue and whatever else writes dv64 (PM3), on stream s:
 // the velocity update and vmax, then the result copies.
-int pp_enqueue_apply(const PPPlan& P, float* d_vp, const double* dv64, hipStream_t s);
+int pp_enqueue_apply(const PPPlan& P, float* d_vp, const float* d_scal, const double* dv64,
+                     hipStream_t s);
+// On the stream that ran beside a split pp_enqueue, after its own work: helps
+// with the pair sums that are left (P.help).
+int pp_enqueue_help(const PPPlan& P, hipStream_t s);
+// Nothing runs beside this pass.
+void pp_alone(PPPlan& P);
 int pp_finish(const PPPlan& P, float* f2max, float* vmax, double* ptotal, double* ttotal,
               uint64_t* pair_counts, double wall_s);
 int pp_force(const int* ires, const int* ixyz3, const float* apm3, const int* ratio_sf,
@@ -63,7 +70,8 @@ int pp_force(const int* ires, const int* ixyz3, const float* apm3, const int* ra
 int vp_runs_move(float* dst, const float* src, const int64_t* runs, int nruns, bool to_compact,
                  hipStream_t s);
 // Blocks of the persistent pair kernel (overlap: beside PM3).
-int pp_tiled_grid(int mode, bool overlap, bool newton = false);
+int pp_tiled_grid(bool overlap);
+int pp_newton_grid(bool overlap);
 // The last PP call's sorted particles and cell lists (for the learned
 // stand-in's training inputs); CUBE2_ERR_STATE if there is none.
 int pp_last(const PPPlan** P, PPArgs* A, const int** tile_first);

@@ -170,9 +170,10 @@ static int enqueue_pm3_pp(const PM3Plan& P3, const PPPlan& P, const int* d_rhoc,
         C2_TRY(pp_enqueue(P, d_rhoc, d_idx, d_xp, d_vp, d_scal, nullptr, s2));
     }
     C2_TRY(pm3_enqueue(P3, d_rhoc, d_idx, d_xp, d_scal, accumulate, dv64, s));
+    C2_TRY(pp_enqueue_help(P, s));
     C2_HIP(hipEventRecord(C.ev_join, s2));
     C2_HIP(hipStreamWaitEvent(s, C.ev_join, 0));
-    return pp_enqueue_apply(P, d_vp, dv64, s);
+    return pp_enqueue_apply(P, d_vp, d_scal, dv64, s);
 }
 
 // The overlapped PM3 + PP of the eager kick driver (prepare, enqueue, wait,
@@ -343,7 +344,7 @@ static int graph_enqueue(const GraphKey& K, const int* d_rhoc, const int64_t* d_
         C2_TRY(pm3_enqueue(g_graph.pm3, d_rhoc, d_idx, d_xp, d_scal, 0, C.dv64.as<double>(), s));
     const double* dv = pm3 ? C.dv64.as<double>() : nullptr;
     C2_TRY(pp_enqueue(g_graph.pp, d_rhoc, d_idx, d_xp, d_vp, d_scal, dv, s));
-    if (g_graph.pp.split) C2_TRY(pp_enqueue_apply(g_graph.pp, d_vp, dv, s));
+    if (g_graph.pp.split) C2_TRY(pp_enqueue_apply(g_graph.pp, d_vp, d_scal, dv, s));
     return CUBE2_OK;
 }
 
@@ -359,8 +360,7 @@ static int graph_record(const GraphKey& K, const int* ixyz3, const float* apm3,
                            g_graph.pm3));
     C2_TRY(pp_prepare(K.ires.data(), ixyz3, apm3, ratio_sf, K.n_used, g_graph.pp,
                       K.overlap || K.learned, K.learned));
-    if (!K.overlap)
-        g_graph.pp.grid_pairs = pp_tiled_grid(g_graph.pp.mode, false, g_graph.pp.newton);
+    if (!K.overlap) pp_alone(g_graph.pp);
     C2_TRY(C.dv64.reserve((size_t)std::max<int64_t>(K.n_used, 1) * 3 * sizeof(double)));
     const float* d_scal = nullptr;
     C2_TRY(scalars_upload(mass, a_mid, dt, s, &d_scal));  // reserves the scalar blocks

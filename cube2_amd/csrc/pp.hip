@@ -36,7 +36,6 @@ namespace cube2 {
 
 int launch_pp_tiled(const PPArgs& a, const int* chunks, const int* nchunks, int grid, int mode,
                     hipStream_t s);
-int pp_tiled_grid(int mode, bool overlap, bool newton);
 
 struct PPState {
     DevBuf nzero, tiles, ires_loc, apm3, counts, scan_tmp, pos4, slot, cellid, red, tile_first;
@@ -47,7 +46,7 @@ struct PPState {
     DevBuf order, order_bin, order_hist;  // chunks heaviest first (k_chunk_cost/order)
     DevBuf term;  // split pass: per slot velocity term [n_used][3] (active slots)
     DevBuf rows_len, rows_base;  // split pass: physical rows' slot counts (scanned) and first slots
-    DevBuf react;  // pairs-once pass: per sorted particle 64-bit fixed-point sums [cap][3]
+    DevBuf react;  // pairs-once pass: per sorted particle 64-bit fixed-point sums [3][cap], then the part counters
     HostBuf h_res;  // PPRed, per-location counts, per-tile pairs, tile_first (pinned)
     std::vector<PPTile> h_tiles;
     std::vector<uint64_t> tile_pairs;  // [ntile][2] of the last call (when counted)
@@ -397,11 +396,19 @@ __global__ void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb, int n
 // subtiles of range occ_range (the network's).  A pairs-once pass (newton)
 // marks both by a negative range (w = -range): to other i they are one-sided
 // sources; every reader of w then takes |w| as the range and w != 0 as active.
+// ntile > 0 (pairs once): flags[a] = the parts the chunk is split into, one
+// per kPartCand candidates j, but at most one per particle, so that the list
+// of all parts fits the capacity.
+// (parts of 4096, 2048, 1024 candidates: 27.8, 28.1, 29.1 ms of pair kernel at
+// 256^3, 4.2, 3.0, 2.9 at 128^3, 5.0, 4.2, 4.1 at 120^3 in level-6 cells; cells
+// of fewer than 16 particles have no chunk worth splitting)
+constexpr int kPartCand = 2048, kPartCount = 16;
 __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
                               const int* __restrict__ cell_start, const int* __restrict__ n_sorted,
                               const int* __restrict__ err, int cap, int dense_lg, int small, int occ,
                               float occ_range, int newton,
+                              const PPTile* __restrict__ tiles, int ntile, int ratio_cs,
                               int* __restrict__ flags, int* __restrict__ dense_list,
                               int* __restrict__ ndense, float4* __restrict__ pos4,
                               uint32_t* __restrict__ slot) {
@@ -423,6 +430,22 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
                 f = 0;
                 if (newton) p.w = -p.w;
             }
+            if (f && ntile && cn >= kPartCount) {
+                const PPTile T = tiles[pp_find_tile(tiles, ntile, c)];
+                const int S = T.S;
+                const unsigned key = c - (unsigned)T.cell_off;
+                const int z = (int)(key / ((unsigned)S * S)), y = (int)(key / S % S), x = (int)(key % S);
+                const int R = (int)ceilf(__fmul_rn(fabsf(p.w), (float)T.rcp) / (float)ratio_cs);
+                const int x0 = max(x - R, 0), x1 = min(x + R, S - 1);
+                long long m = 0;
+                for (int zz = max(z - R, 0); zz <= min(z + R, S - 1); zz++)
+                    for (int yy = max(y - R, 0); yy <= min(y + R, S - 1); yy++) {
+                        const int* row = cell_start + T.cell_off + ((long long)zz * S + yy) * S;
+                        m += row[x1 + 1] - row[x0];
+                    }
+                const int ni = min(dense ? 1 << dense_lg : 64, c0 + cn - a);
+                f = max(1, (int)min(m / kPartCand, (long long)ni));
+            }
         }
         if (!dense) {
             pos4[a] = p;
@@ -435,7 +458,7 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
 __global__ void k_chunk_emit(const int* __restrict__ scanned, int n, int* __restrict__ chunks) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= n) return;
-    if (scanned[a + 1] != scanned[a]) chunks[scanned[a]] = a;
+    for (int k = scanned[a]; k < scanned[a + 1]; k++) chunks[k] = a;
 }
 
 // Chunk order of the pair kernel.  Its wavefronts take chunks by a static
@@ -835,7 +858,9 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
         C2_TRY(g_pp.rows_len.reserve((rows + 1) * sizeof(int)));
         C2_TRY(g_pp.rows_base.reserve(std::max<int64_t>(rows, 1) * sizeof(int64_t)));
     }
-    if (P.newton) C2_TRY(g_pp.react.reserve(P.cap * 3 * sizeof(unsigned long long)));
+    if (P.newton)
+        C2_TRY(g_pp.react.reserve(P.cap * 3 * sizeof(unsigned long long) +
+                                  kPartRuns * kRunPad * sizeof(int)));
     P.all_active = true;
     for (int lv : P.iloc) P.all_active = P.all_active && lv >= 1 && lv <= 7 && apm3[lv - 1] > 0.0f;
     if (learned) {
@@ -851,7 +876,10 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
     C2_HIP(hipMemcpyAsync(g_pp.apm3.ptr, apm3, 7 * sizeof(float), hipMemcpyHostToDevice, s));
     C2_HIP(hipStreamSynchronize(s));  // host tables may go out of scope
     buffers_changed();                 // the device tables now describe this call
-    P.grid_pairs = pp_tiled_grid(P.mode, split, P.newton);
+    // below a million slots the pair kernel is done before PM3 and the joining
+    // launch and its events only cost (3600 particles: 340 us with it, 320)
+    P.help = split && P.newton && n_used >= 1 << 20;
+    P.grid_pairs = P.newton ? pp_newton_grid(P.help) : pp_tiled_grid(split);
     g_pp.valid = false;
     return CUBE2_OK;
 }
@@ -904,12 +932,15 @@ int vp_runs_move(float* dst, const float* src, const int64_t* runs, int nruns, b
 }
 
 // Pairs-once pass: clears the fixed-point sums of the sorted particles.
-__global__ void k_react_zero(unsigned long long* __restrict__ react, const int* __restrict__ n_sorted,
-                             int cap, const int* __restrict__ err) {
-    const int64_t n = (*err & 4) ? 0 : 3 * (int64_t)min(*n_sorted, cap);
+__global__ void k_react_zero(unsigned long long* __restrict__ react, int* __restrict__ taken,
+                             const int* __restrict__ n_sorted, int cap, const int* __restrict__ err) {
+    if (blockIdx.x == 0)
+        for (int k = threadIdx.x; k < kPartRuns * kRunPad; k += blockDim.x) taken[k] = 0;
+    const int n = (*err & 4) ? 0 : min(*n_sorted, cap);
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
          q += (int64_t)gridDim.x * blockDim.x)
-        react[q] = 0;
+#pragma unroll
+        for (int c = 0; c < 3; c++) react[c * (size_t)cap + q] = 0;
 }
 
 // Pairs-once pass, after the pair kernel: each active sorted particle's
@@ -919,17 +950,19 @@ __global__ void k_react_zero(unsigned long long* __restrict__ react, const int* 
 __global__ __launch_bounds__(256) void k_pp_newton_terms(
     const float4* __restrict__ pos4, const uint32_t* __restrict__ slot,
     const unsigned long long* __restrict__ react, const int* __restrict__ n_sorted, int cap,
-    const float* __restrict__ scal, double inv_scale, float* __restrict__ term, PPRed* red) {
+    const float* __restrict__ scal, double inv_scale, float net_range, float* __restrict__ term,
+    PPRed* red) {
 #pragma clang fp contract(off)
     float f2 = 0.0f;
     const int n = red->err == 0 ? min(*n_sorted, cap) : 0;
     const float mass = scal[0], a_mid = scal[1], dt = scal[2];
     for (int a = blockIdx.x * blockDim.x + threadIdx.x; a < n; a += gridDim.x * blockDim.x) {
-        if (pos4[a].w == 0.0f) continue;  // halo sources
+        const float w = pos4[a].w;
+        if (w == 0.0f || w == -net_range) continue;  // halo sources; the network's (learned kick)
         float acc[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const float v = (float)((double)(long long)react[3 * (size_t)a + c] * inv_scale);
+            const float v = (float)((double)(long long)react[c * (size_t)cap + a] * inv_scale);
             acc[c] = v * mass * mass;
         }
         f2 = fmaxf(f2, acc[0] * acc[0] + acc[1] * acc[1] + acc[2] * acc[2]);
@@ -985,6 +1018,52 @@ __global__ __launch_bounds__(256) void k_pp_apply_rows(const int* __restrict__ p
         __syncthreads();  // srow is rewritten for the next segment
     }
     block_max_to<3>(red->vmax_bits, vm);
+}
+
+// What the pair kernels read of a pass.
+static PPArgs pair_args(const PPPlan& P, float* d_vp, const float* d_scal, const double* dv64) {
+    const Geom& g = ctx().g;
+    PPArgs A{};
+    A.pos4 = g_pp.pos4.as<float4>();
+    A.slot = g_pp.slot.as<uint32_t>();
+    A.cellid = g_pp.cellid.as<uint32_t>();
+    A.cell_start = g_pp.counts.as<int>();
+    A.tiles = g_pp.tiles.as<PPTile>();
+    A.ntile = P.ntile;
+    A.n_sorted = g_pp.counts.as<int>() + P.c_tot;
+    A.cap = (int)P.cap;
+    A.ratio_cs = g.p.ratio_cs;
+    A.app = (float)g.p.app;
+    A.scal = d_scal;
+    A.dv64 = P.split ? nullptr : dv64;
+    A.vp = P.split ? nullptr : d_vp;
+    A.term = P.split ? g_pp.term.as<float>() : nullptr;
+    A.red = g_pp.red.as<PPRed>();
+    A.tile_pairs = P.count_tiles ? reinterpret_cast<unsigned long long*>(A.red + 1) + g.ns3 : nullptr;
+    A.learned_occ = P.learned ? P.lp.args.occupancy : 0;
+    A.learned_range = P.learned ? P.lp.args.range : 0.0f;
+    A.ntt = g.ntt;
+    if (P.newton) {
+        A.term = g_pp.term.as<float>();
+        A.react = g_pp.react.as<unsigned long long>();
+        A.react_scale = P.react_scale;
+        A.taken = reinterpret_cast<int*>(A.react + P.cap * 3);
+    }
+    return A;
+}
+
+static const int* pair_chunks() {
+    return pp_heavy_lg() ? g_pp.order.as<int>() : g_pp.chunks.as<int>();
+}
+
+// Velocity terms of a pairs-once pass, once every chunk has added to react.
+static int newton_terms(const PPPlan& P, const PPArgs& A, hipStream_t s) {
+    Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));
+    k_pp_newton_terms<<<4096, 256, 0, s>>>(A.pos4, A.slot, A.react, A.n_sorted, (int)P.cap, A.scal,
+                                            1.0 / (double)P.react_scale, A.learned_range, A.term,
+                                            A.red);
+    C2_HIP(hipGetLastError());
+    return CUBE2_OK;
 }
 
 int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const int16_t* d_xp,
@@ -1053,31 +1132,7 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                                                               g_pp.tile_first.as<int>());
         C2_HIP(hipGetLastError());
     }
-    PPArgs A{};
-    A.pos4 = g_pp.pos4.as<float4>();
-    A.slot = g_pp.slot.as<uint32_t>();
-    A.cellid = g_pp.cellid.as<uint32_t>();
-    A.cell_start = counts;
-    A.tiles = g_pp.tiles.as<PPTile>();
-    A.ntile = P.ntile;
-    A.n_sorted = n_sorted;
-    A.cap = (int)P.cap;
-    A.ratio_cs = g.p.ratio_cs;
-    A.app = (float)g.p.app;
-    A.scal = d_scal;
-    A.dv64 = P.split ? nullptr : dv64;
-    A.vp = P.split ? nullptr : d_vp;
-    A.term = P.split ? g_pp.term.as<float>() : nullptr;
-    A.red = red;
-    A.tile_pairs = P.count_tiles ? ploc + g.ns3 : nullptr;
-    A.learned_occ = P.learned ? P.lp.args.occupancy : 0;
-    A.learned_range = P.learned ? P.lp.args.range : 0.0f;
-    A.ntt = g.ntt;
-    if (P.newton) {
-        A.term = g_pp.term.as<float>();
-        A.react = g_pp.react.as<unsigned long long>();
-        A.react_scale = P.react_scale;
-    }
+    const PPArgs A = pair_args(P, d_vp, d_scal, dv64);
     if (P.mode == CUBE2_PP_EXACT) {
         C2_TRY(launch_pp_pairs(A, P.mode, s));
     } else {
@@ -1087,7 +1142,8 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
             k_chunk_flags<<<ceil_div(P.cap, 256), 256, 0, s>>>(
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cellid, A.cell_start,
                 n_sorted, &red->err, (int)P.cap, pp_dense_lg(P.newton),
-                P.small, A.learned_occ, A.learned_range, P.newton, flags, g_pp.dense.as<int>(),
+                P.small, A.learned_occ, A.learned_range, P.newton, A.tiles,
+                P.newton && !pp_heavy_lg() ? P.ntile : 0, g.p.ratio_cs, flags, g_pp.dense.as<int>(),
                 &red->ndense, g_pp.pos4.as<float4>(), g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(flags, (int64_t)P.cap, g_pp.scan_tmp, s));
@@ -1097,47 +1153,40 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
         {
             Stage st("pp_subsort", (double)P.n_used * 24);
             // one wavefront per chunk (only first chunks of dense cells work)
-            k_pp_subsort<<<(unsigned)std::max(1, P.grid_pairs), 256, 0, s>>>(
+            k_pp_subsort<<<(unsigned)std::max(1, pp_tiled_grid(false)), 256, 0, s>>>(
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cell_start, A.tiles,
                 P.ntile, g_pp.dense.as<int>(), &red->ndense, g.p.ratio_cs, g_pp.pos4.as<float4>(),
                 g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
         }
-        const int* chunks = g_pp.chunks.as<int>();
+        const int* chunks = pair_chunks();
         if (pp_heavy_lg()) {
             Stage st("pp_order", (double)P.cap * 9);
             int* hist = g_pp.order_hist.as<int>();
-            k_chunk_cost<<<kOrderBlocks, kOrderBins, 0, s>>>(A, chunks, flags + P.cap,
+            k_chunk_cost<<<kOrderBlocks, kOrderBins, 0, s>>>(A, g_pp.chunks.as<int>(), flags + P.cap,
                                                              pp_dense_lg(P.newton),
                                                              pp_heavy_lg(),
                                                              g_pp.order_bin.as<unsigned char>(), hist);
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(hist, (int64_t)kOrderBins * kOrderBlocks, g_pp.scan_tmp, s));
-            k_chunk_order<<<kOrderBlocks, kOrderBins, 0, s>>>(chunks, g_pp.order_bin.as<unsigned char>(),
+            k_chunk_order<<<kOrderBlocks, kOrderBins, 0, s>>>(g_pp.chunks.as<int>(), g_pp.order_bin.as<unsigned char>(),
                                                               flags + P.cap, hist, g_pp.order.as<int>());
             C2_HIP(hipGetLastError());
-            chunks = g_pp.order.as<int>();
         }
         if (P.newton) {
             Stage st("pp_react_zero", (double)P.n_used * 24);
-            k_react_zero<<<2048, 256, 0, s>>>(A.react, n_sorted, (int)P.cap, &red->err);
+            k_react_zero<<<2048, 256, 0, s>>>(A.react, A.taken, n_sorted, (int)P.cap, &red->err);
             C2_HIP(hipGetLastError());
         }
         if (P.small)
             C2_TRY(launch_pp_sparse(A, d_rhoc, g.nt, g.ncb, (int)((int64_t)P.ntile * g.nt * g.nt * g.nt),
                                     P.small, P.mode, s));
+        if (P.help) C2_HIP(hipEventRecord(ctx().ev_pairs, s));
         if (P.newton)
-            C2_TRY(launch_pp_newton(A, chunks, flags + P.cap, P.grid_pairs, P.small, P.mode, s));
+            C2_TRY(launch_pp_newton(A, chunks, flags, P.grid_pairs, P.small, P.mode, s));
         else
             C2_TRY(launch_pp_tiled(A, chunks, flags + P.cap, P.grid_pairs, P.mode, s));
-        if (P.newton) {
-            Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));
-            k_pp_newton_terms<<<4096, 256, 0, s>>>(A.pos4, A.slot, A.react, n_sorted, (int)P.cap,
-                                                    d_scal, 1.0 / (double)P.react_scale, A.term,
-                                                    red);
-            C2_HIP(hipGetLastError());
-        }
-        // (after the pairs-once terms, which are 0 for the network's particles)
+        if (P.newton && !P.help) C2_TRY(newton_terms(P, A, s));
         if (P.learned) C2_TRY(learned_enqueue(P.lp, A, g_pp.tile_first.as<int>(), s));
     }
     if (P.split) return CUBE2_OK;  // pp_enqueue_apply updates vp and copies the results
@@ -1202,11 +1251,26 @@ static int pp_apply_kernels(const PPPlan& P, float* d_vp, const double* dv64, hi
     return CUBE2_OK;
 }
 
-int pp_enqueue_apply(const PPPlan& P, float* d_vp, const double* dv64, hipStream_t s) {
+int pp_enqueue_help(const PPPlan& P, hipStream_t s) {
+    if (!P.help) return CUBE2_OK;
+    C2_HIP(hipStreamWaitEvent(s, ctx().ev_pairs, 0));
+    return launch_pp_newton(pair_args(P, nullptr, nullptr, nullptr), pair_chunks(),
+                            g_pp.chunk_flags.as<int>(), pp_newton_grid(false), P.small,
+                            P.mode, s);
+}
+
+void pp_alone(PPPlan& P) {
+    P.help = false;
+    P.grid_pairs = P.newton ? pp_newton_grid(false) : pp_tiled_grid(false);
+}
+
+int pp_enqueue_apply(const PPPlan& P, float* d_vp, const float* d_scal, const double* dv64,
+                     hipStream_t s) {
     if (!P.split) {
         set_error("velocity apply of an unsplit PP pass");
         return CUBE2_ERR_STATE;
     }
+    if (P.help) C2_TRY(newton_terms(P, pair_args(P, nullptr, d_scal, nullptr), s));
     C2_TRY(pp_apply_kernels(P, d_vp, dv64, s));
     return pp_results_to_host(P, s);
 }
@@ -1328,7 +1392,7 @@ int pp_force(const int* ires, const int* ixyz3, const float* apm3, const int* ra
     if (fill_vp && !late) C2_TRY(fill_vp(C.stream));
     PPPlan P;
     C2_TRY(pp_prepare(ires, ixyz3, apm3, ratio_sf, n_used, P, learned || late, learned));
-    P.grid_pairs = pp_tiled_grid(P.mode, false, P.newton);  // nothing runs beside it here
+    pp_alone(P);  // nothing runs beside it here
     const double* dv = (C.dv_state == 1) ? C.dv64.as<double>() : nullptr;
     const float* d_scal = nullptr;
     C2_TRY(scalars_upload(mass, a_mid, dt, C.stream, &d_scal));
@@ -1340,7 +1404,7 @@ int pp_force(const int* ires, const int* ixyz3, const float* apm3, const int* ra
         C2_HIP(hipEventRecord(filled, C.stream2));
         C2_HIP(hipStreamWaitEvent(C.stream, filled, 0));
     }
-    if (P.split) C2_TRY(pp_enqueue_apply(P, d_vp, dv, C.stream));
+    if (P.split) C2_TRY(pp_enqueue_apply(P, d_vp, d_scal, dv, C.stream));
     C2_TRY(sync_and_flush());
     C.dv_state = 0;
     const double wall = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

@@ -10,6 +10,10 @@ struct PPTile {
     long long cell_off;  // first cell of the tile in the concatenated grids
 };
 
+// The pairs-once pair kernel's list in runs, each with a counter of its own
+// (on a cache line of its own) from which wavefronts take the next part.
+constexpr int kPartRuns = 64, kRunPad = 32;
+
 struct PPRed {
     unsigned long long p_cand, p_acc;  // examined / accepted ordered pairs
     unsigned f2max_bits;               // max |a|^2 (non-negative float bits)
@@ -71,17 +75,31 @@ struct PPArgs {
     // pairs-once pass (non-null): each pair of two active particles of one
     // range is evaluated once and its force added to both, the per-particle
     // sums kept as signed 64-bit fixed point (value * react_scale) at
-    // react[3 * sorted index]; k_pp_newton_terms turns them into term
+    // react[c * cap + sorted index]; k_pp_newton_terms turns them into term
     unsigned long long* react;
+    int* taken;  // per run of the part list (kPartRuns, kRunPad apart): parts taken
     float react_scale;
     int ntt;  // coarse cells per subtile side
 };
 
 int launch_pp_pairs(const PPArgs& a, int mode, hipStream_t s);
 
-// Pairs-once pair kernel (pp_newton.hip) over the chunks; cells of at most
-// `small` particles are k_pp_sparse's (0: none).
-int launch_pp_newton(const PPArgs& a, const int* chunks, const int* nchunks, int grid, int small,
+// Tile of a PP cell.
+__device__ inline int pp_find_tile(const PPTile* __restrict__ T, int ntile, uint32_t c) {
+    int lo = 0, hi = ntile - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (T[mid].cell_off <= (long long)c) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// Pairs-once pair kernel (pp_newton.hip) over the parts of the chunks:
+// chunks[k] is the chunk of part k, first[a] the first part of chunk a, in the
+// order of the list or (a list ordered otherwise) one each; first[cap] is their
+// number.  Cells of at most `small` particles are k_pp_sparse's (0: none).
+int launch_pp_newton(const PPArgs& a, const int* chunks, const int* first, int grid, int small,
                      int mode, hipStream_t s);
 
 // The small cells' particles of a pairs-once pass (pp_sparse.hip): nt coarse

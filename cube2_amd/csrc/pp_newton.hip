@@ -10,11 +10,19 @@
 // (integer adds commute: the result does not depend on the order of the
 // atomics).
 //
-// Wavefronts take chunks of physical particles of one PP cell by a static
-// stride (a grid of 64 blocks per CU, far more than are resident, so that the
-// hardware balances the chunks' uneven costs): the whole cell if it holds
+// A chunk is physical particles of one PP cell: the whole cell if it holds
 // fewer than 64, else 2^dense_lg at a time (32 built in) in the Morton sub-cell
-// order of k_pp_subsort, so that a chunk is spatially compact.  The j of the
+// order of k_pp_subsort, so that a chunk is spatially compact.  A chunk of many
+// candidates is split into parts of about 2048 of them (k_chunk_flags), any
+// wavefront taking any part: whole chunks took 0.3 ms on average but up to 29
+// ms in a clump, and the kernel waited for the last of them (the chunks' times
+// at 256^3 summed to 19.5 ms of all wavefronts' time, the kernel took 32; at
+// 128^3 1.9 and 3.9).  Wavefronts take parts from counters, one for each of
+// kPartRuns runs of the list (one counter for all serialised them, 15 ns a
+// part: a 64^3 lattice 0.50 ms, with runs 0.15), so that a second launch on
+// another stream can join at any time: beside PM3 the kernel runs at half its
+// occupancy, which leaves registers for the mesh kernels, and PM3's stream
+// helps once it is done.  The j of the
 // (2R+1)^2 neighbour rows are contiguous runs of the sorted particles; a
 // wavefront concatenates them into one candidate list, fetches it 64 at a
 // time (one coalesced load, a batch ahead) and keeps the j within the range
@@ -28,10 +36,14 @@
 // one such block and in FP64 over the blocks.
 //
 // Bound by VALU issue (about 95 instructions per step) and, in clumps, the
-// reactions' atomics.  REF at 256^3 (16.7 M particles, clustered): 32.4 ms of
-// the kick's 88.6, beside 7.9 ms for the small cells (57.8 ms in one kernel
-// with a chunk for every cell, the kick 104.2; 60.9 and 109.7 with each j's
-// reaction summed over the lanes at each step).
+// reactions' atomics: they are laid out by component, so that the 64 lanes'
+// atomics of one instruction fall into a few cache lines (by particle, three
+// times as many: 64^3 lattice 0.154 -> 0.115 ms).  REF at 256^3 (16.7 M
+// particles, clustered): 28 ms of the kick's 85, beside 7.9 ms for the small
+// cells (57.8 ms in one kernel with a chunk for every cell, the kick 104.2;
+// 60.9 and 109.7 with each j's reaction summed over the lanes at each step);
+// at 128^3 3.0 ms, 512 uneven tiles 5.3, 120^3 in level-6 cells 4.2 (whole
+// chunks by a static stride 3.9, 5.4, 8.2).
 #include <algorithm>
 #include <climits>
 
@@ -41,6 +53,8 @@
 #include "reduce.h"
 
 namespace cube2 {
+
+static_assert(kPartRuns == 64, "one lane per run");
 
 constexpr int kJBlock = 96;  // a block of 64 j and its first 32 again
 
@@ -56,31 +70,44 @@ __device__ inline float wave_rol1(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x134, 0xf, 0xf, true));
 }
 
-__device__ inline int find_tile2(const PPTile* __restrict__ T, int ntile, uint32_t c) {
-    int lo = 0, hi = ntile - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (T[mid].cell_off <= (long long)c) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
+// First of the candidates [0, m) that part p of np takes.
+__device__ inline int part_of(int m, int p, int np) { return (int)((long long)m * p / np); }
 
 template <int kMode, int kJB>
 __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __restrict__ chunks,
-                                                      const int* __restrict__ nchunks_dev,
-                                                      int small, int dense_lg) {
+                                                      const int* __restrict__ first, int small,
+                                                      int dense_lg) {
     static_assert(kJB == 64 || kJB == 128, "j batch of 64 or 128");
     constexpr int kH = kJB / 64;  // fetched float4 per lane per batch
     __shared__ NewtonLDS lds[4];
     const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     NewtonLDS& L = lds[wave];
-    const int nchunks = uni(*nchunks_dev);
+    const int nparts = uni(first[A.cap]);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     const FraK Ka = uni(make_frak(A.app));
     unsigned long long pc = 0, pa = 0;  // (wavefront-uniform)
-    for (int ck = blockIdx.x * 4 + wave; ck < nchunks; ck += gridDim.x * 4) {
+    // run r of the list: parts [r len, (r + 1) len)
+    const int len = (nparts + kPartRuns - 1) / kPartRuns;
+    int run = (int)(blockIdx.x % kPartRuns);
+    auto take = [&]() { return lane == 0 ? atomicAdd(&A.taken[run * kRunPad], 1) : 0; };
+    int got = uni(take());
+    for (;;) {
+        if (got >= len || run * len + got >= nparts) {  // run done: the next one that is not
+            const int have = __hip_atomic_load(&A.taken[lane * kRunPad], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint64_t open = __ballot(have < len && lane * len + have < nparts);
+            if (!open) break;
+            const uint64_t after = run == 63 ? 0ull : open & (~0ull << (run + 1));
+            run = __ffsll((unsigned long long)(after ? after : open)) - 1;
+            got = uni(take());
+            continue;
+        }
+        const int ck = run * len + got;
+        const int nxt = take();  // (in flight during the part)
         const int a0 = uni(chunks[ck]);
+        // its part and the number of parts of the chunk (one if the list is in
+        // another order)
+        const int f0 = uni(first[a0]), np = max(uni(first[a0 + 1]) - f0, 1);
+        const int part = np > 1 ? ck - f0 : 0;
         const uint32_t cid = (uint32_t)uni((int)A.cellid[a0]);
         const int cend = uni(A.cell_start[cid + 1]), cbeg = uni(A.cell_start[cid]);
         const bool grouped = cend - cbeg >= 64;
@@ -92,7 +119,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
         const bool vi = islot < ni;
         const int ia = a0 + (vi ? islot : 0);
         const float4 p = A.pos4[ia];
-        const int ti = uni(find_tile2(A.tiles, A.ntile, cid));
+        const int ti = uni(pp_find_tile(A.tiles, A.ntile, cid));
         const PPTile T = A.tiles[ti];
         const unsigned long long pc0 = pc, pa0 = pa;
         const int S = T.S;
@@ -182,14 +209,16 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
             int sf = cfull;
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) sf += __shfl_xor(sf, o, 64);
-            ncand += (unsigned)uni(sf);
+            if (part == 0) ncand += (unsigned)uni(sf);
             int inc = cnt;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
                 const int t = __shfl_up(inc, o, 64);
                 if (lane >= o) inc += t;
             }
-            const int M = uni(__shfl(inc, 63, 64));
+            const int M0 = uni(__shfl(inc, 63, 64));
+            // the part's candidates [v0, M) of the group's
+            const int v0 = part_of(M0, part, np), M = part_of(M0, part + 1, np);
             L.rs[lane] = js - (inc - cnt);
             L.rp[lane] = inc;
             wave_lds_sync();
@@ -197,7 +226,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
             // first with rp > v) is found by walking forward from the last
             // one: rp of the rows past the group is M > v, so the walk stops
             // inside the group
-            int frow = 0;
+            int frow = 0;  // (rp of the last row is the group's M0 >= M)
             auto fetch = [&](int vb, int& jx) {
                 const int v = vb + lane;
                 float4 q4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -211,11 +240,11 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
             float4 qcur[kH];
             int jcur[kH] = {};
 #pragma unroll
-            for (int h = 0; h < kH; h++) qcur[h] = fetch(64 * h, jcur[h]);
+            for (int h = 0; h < kH; h++) qcur[h] = fetch(v0 + 64 * h, jcur[h]);
             // (a last step without candidates takes the j left over)
             const bool last = rg + 64 >= nrows;
-            const int vend = last ? (M + kJB - 1) / kJB * kJB + kJB : M;
-            for (int vb = 0; vb < vend; vb += kJB) {
+            const int vend = last ? v0 + (M - v0 + kJB - 1) / kJB * kJB + kJB : M;
+            for (int vb = v0; vb < vend; vb += kJB) {
 #pragma unroll
                 for (int h = 0; h < kH; h++) {
                     float4 qh = qcur[h];
@@ -284,10 +313,10 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
                     // lane l now holds the reaction of j (l + I - 1) mod 64
                     const int jw = __float_as_int(L.jb[bb + ((lane + I - 1) & 63)].w);
                     if (jw != INT_MAX) {
-                        unsigned long long* d = A.react + 3 * (size_t)jw;
+                        unsigned long long* d = A.react + jw;
                         fixed_add(d, -rx, A.react_scale);
-                        fixed_add(d + 1, -ry, A.react_scale);
-                        fixed_add(d + 2, -rz, A.react_scale);
+                        fixed_add(d + A.cap, -ry, A.react_scale);
+                        fixed_add(d + 2 * (size_t)A.cap, -rz, A.react_scale);
                     }
                     jhead += 64;
                     wave_lds_sync();
@@ -302,34 +331,36 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
             for (int c = 0; c < 3; c++) {
                 double v = 0.0;
                 for (int q = lane; q < 64; q += I) v += L.acc[c][q];
-                fixed_add(A.react + 3 * (size_t)ia + c, v, A.react_scale);
+                fixed_add(A.react + c * (size_t)A.cap + ia, v, A.react_scale);
             }
         }
-        pc += (unsigned long long)(ncand - 1u) * (unsigned)ni;  // (not the particle itself)
+        // (each i once for the chunk, and not with itself)
+        if (part == 0) pc += (unsigned long long)(ncand - 1u) * (unsigned)ni;
         pa += npa;
         if (A.tile_pairs && lane == 0) {  // per-tile counts (on request only)
             atomicAdd(&A.tile_pairs[2 * ti], pc - pc0);
             atomicAdd(&A.tile_pairs[2 * ti + 1], pa - pa0);
         }
         wave_lds_sync();  // acc and the blocks are reused by the next chunk
+        got = uni(nxt);
     }
     const unsigned long long sm[2] = {lane == 0 ? pc : 0ull, lane == 0 ? pa : 0ull};
     block_sum_to<2>(&A.red->p_cand, sm);
 }
 
-int launch_pp_newton(const PPArgs& a, const int* chunks, const int* nchunks, int grid, int small,
+int launch_pp_newton(const PPArgs& a, const int* chunks, const int* first, int grid, int small,
                      int mode, hipStream_t s) {
     Stage st(mode == CUBE2_PP_REF ? "pp_pairs_ref" : "pp_pairs_fastq");
     const unsigned blocks = (unsigned)std::max(1, grid);
     const int dl = pp_dense_lg(true);
     if (mode == CUBE2_PP_REF && pp_jbatch() == 128)
-        k_pp_newton<kModeRef, 128><<<blocks, 256, 0, s>>>(a, chunks, nchunks, small, dl);
+        k_pp_newton<kModeRef, 128><<<blocks, 256, 0, s>>>(a, chunks, first, small, dl);
     else if (mode == CUBE2_PP_REF)
-        k_pp_newton<kModeRef, 64><<<blocks, 256, 0, s>>>(a, chunks, nchunks, small, dl);
+        k_pp_newton<kModeRef, 64><<<blocks, 256, 0, s>>>(a, chunks, first, small, dl);
     else if (pp_jbatch() == 128)
-        k_pp_newton<kModeFast, 128><<<blocks, 256, 0, s>>>(a, chunks, nchunks, small, dl);
+        k_pp_newton<kModeFast, 128><<<blocks, 256, 0, s>>>(a, chunks, first, small, dl);
     else
-        k_pp_newton<kModeFast, 64><<<blocks, 256, 0, s>>>(a, chunks, nchunks, small, dl);
+        k_pp_newton<kModeFast, 64><<<blocks, 256, 0, s>>>(a, chunks, first, small, dl);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }

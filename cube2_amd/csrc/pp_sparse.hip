@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __res
             pc -= (unsigned)ni;  // the particles themselves
             if (vi && jslot == 0)
 #pragma unroll
-                for (int c = 0; c < 3; c++) A.react[3 * (size_t)ia + c] = L.acc[islot][c];
+                for (int c = 0; c < 3; c++) A.react[c * (size_t)A.cap + ia] = L.acc[islot][c];
             wave_lds_sync();  // acc, the queue and the list are reused
         }
         if (A.tile_pairs && lane == 0) {  // per-tile counts (on request only)

@@ -359,25 +359,32 @@ bool pp_newton_mode(int mode) { return mode == CUBE2_PP_REF || mode == CUBE2_PP_
 // Blocks of the pair kernel: 64 per CU, ten times the resident maximum (6),
 // unless tuned.  Its wavefronts take chunks by a static stride over the
 // list; with a grid far beyond what is resident, the hardware hands out
-// blocks as others retire, which evens out the uneven chunk costs (at 256^3
-// pairs once, alone: 67.3 ms at 6 blocks per CU, 63.3 at 24, 56.1 at 64,
-// 57.4 at 128) and lets the PM3 mesh kernels on the other stream take the
-// slots of retiring blocks throughout (overlapped kick: 111.5 ms at 6, 105.3
-// at 24, 103.3 at 64).  overlap: the kernel runs beside PM3
-// (CUBE2_TUNE_PP_OVERLAP_BLOCKS per CU if set).
-int pp_tiled_grid(int mode, bool overlap, bool newton) {
-    (void)mode;
-    (void)newton;
-    constexpr int kBlocksPerCU = 64;
+// blocks as others retire, which evens out the uneven chunk costs.  overlap:
+// the kernel runs beside PM3 (CUBE2_TUNE_PP_OVERLAP_BLOCKS per CU if set).
+static int per_cu(int blocks) {
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         ncu = 256;
-    ncu = std::max(1, ncu);
+    return std::max(1, ncu) * blocks;
+}
+
+int pp_tiled_grid(bool overlap) {
     const int forced = ctx().tune[CUBE2_TUNE_PP_BLOCKS_PER_CU];
     const int over = ctx().tune[CUBE2_TUNE_PP_OVERLAP_BLOCKS];
-    if (overlap && over) return ncu * over;
-    return ncu * (forced ? forced : kBlocksPerCU);
+    if (overlap && over) return per_cu(over);
+    return per_cu(forced ? forced : 64);
+}
+
+// Blocks of the pairs-once pair kernel, whose wavefronts take parts from
+// counters: all that are resident, or half of them beside PM3, whose stream
+// launches the rest at its end (256^3 kick, blocks per CU 2, 3, 4, 6: 86.0,
+// 85.4, 86.6, 88.4 ms).
+int pp_newton_grid(bool overlap) {
+    const int forced = ctx().tune[CUBE2_TUNE_PP_BLOCKS_PER_CU];
+    const int over = ctx().tune[CUBE2_TUNE_PP_OVERLAP_BLOCKS];
+    if (overlap) return per_cu(over ? over : 3);
+    return per_cu(forced ? forced : 6);
 }
 
 template <int kJB>

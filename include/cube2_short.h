@@ -120,7 +120,8 @@ int cube2_set_pp_mode(int mode);
  * choice.  Valid values:
  *   PP_BLOCKS_PER_CU  1..256, blocks per CU of the pair kernel (built-in:
  *                     64, beyond the resident maximum, so that the hardware
- *                     balances the chunks' uneven costs);
+ *                     balances the chunks' uneven costs; 6, the resident
+ *                     maximum, when PP_NEWTON evaluates pairs once);
  *   PP_DIRECT_LG      1..7, chunks of > 2^(v-1) particles (lanes for >= 2^v
  *                     i slots) sum directly, smaller ones queue pairs (2);
  *                     where PP_NEWTON evaluates pairs once, cells of at most
@@ -136,14 +137,16 @@ int cube2_set_pp_mode(int mode);
  *                     on a second stream beside PM3, the velocity update
  *                     after both (built-in); 2: PM3, then PP;
  *   PP_OVERLAP_BLOCKS 1..256, blocks per CU of the pair kernel while PM3
- *                     runs beside it (built-in: as PP_BLOCKS_PER_CU);
+ *                     runs beside it (built-in: as PP_BLOCKS_PER_CU; 3
+ *                     when PP_NEWTON evaluates pairs once, PM3's stream
+ *                     joining in when PM3 is done);
  *   PP_ORDER          1: the pair kernel takes its chunks in cell order
  *                     (built-in); 2..30: chunks of an estimated 2^v
  *                     candidate pairs or more first, heaviest first, then
  *                     the rest in cell order;
  *   PP_JBATCH         1: the pair kernel fetches and tests j candidates 64
  *                     at a time (built-in); 2: 128 at a time;
- *   PP_NEWTON         1: REF and FAST passes (not the learned kick)
+ *   PP_NEWTON         1: REF and FAST passes
  *                     evaluate each pair of two active particles of one
  *                     range once and add its force to both, summing in
  *                     64-bit fixed point at 2^k, k = min(40, floor(62 -
