@@ -1,7 +1,8 @@
 // Kernels of the learned PP stand-in: a 3-D CNN of 3^3 valid convolutions
 // in channels-last layout (activation [patch][z][y][x][channel], FP32),
-// each layer an im2col (BF16) and a BF16 GEMM on the matrix cores with FP32
-// accumulation; backward by the same GEMM on transposed operands.
+// convolved on the matrix cores (k_conv3); for grids larger than training
+// patches (those: cnn_bwd.hip) the backward is im2col (BF16) and a BF16 GEMM
+// with FP32 accumulation on transposed operands.
 //
 // GEMM: C[m][n] (+)= sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak],
 // B(k,n) = B[k*sbk + n*sbn], C row-major with leading dimension ldc.  One

@@ -47,6 +47,7 @@ struct PPState {
     DevBuf term;  // split pass: per slot velocity term [n_used][3] (active slots)
     DevBuf rows_len, rows_base;  // split pass: physical rows' slot counts (scanned) and first slots
     DevBuf react;  // pairs-once pass: per sorted particle 64-bit fixed-point sums [3][cap], then the part counters
+    DevBuf items;  // k_pp_sparse's work items
     HostBuf h_res;  // PPRed, per-location counts, per-tile pairs, tile_first (pinned)
     std::vector<PPTile> h_tiles;
     std::vector<uint64_t> tile_pairs;  // [ntile][2] of the last call (when counted)
@@ -369,19 +370,23 @@ __global__ __launch_bounds__(64 * kBigWaves) void k_pp_scatter_big(
 }
 
 // Physical particles per subtile location (pp_force_kernel.cu:691-705).
-__global__ void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb, int nte, int nnt,
-                            int nns, int ntt, unsigned long long* __restrict__ ploc) {
-    const int64_t per = (int64_t)nt * nt * nt;
-    int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= per * nnt * nnt * nnt) return;
-    const int t = (int)(w / per);
-    int64_t r = w - (int64_t)t * per;
-    const int i = (int)(r % nt), j = (int)((r / nt) % nt), k = (int)(r / ((int64_t)nt * nt));
-    const int v = rhoc[(((int64_t)t * nte + k + ncb) * nte + j + ncb) * nte + i + ncb];
-    if (!v) return;
-    const int tx = t % nnt, ty = (t / nnt) % nnt, tz = t / (nnt * nnt);
-    const int loc = (((tz * nnt + ty) * nnt + tx) * nns + k / ntt) * nns * nns + (j / ntt) * nns + i / ntt;
-    atomicAdd(&ploc[loc], (unsigned long long)v);
+// One block per subtile and up to kPtotalCells of its coarse cells: one atomic
+// per block (one per cell, all cells of a subtile adding to one word: 52 us for
+// 64 subtiles of 8^3 cells).
+constexpr int kPtotalCells = 4096;
+__global__ __launch_bounds__(256) void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb,
+                                                   int nte, int nns, int ntt,
+                                                   unsigned long long* __restrict__ ploc) {
+    const int q = (int)(blockIdx.x % (unsigned)(nns * nns * nns)), t = (int)(blockIdx.x / (unsigned)(nns * nns * nns));
+    const int sx = q % nns * ntt, sy = q / nns % nns * ntt, sz = q / (nns * nns) * ntt;
+    const int per = ntt * ntt * ntt, c1 = min(per, ((int)blockIdx.y + 1) * kPtotalCells);
+    unsigned long long v = 0;
+    for (int c = blockIdx.y * kPtotalCells + threadIdx.x; c < c1; c += blockDim.x) {
+        const int i = sx + c % ntt, j = sy + c / ntt % ntt, k = sz + c / (ntt * ntt);
+        v += (unsigned long long)(long long)rhoc[(((int64_t)t * nte + k + ncb) * nte + j + ncb) * nte + i + ncb];
+    }
+    const unsigned long long sm[1] = {v};
+    block_sum_to<1>(&ploc[blockIdx.x], sm);
 }
 
 // Work chunks of the pair kernel: <= 64 consecutive physical particles of
@@ -397,18 +402,21 @@ __global__ void k_pp_ptotal(const int* __restrict__ rhoc, int nt, int ncb, int n
 // marks both by a negative range (w = -range): to other i they are one-sided
 // sources; every reader of w then takes |w| as the range and w != 0 as active.
 // ntile > 0 (pairs once): flags[a] = the parts the chunk is split into, one
-// per kPartCand candidates j, but at most one per particle, so that the list
+// per `part` candidates j, but at most one per particle, so that the list
 // of all parts fits the capacity.
 // (parts of 4096, 2048, 1024 candidates: 27.8, 28.1, 29.1 ms of pair kernel at
 // 256^3, 4.2, 3.0, 2.9 at 128^3, 5.0, 4.2, 4.1 at 120^3 in level-6 cells; cells
 // of fewer than 16 particles have no chunk worth splitting)
-constexpr int kPartCand = 2048, kPartCount = 16;
+// Below kFewSlots slots there are few chunks for all the wavefronts, and a part
+// is a serial chain of its candidates (pair kernel with 2048, 256, 64 of them:
+// 3600 particles 95, 96, 57 us, 64^3 lattice 115, 114, 117).
+constexpr int kPartCand = 2048, kPartFew = 64, kPartCount = 16, kFewSlots = 1 << 20;
 __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
                               const int* __restrict__ cell_start, const int* __restrict__ n_sorted,
                               const int* __restrict__ err, int cap, int dense_lg, int small, int occ,
                               float occ_range, int newton,
-                              const PPTile* __restrict__ tiles, int ntile, int ratio_cs,
+                              const PPTile* __restrict__ tiles, int ntile, int ratio_cs, int part,
                               int* __restrict__ flags, int* __restrict__ dense_list,
                               int* __restrict__ ndense, float4* __restrict__ pos4,
                               uint32_t* __restrict__ slot) {
@@ -444,7 +452,7 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
                         m += row[x1 + 1] - row[x0];
                     }
                 const int ni = min(dense ? 1 << dense_lg : 64, c0 + cn - a);
-                f = max(1, (int)min(m / kPartCand, (long long)ni));
+                f = max(1, (int)min(m / part, (long long)ni));
             }
         }
         if (!dense) {
@@ -529,7 +537,8 @@ __global__ __launch_bounds__(kOrderBins) void k_chunk_cost(PPArgs A, const int* 
 // Stable scatter of the chunks by bin: within a block's segment, 256 chunks
 // at a time in order; a chunk's place is its bin's base, the chunks of its bin
 // in the earlier wavefronts of the step, and its rank among its wavefront's
-// lanes of the same bin (found with 8 ballots on the bin's bits).
+// lanes of the same bin (found with 8 ballots on the bin's bits).  out holds
+// the chunks or (chunks null) their places in the list.
 __global__ __launch_bounds__(kOrderBins) void k_chunk_order(const int* __restrict__ chunks,
                                                          const unsigned char* __restrict__ bin,
                                                          const int* __restrict__ nchunks_dev,
@@ -560,7 +569,7 @@ __global__ __launch_bounds__(kOrderBins) void k_chunk_order(const int* __restric
         if (valid) {
             int pos = base[b] + rank;
             for (int w = 0; w < wave; w++) pos += wc[w][b];
-            out[pos] = chunks[ck];
+            out[pos] = chunks ? chunks[ck] : ck;
         }
         __syncthreads();
         base[t] += wc[0][t] + wc[1][t] + wc[2][t] + wc[3][t];
@@ -860,7 +869,9 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
     }
     if (P.newton)
         C2_TRY(g_pp.react.reserve(P.cap * 3 * sizeof(unsigned long long) +
-                                  kPartRuns * kRunPad * sizeof(int)));
+                                  kTakenInts * sizeof(int)));
+    const int64_t ncoarse = (int64_t)g.ntile * g.nt * g.nt * g.nt;
+    if (P.small) C2_TRY(g_pp.items.reserve(pp_sparse_items(ncoarse, n_used) * sizeof(int2)));
     P.all_active = true;
     for (int lv : P.iloc) P.all_active = P.all_active && lv >= 1 && lv <= 7 && apm3[lv - 1] > 0.0f;
     if (learned) {
@@ -878,7 +889,7 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
     buffers_changed();                 // the device tables now describe this call
     // below a million slots the pair kernel is done before PM3 and the joining
     // launch and its events only cost (3600 particles: 340 us with it, 320)
-    P.help = split && P.newton && n_used >= 1 << 20;
+    P.help = split && P.newton && n_used >= kFewSlots;
     P.grid_pairs = P.newton ? pp_newton_grid(P.help) : pp_tiled_grid(split);
     g_pp.valid = false;
     return CUBE2_OK;
@@ -935,7 +946,7 @@ int vp_runs_move(float* dst, const float* src, const int64_t* runs, int nruns, b
 __global__ void k_react_zero(unsigned long long* __restrict__ react, int* __restrict__ taken,
                              const int* __restrict__ n_sorted, int cap, const int* __restrict__ err) {
     if (blockIdx.x == 0)
-        for (int k = threadIdx.x; k < kPartRuns * kRunPad; k += blockDim.x) taken[k] = 0;
+        for (int k = threadIdx.x; k < kTakenInts; k += blockDim.x) taken[k] = 0;
     const int n = (*err & 4) ? 0 : min(*n_sorted, cap);
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n;
          q += (int64_t)gridDim.x * blockDim.x)
@@ -991,14 +1002,16 @@ __global__ __launch_bounds__(256) void k_pp_apply_rows(const int* __restrict__ p
     float vm[3] = {0.f, 0.f, 0.f};
     const int total = red->err == 0 ? prefix[nrows] : 0;  // a failed call leaves no terms
     for (int seg0 = blockIdx.x * kApplySeg; seg0 < total; seg0 += gridDim.x * kApplySeg) {
-        if (threadIdx.x == 0) {  // last row starting at or before seg0
-            int lo = 0, hi = nrows - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (prefix[mid] <= seg0) lo = mid;
-                else hi = mid - 1;
+        if (threadIdx.x < 64) {  // last row starting at or before seg0: 64 probes at a time
+            int lo = 0, n = nrows;
+            while (n > 1) {
+                const int step = (n + 63) / 64, at = (int)threadIdx.x * step;
+                const bool le = at < n && prefix[lo + at] <= seg0;
+                const int k = 63 - __clzll((long long)(__ballot(le) | 1ull));
+                lo += k * step;
+                n = min(step, n - k * step);
             }
-            srow = lo;
+            if (threadIdx.x == 0) srow = lo;
         }
         __syncthreads();
         int row = srow;
@@ -1047,19 +1060,16 @@ static PPArgs pair_args(const PPPlan& P, float* d_vp, const float* d_scal, const
         A.term = g_pp.term.as<float>();
         A.react = g_pp.react.as<unsigned long long>();
         A.react_scale = P.react_scale;
+        A.order = pp_heavy_lg() ? g_pp.order.as<int>() : nullptr;
         A.taken = reinterpret_cast<int*>(A.react + P.cap * 3);
     }
     return A;
 }
 
-static const int* pair_chunks() {
-    return pp_heavy_lg() ? g_pp.order.as<int>() : g_pp.chunks.as<int>();
-}
-
 // Velocity terms of a pairs-once pass, once every chunk has added to react.
 static int newton_terms(const PPPlan& P, const PPArgs& A, hipStream_t s) {
     Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));
-    k_pp_newton_terms<<<4096, 256, 0, s>>>(A.pos4, A.slot, A.react, A.n_sorted, (int)P.cap, A.scal,
+    k_pp_newton_terms<<<std::min(ceil_div(P.cap, 1024), 4096u), 256, 0, s>>>(A.pos4, A.slot, A.react, A.n_sorted, (int)P.cap, A.scal,
                                             1.0 / (double)P.react_scale, A.learned_range, A.term,
                                             A.red);
     C2_HIP(hipGetLastError());
@@ -1123,9 +1133,10 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
     }
     {
         const int64_t nphys = (int64_t)P.ntile * g.nt * g.nt * g.nt;
-        if (nphys > 0)
-            k_pp_ptotal<<<ceil_div(nphys, 256), 256, 0, s>>>(d_rhoc, g.nt, g.ncb, g.nte, g.p.nnt,
-                                                              g.p.nns, g.ntt, ploc);
+        if (nphys > 0) {
+            const dim3 grid((unsigned)g.ns3, ceil_div((size_t)g.ntt * g.ntt * g.ntt, kPtotalCells));
+            k_pp_ptotal<<<grid, 256, 0, s>>>(d_rhoc, g.nt, g.ncb, g.nte, g.p.nns, g.ntt, ploc);
+        }
         C2_HIP(hipGetLastError());
         k_tile_first<<<ceil_div(P.ntile + 1, 64), 64, 0, s>>>(counts, g_pp.tiles.as<PPTile>(),
                                                               P.ntile, P.c_tot,
@@ -1143,7 +1154,8 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cellid, A.cell_start,
                 n_sorted, &red->err, (int)P.cap, pp_dense_lg(P.newton),
                 P.small, A.learned_occ, A.learned_range, P.newton, A.tiles,
-                P.newton && !pp_heavy_lg() ? P.ntile : 0, g.p.ratio_cs, flags, g_pp.dense.as<int>(),
+                P.newton ? P.ntile : 0, g.p.ratio_cs,
+                P.n_used < kFewSlots ? kPartFew : kPartCand, flags, g_pp.dense.as<int>(),
                 &red->ndense, g_pp.pos4.as<float4>(), g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(flags, (int64_t)P.cap, g_pp.scan_tmp, s));
@@ -1159,19 +1171,21 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                 g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
         }
-        const int* chunks = pair_chunks();
+        const int* chunks = g_pp.chunks.as<int>();
         if (pp_heavy_lg()) {
             Stage st("pp_order", (double)P.cap * 9);
             int* hist = g_pp.order_hist.as<int>();
-            k_chunk_cost<<<kOrderBlocks, kOrderBins, 0, s>>>(A, g_pp.chunks.as<int>(), flags + P.cap,
+            k_chunk_cost<<<kOrderBlocks, kOrderBins, 0, s>>>(A, chunks, flags + P.cap,
                                                              pp_dense_lg(P.newton),
                                                              pp_heavy_lg(),
                                                              g_pp.order_bin.as<unsigned char>(), hist);
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(hist, (int64_t)kOrderBins * kOrderBlocks, g_pp.scan_tmp, s));
-            k_chunk_order<<<kOrderBlocks, kOrderBins, 0, s>>>(g_pp.chunks.as<int>(), g_pp.order_bin.as<unsigned char>(),
+            k_chunk_order<<<kOrderBlocks, kOrderBins, 0, s>>>(P.newton ? nullptr : chunks,
+                                                              g_pp.order_bin.as<unsigned char>(),
                                                               flags + P.cap, hist, g_pp.order.as<int>());
             C2_HIP(hipGetLastError());
+            if (!P.newton) chunks = g_pp.order.as<int>();
         }
         if (P.newton) {
             Stage st("pp_react_zero", (double)P.n_used * 24);
@@ -1180,10 +1194,12 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
         }
         if (P.small)
             C2_TRY(launch_pp_sparse(A, d_rhoc, g.nt, g.ncb, (int)((int64_t)P.ntile * g.nt * g.nt * g.nt),
+                                    g_pp.items.as<int2>(),
+                                    pp_sparse_items((int64_t)P.ntile * g.nt * g.nt * g.nt, P.n_used),
                                     P.small, P.mode, s));
         if (P.help) C2_HIP(hipEventRecord(ctx().ev_pairs, s));
         if (P.newton)
-            C2_TRY(launch_pp_newton(A, chunks, flags, P.grid_pairs, P.small, P.mode, s));
+            C2_TRY(launch_pp_newton(A, chunks, flags, P.grid_pairs, P.small, P.mode, false, s));
         else
             C2_TRY(launch_pp_tiled(A, chunks, flags + P.cap, P.grid_pairs, P.mode, s));
         if (P.newton && !P.help) C2_TRY(newton_terms(P, A, s));
@@ -1254,9 +1270,9 @@ static int pp_apply_kernels(const PPPlan& P, float* d_vp, const double* dv64, hi
 int pp_enqueue_help(const PPPlan& P, hipStream_t s) {
     if (!P.help) return CUBE2_OK;
     C2_HIP(hipStreamWaitEvent(s, ctx().ev_pairs, 0));
-    return launch_pp_newton(pair_args(P, nullptr, nullptr, nullptr), pair_chunks(),
+    return launch_pp_newton(pair_args(P, nullptr, nullptr, nullptr), g_pp.chunks.as<int>(),
                             g_pp.chunk_flags.as<int>(), pp_newton_grid(false), P.small,
-                            P.mode, s);
+                            P.mode, true, s);
 }
 
 void pp_alone(PPPlan& P) {
@@ -1460,7 +1476,7 @@ void pp_release() {
     for (DevBuf* b : {&p.nzero, &p.tiles, &p.ires_loc, &p.apm3, &p.counts, &p.scan_tmp, &p.pos4,
                       &p.slot, &p.cellid, &p.red, &p.tile_first, &p.chunk_flags, &p.chunks,
                       &p.raw_pos4, &p.raw_slot, &p.big, &p.dense, &p.term, &p.rows_len,
-                      &p.rows_base, &p.order, &p.order_bin, &p.order_hist, &p.react})
+                      &p.rows_base, &p.order, &p.order_bin, &p.order_hist, &p.react, &p.items})
         b->release();
     p.valid = false;
 }

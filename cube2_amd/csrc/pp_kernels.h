@@ -13,6 +13,7 @@ struct PPTile {
 // The pairs-once pair kernel's list in runs, each with a counter of its own
 // (on a cache line of its own) from which wavefronts take the next part.
 constexpr int kPartRuns = 64, kRunPad = 32;
+constexpr int kTakenInts = (kPartRuns + 2) * kRunPad;  // (and k_pp_sparse's two)
 
 struct PPRed {
     unsigned long long p_cand, p_acc;  // examined / accepted ordered pairs
@@ -77,6 +78,7 @@ struct PPArgs {
     // sums kept as signed 64-bit fixed point (value * react_scale) at
     // react[c * cap + sorted index]; k_pp_newton_terms turns them into term
     unsigned long long* react;
+    const int* order;  // the parts in another order than the list's, or null
     int* taken;  // per run of the part list (kPartRuns, kRunPad apart): parts taken
     float react_scale;
     int ntt;  // coarse cells per subtile side
@@ -96,17 +98,18 @@ __device__ inline int pp_find_tile(const PPTile* __restrict__ T, int ntile, uint
 }
 
 // Pairs-once pair kernel (pp_newton.hip) over the parts of the chunks:
-// chunks[k] is the chunk of part k, first[a] the first part of chunk a, in the
-// order of the list or (a list ordered otherwise) one each; first[cap] is their
-// number.  Cells of at most `small` particles are k_pp_sparse's (0: none).
+// chunks[k] is the chunk of part k, first[a] the first part of chunk a;
+// first[cap] is their number; they are taken in the order of the list or of
+// a.order.  help: a second launch that joins the first.  Cells of at most `small` particles are k_pp_sparse's (0: none).
 int launch_pp_newton(const PPArgs& a, const int* chunks, const int* first, int grid, int small,
-                     int mode, hipStream_t s);
+                     int mode, bool help, hipStream_t s);
 
 // The small cells' particles of a pairs-once pass (pp_sparse.hip): nt coarse
 // cells per tile side and ncb halo ones, ncoarse physical coarse cells in all.
 bool pp_sparse_fits(int rcp, float range, int ratio_cs);
-int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int small,
-                     int mode, hipStream_t s);
+size_t pp_sparse_items(int64_t ncoarse, int64_t n_used);  // capacity of its list of work items
+int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int2* items,
+                     size_t cap, int small, int mode, hipStream_t s);
 
 // Whether the pair kernel has a pairs-once variant for this PP mode.
 bool pp_newton_mode(int mode);

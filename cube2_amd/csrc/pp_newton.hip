@@ -103,11 +103,9 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
         }
         const int ck = run * len + got;
         const int nxt = take();  // (in flight during the part)
-        const int a0 = uni(chunks[ck]);
-        // its part and the number of parts of the chunk (one if the list is in
-        // another order)
-        const int f0 = uni(first[a0]), np = max(uni(first[a0 + 1]) - f0, 1);
-        const int part = np > 1 ? ck - f0 : 0;
+        const int k = A.order ? uni(A.order[ck]) : ck, a0 = uni(chunks[k]);
+        // the part of the chunk, and the chunk's parts
+        const int f0 = uni(first[a0]), np = uni(first[a0 + 1]) - f0, part = k - f0;
         const uint32_t cid = (uint32_t)uni((int)A.cellid[a0]);
         const int cend = uni(A.cell_start[cid + 1]), cbeg = uni(A.cell_start[cid]);
         const bool grouped = cend - cbeg >= 64;
@@ -349,8 +347,8 @@ __global__ __launch_bounds__(256, 6) void k_pp_newton(PPArgs A, const int* __res
 }
 
 int launch_pp_newton(const PPArgs& a, const int* chunks, const int* first, int grid, int small,
-                     int mode, hipStream_t s) {
-    Stage st(mode == CUBE2_PP_REF ? "pp_pairs_ref" : "pp_pairs_fastq");
+                     int mode, bool help, hipStream_t s) {
+    Stage st(help ? "pp_pairs_help" : mode == CUBE2_PP_REF ? "pp_pairs_ref" : "pp_pairs_fastq");
     const unsigned blocks = (unsigned)std::max(1, grid);
     const int dl = pp_dense_lg(true);
     if (mode == CUBE2_PP_REF && pp_jbatch() == 128)

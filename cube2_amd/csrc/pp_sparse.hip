@@ -8,8 +8,8 @@
 // and most of its memory traffic (cell starts, and registers spilled around
 // each chunk).
 //
-// Here a wavefront takes a coarse cell: it lists the particles of its small
-// cells, up to 64 at a time, and walks the cells within R of any of them once
+// Here a wavefront takes part of a coarse cell: it lists the particles of its
+// small cells, up to 64 at a time, and walks the cells within R of any of them once
 // for all, each row of cells being read once instead of once per particle.  Every j of that
 // region is tested against every i (lane (i, s) takes j slot t + s); whether
 // j's cell lies in i's stencil, for the count of candidates, is one packed
@@ -17,13 +17,14 @@
 // forces evaluated 64 at a time, summed per i as 64-bit fixed point (integer
 // LDS atomics; float ones cost ~190 cycles an instruction on gfx950).  These
 // particles evaluate all their pairs themselves and nothing else adds to
-// them (k_chunk_flags marks them), so their sums are stored, not added.
+// them (k_chunk_flags marks them), so their sums are stored, not added, unless
+// their j are split.
 // Bound by VALU issue: the region's tests.  The particles beside a clump cost
-// the most by far, one batch of them up to 1 ms; kParts wavefronts share a
-// coarse cell, so that such batches run side by side.  REF, clustered: 7.9 ms
-// at 256^3 (kParts 1: 12.1, 4: 7.9, 16: 11.7, empty parts counting), 2.0 ms
-// at 128^3 (3.8, 2.1, 1.9); the pair kernel falls from 57.8 to 32.4 and from
-// 7.8 to 3.9 ms.
+// the most by far, one batch of them up to 1 ms, and the kernel waits for the
+// last: k_sparse_items shares a coarse cell among wavefronts and lists the
+// costly ones first.  REF, clustered, ms at 256^3 / 128^3 / 120^3 in level-6
+// cells: a wavefront per coarse cell 12.1 / 3.8 / 2.3, eight 7.9 / 2.0 / 1.1,
+// with j split too 8.1 / 1.1 / 0.94 (128^3 drop-in call 14.7 -> 13.7).
 #include <algorithm>
 
 #include "common.h"
@@ -73,46 +74,107 @@ __device__ inline int quot(int n, unsigned recip) { return (int)__umulhi((unsign
 // their particles needs, large ones read rows less often (at 256^3 with one
 // wavefront per coarse cell 4: 17.1 ms, 8: 13.0, 16: 12.1, 32: 13.2).
 constexpr float kBlockCount = 16.0f;
-// Wavefronts that share a coarse cell's blocks.
-constexpr int kParts = 8;
+// Items of a coarse cell: its blocks in kParts, each once per kItemCount
+// particles of the 27 coarse cells (at most kMaxSplit), the j of the regions
+// split among the latter (ms as above: 4096: 8.6 / 1.15 / 0.84, 16384: 8.1 /
+// 1.1 / 0.94, 65536: 7.7 / 1.45 / 1.1).
+constexpr int kParts = 8, kItemCount = 16384, kMaxSplit = 16;
+
+// The items of every coarse cell that holds particles: x = the cell, y = part,
+// split, splits and blocks per side.  Those of split cells go to the front of
+// the list (count[0]) and are taken first, the others to its end
+// (count[kRunPad]).
+__global__ __launch_bounds__(256) void k_sparse_items(const int* __restrict__ rhoc, int nt, int ncb,
+                                                      int ncoarse, const PPTile* __restrict__ tiles,
+                                                      const int* __restrict__ err, int cap,
+                                                      int2* __restrict__ items, int* __restrict__ count) {
+    const int w = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+    __shared__ int wsum[2][4], first[2];
+    int nitem = 0, parts = 0, splits = 1, nb1 = 1;
+    if (w < ncoarse && *err == 0) {
+        const int t = w / (nt * nt * nt), wr = w - t * nt * nt * nt, nte = nt + 2 * ncb;
+        const int x = wr % nt + ncb, y = wr / nt % nt + ncb, z = wr / (nt * nt) + ncb;
+        const int* c0 = rhoc + (((size_t)t * nte + z) * nte + y) * nte + x;
+        if (*c0 > 0) {
+            long long n27 = 0;
+            for (int dz = -1; dz <= 1; dz++)
+                for (int dy = -1; dy <= 1; dy++)
+                    for (int dx = -1; dx <= 1; dx++)
+                        n27 += max(c0[((long long)dz * nte + dy) * nte + dx], 0);
+            const int rcp = tiles[t].rcp;
+            const float mean = (float)n27 * (1.0f / 27.0f);
+            nb1 = min(rcp, max(1, (int)ceilf(cbrtf(mean * (1.0f / kBlockCount)))));
+            const int Bs = (rcp + nb1 - 1) / nb1, nbl = (rcp + Bs - 1) / Bs;
+            parts = min(kParts, nbl * nbl * nbl);
+            splits = (int)min(1 + n27 / kItemCount, (long long)kMaxSplit);
+            nitem = parts * splits;
+        }
+    }
+#pragma unroll
+    for (int heavy = 0; heavy < 2; heavy++) {
+        const int mine = (splits > 1) == (heavy == 1) ? nitem : 0;
+        int inc = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += u;
+        }
+        if (lane == 63) wsum[heavy][threadIdx.x >> 6] = inc;
+        __syncthreads();
+        if (threadIdx.x == 0) {  // one atomic per block
+            int tot = 0;
+            for (int v = 0; v < 4; v++) {
+                const int n = wsum[heavy][v];
+                wsum[heavy][v] = tot;
+                tot += n;
+            }
+            first[heavy] = tot ? atomicAdd(&count[heavy ? 0 : kRunPad], tot) : 0;
+        }
+        __syncthreads();
+        int at = first[heavy] + wsum[heavy][threadIdx.x >> 6] + inc - mine;
+        for (int k = 0; k < mine; k++, at++)
+            if (at < cap)
+                items[heavy ? at : cap - 1 - at] =
+                    make_int2(w, k % parts | parts << 4 | k / parts << 8 | splits << 16 | nb1 << 24);
+    }
+}
 
 template <int kMode>
-__global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __restrict__ rhoc, int nt,
-                                                      int ncb, int ncoarse, int small) {
+__global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __restrict__ items, int cap,
+                                                      const int* __restrict__ count, int nt, int small) {
     __shared__ SparseLDS lds[4];
     const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     SparseLDS& L = lds[wave];
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     const FraK Ka = uni(make_frak(A.app));
     unsigned long long pc = 0, pa = 0;  // (wavefront-uniform)
-    const int nw = A.red->err == 0 ? ncoarse * kParts : 0;
-    // neighbouring coarse cells share most of their j: one XCD takes a run
-    for (int w = (int)xcd_remap(blockIdx.x, gridDim.x) * 4 + wave; w < nw; w += gridDim.x * 4) {
-        const int cw = w / kParts, part = w % kParts;
+    // the split cells' items by all blocks alike; neighbouring coarse cells
+    // share most of their j: one XCD takes a run of the others
+    const int nheavy = min(count[0], cap), nlight = min(count[kRunPad], cap - nheavy);
+    bool heavy = true;
+    int w = (int)blockIdx.x * 4 + wave;
+    for (;; w += gridDim.x * 4) {
+        if (heavy && w >= nheavy) {
+            heavy = false;
+            w = (int)xcd_remap(blockIdx.x, gridDim.x) * 4 + wave;
+        }
+        if (!heavy && w >= nlight) break;
+        const int2 item = items[heavy ? w : cap - 1 - w];
+        const int cw = uni(item.x), code = uni(item.y);
+        const int part = code & 15, parts = code >> 4 & 15, sp = code >> 8 & 255, splits = code >> 16 & 255;
         const int t = cw / (nt * nt * nt), wr = cw - t * nt * nt * nt;
         const PPTile T = A.tiles[t];
         const int S = T.S, rcp = T.rcp;
         const int bx = (wr % nt + 1) * rcp, by = (wr / nt % nt + 1) * rcp, bz = (wr / (nt * nt) + 1) * rcp;
         const unsigned off = (unsigned)T.cell_off;
-        // mean count of the 27 coarse cells around -> side of a block
-        float mean = 0.0f;
-        {
-            const int nte = nt + 2 * ncb, l = min(lane, 26);
-            const size_t cc = (((size_t)t * nte + wr / (nt * nt) + ncb - 1 + l / 9) * nte + wr / nt % nt +
-                               ncb - 1 + l / 3 % 3) * nte + wr % nt + ncb - 1 + l % 3;
-            int c = lane < 27 ? rhoc[cc] : 0;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-            mean = (float)uni(c) * (1.0f / 27.0f);
-        }
-        const int nb1 = min(rcp, max(1, (int)ceilf(cbrtf(mean * (1.0f / kBlockCount)))));
+        const int nb1 = code >> 24;  // (from the mean count of the 27 coarse cells around)
         const int Bs = uni((rcp + nb1 - 1) / nb1), nbl = (rcp + Bs - 1) / Bs;  // blocks of Bs^3 cells
         const int nblk = nbl * nbl * nbl, cblk = Bs * Bs * Bs;  // blocks, cells of one
-        const int ncell = nblk * (part + 1) / kParts * cblk;
+        const int ncell = nblk * (part + 1) / parts * cblk;
         const unsigned i1 = recip_u32(Bs), i2 = recip_u32(Bs * Bs), i3 = recip_u32(Bs * Bs * Bs);
         const unsigned k1 = recip_u32(nbl), k2 = recip_u32(nbl * nbl);
         const unsigned long long pc0 = pc, pa0 = pa;
-        int c0 = nblk * part / kParts * cblk, depth = 0, n = 0, first = 0, blk = 0, head = 0, tail = 0;
+        int c0 = nblk * part / parts * cblk, depth = 0, n = 0, first = 0, blk = 0, head = 0, tail = 0;
         unsigned cpk = 0;
         float range = 0.0f;
         FraK Kr = Ka;
@@ -211,7 +273,9 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __res
                     const int u = __shfl_up(inc, o, 64);
                     if (lane >= o) inc += u;
                 }
-                const int M = uni(__shfl(inc, 63, 64));
+                const int M0 = uni(__shfl(inc, 63, 64));
+                // this split's candidates [v0, M) of the group's
+                const int v0 = (int)((long long)M0 * sp / splits), M = (int)((long long)M0 * (sp + 1) / splits);
                 L.rs[lane] = js - (inc - cnt);
                 L.rp[lane] = inc;
                 wave_lds_sync();
@@ -229,8 +293,8 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __res
                     }
                     return q4;
                 };
-                float4 qc = fetch(0);
-                for (int vb = 0; vb < M; vb += 64) {
+                float4 qc = fetch(v0);
+                for (int vb = v0; vb < M; vb += 64) {
                     const int nb = min(64, M - vb);
                     qc.w = __uint_as_float(rc + jc);
                     L.jb[lane] = qc;
@@ -290,10 +354,14 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int* __res
             wave_lds_sync();
             if (qtail > qhead) sparse_flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr, A.react_scale);
             pa += (unsigned)qtail;
-            pc -= (unsigned)ni;  // the particles themselves
+            if (sp == 0) pc -= (unsigned)ni;  // the particles themselves
             if (vi && jslot == 0)
 #pragma unroll
-                for (int c = 0; c < 3; c++) A.react[c * (size_t)A.cap + ia] = L.acc[islot][c];
+                for (int c = 0; c < 3; c++) {
+                    unsigned long long* d = A.react + c * (size_t)A.cap + ia;
+                    if (splits > 1) atomicAdd(d, L.acc[islot][c]);
+                    else *d = L.acc[islot][c];
+                }
             wave_lds_sync();  // acc, the queue and the list are reused
         }
         if (A.tile_pairs && lane == 0) {  // per-tile counts (on request only)
@@ -312,8 +380,14 @@ bool pp_sparse_fits(int rcp, float range, int ratio_cs) {
     return R < 512.0 && rcp + 3.0 * R < 512.0;
 }
 
-int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int small,
-                     int mode, hipStream_t s) {
+// A coarse cell has up to kParts items and kParts more per kItemCount particles
+// around it; a slot is around 27 coarse cells.
+size_t pp_sparse_items(int64_t ncoarse, int64_t n_used) {
+    return (size_t)(ncoarse * kParts + n_used * 27 * kParts / kItemCount + 1);
+}
+
+int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int2* items,
+                     size_t cap, int small, int mode, hipStream_t s) {
     if (ncoarse <= 0) return CUBE2_OK;
     Stage st("pp_pairs_sparse");
     int dev = 0, ncu = 0;
@@ -323,8 +397,12 @@ int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoa
     // as the pair kernel's: far more blocks than are resident, so that the
     // hardware balances their uneven costs
     const unsigned blocks = (unsigned)std::min(ceil_div((size_t)ncoarse * kParts, 4), (unsigned)std::max(1, ncu) * 64u);
-    if (mode == CUBE2_PP_REF) k_pp_sparse<kModeRef><<<blocks, 256, 0, s>>>(a, rhoc, nt, ncb, ncoarse, small);
-    else k_pp_sparse<kModeFast><<<blocks, 256, 0, s>>>(a, rhoc, nt, ncb, ncoarse, small);
+    int* count = a.taken + kPartRuns * kRunPad;
+    k_sparse_items<<<ceil_div((size_t)ncoarse, 256), 256, 0, s>>>(rhoc, nt, ncb, ncoarse, a.tiles, &a.red->err,
+                                                                  (int)cap, items, count);
+    C2_HIP(hipGetLastError());
+    if (mode == CUBE2_PP_REF) k_pp_sparse<kModeRef><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small);
+    else k_pp_sparse<kModeFast><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }

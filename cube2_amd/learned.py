@@ -13,9 +13,11 @@ Training (this module): samples are the particles the network stands in for
 particles) of C1-style boxes kicked by the plain PP alone; a sample is the
 10^3 x 4 input patch whose 2^3 outputs surround the particle, its CIC
 fractions and its plain-PP acceleration.  The forward pass runs the
-library's matrix-core convolution (cube2_cnn_conv3_dev); the backward pass
-im2col and BF16 GEMMs (cube2_gemm_bf16_dev); the loss is the CIC
-combination's MSE (cube2_cnn_cic_mse_dev); Adam updates FP32 master weights.
+library's matrix-core convolution (cube2_cnn_conv3_dev) in one call for all
+layers, the backward pass over patches one product kernel per gradient
+(cube2_cnn_net_backward_dev; larger grids im2col and BF16 GEMMs,
+cube2_gemm_bf16_dev); the loss is the CIC combination's MSE
+(cube2_cnn_cic_mse_dev); Adam updates FP32 master weights.
 
 In the kick (cube2_kick_dev with CUBE2_KICK_LEARNED, after
 ``LearnedPP.load``), the library evaluates the same layers over each

@@ -1,10 +1,10 @@
 """The pairs-once pair kernel's work list: a chunk of many candidates in parts,
 taken from counters by whatever wavefronts there are.  One block per CU or 64,
-beside PM3 (whose stream joins at the end) or after it: the same partial sums
-in integers, so the same bits.  Whole chunks (a list ordered by cost) are the
-same pairs in other groups of at most 64 summed in FP32: the same counts,
-Delta-v to 1e-6 relative RMS.  From fewer parts than runs of the list to cells
-of thousands of particles."""
+beside PM3 (whose stream joins at the end) or after it, in list order or by
+cost: the same partial sums in integers, so the same bits.  Chunks of 16
+particles are the same pairs in other groups of at most 64 summed in FP32: the
+same counts, Delta-v to 1e-6 relative RMS.  From fewer parts than runs of the
+list to cells of thousands of particles."""
 from __future__ import annotations
 
 import numpy as np
@@ -42,15 +42,15 @@ def test_parts_and_joining_streams_give_the_same_sums(n, clump, width, levels):
 
     print(f"parts: {n} + {clump} particles, levels {levels}", flush=True)
     v, cnt = kick(False)
-    for blocks in (1, 64):
-        v1, c1 = kick(False, pp_blocks_per_cu=blocks)
+    for tune in (dict(pp_blocks_per_cu=1), dict(pp_blocks_per_cu=64), dict(pp_order=2)):
+        v1, c1 = kick(False, **tune)
         assert c1 == cnt and np.array_equal(v1.view(np.uint32), v.view(np.uint32))
     va, ca = kick(True, kick_overlap=2)
     for blocks in (1, 3):
         vb, cb = kick(True, pp_overlap_blocks=blocks)
         assert ca == cb == cnt and np.array_equal(va.view(np.uint32), vb.view(np.uint32))
-    vo, co = kick(False, pp_order=2)
+    vo, co = kick(False, pp_dense_lg=4)
     err = np.sqrt(((vo - v).astype(np.float64) ** 2).sum() / max((v.astype(np.float64) ** 2).sum(), 1e-300))
-    print(f"  P_cand {cnt[0]} P_acc {cnt[1]}, whole chunks {err:.1e}", flush=True)
+    print(f"  P_cand {cnt[0]} P_acc {cnt[1]}, chunks of 16 {err:.1e}", flush=True)
     assert co == cnt
     assert err < 1e-6
