@@ -93,9 +93,12 @@ __device__ inline int find_tile2(const PPTile* __restrict__ T, int ntile, uint32
 // capped for 6 wavefronts per SIMD (REF at 256^3, ordered pairs: 80.7 ms;
 // budgets for 5 and 7 wavefronts 89.2 and 86.0 ms; 4 blocks per CU instead
 // of 6: 105 ms).  The REF variant spills a few registers outside its inner
-// loops.
+// loops.  PRECISE and PLUMMER with their FP64 sums have the budget for 5, which
+// takes no spills (6: 21 to 29 around each chunk): PRECISE on a 96^3 lattice
+// 1.78 -> 1.54 ms, a PLUMMER kick of 64^3 clustered particles 4.07 -> 3.91; where
+// a clump's long chunks decide, the same (64^3 2.58, 2.60; 96^3 6.95, 6.93).
 template <int kMode, int kJB>
-__global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __restrict__ chunks,
+__global__ __launch_bounds__(256, kMode >= kModePrecise ? 5 : 6) void k_pp_tiled(PPArgs A, const int* __restrict__ chunks,
                                                   const int* __restrict__ nchunks_dev,
                                                   int direct_lg, int dense_lg) {
     static_assert(kJB == 64 || kJB == 128, "j batch of 64 or 128");
@@ -106,7 +109,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
     const int nchunks = uni(*nchunks_dev);
 
     float f2 = 0.f, v0 = 0.f, v1 = 0.f, v2 = 0.f;
-    unsigned long long pc = 0, pa = 0;
+    unsigned long long pc = 0, pa = 0;  // (pc wavefront-uniform)
     for (int ck = blockIdx.x * 4 + wave; ck < nchunks; ck += gridDim.x * 4) {
         const int a0 = uni(chunks[ck]);
         const uint32_t cid = (uint32_t)uni((int)A.cellid[a0]);
@@ -126,10 +129,10 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
         const float4 p = A.pos4[ia];
         const int ti = uni(find_tile2(A.tiles, A.ntile, cid));
         const PPTile T = A.tiles[ti];
-        const unsigned long long pc0 = pc, pa0 = pa;
-        const long long key = (long long)cid - T.cell_off;
+        unsigned ncand = 0;  // (wavefront-uniform)
         const int S = T.S;
-        const int x = (int)(key % S), y = (int)((key / S) % S), z = (int)(key / ((long long)S * S));
+        const unsigned key = cid - (unsigned)T.cell_off;
+        const int x = (int)(key % S), y = (int)(key / S % S), z = (int)(key / ((unsigned)S * S));
         // one subtile per PP cell: same range for the chunk
         const float range = uni(p.w);
         int R;
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             if (r < nrows) {
                 const int zz = z + r / W - R, yy = y + r % W - R;
                 if (zz >= 0 && zz < S && yy >= 0 && yy < S) {
-                    const long long row = T.cell_off + ((long long)zz * S + yy) * S;
+                    const unsigned row = (unsigned)T.cell_off + ((unsigned)zz * S + yy) * S;
                     js = A.cell_start[row + xlo];
                     cnt = A.cell_start[row + xhi + 1] - js;
                 }
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             L.rs[lane] = js - (inc - cnt);
             L.rp[lane] = inc;
             wave_lds_sync();
-            if (vi && jslot == 0) pc += (unsigned long long)M;
+            ncand += (unsigned)M;
             // a lane's candidates v = vb + lane only grow, so its row (the
             // first with rp > v) is found by walking forward from the last
             // one: rp of the rows past the group is M > v, so the walk stops
@@ -304,14 +307,14 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
                 atomicAdd(&L.acc[islot][1], day);
                 atomicAdd(&L.acc[islot][2], daz);
             }
-            pa += npa;
             wave_lds_sync();
         }
         if (qtail > qhead) flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr);
-        if (lane == 0) pa += (unsigned long long)qtail;
+        if (lane == 0) npa += (unsigned)qtail;
+        pa += npa;
+        pc += (unsigned long long)(ncand - 1u) * (unsigned)ni;  // (not the particle itself)
         if (vi && jslot == 0) {
 #pragma clang fp contract(off)
-            pc -= 1;  // the particle itself
             const int a = ia;
             const float ax = (float)L.acc[islot][0], ay = (float)L.acc[islot][1],
                         az = (float)L.acc[islot][2];
@@ -340,9 +343,9 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
             }
         }
         if (A.tile_pairs) {  // per-tile counts (on request only)
-            const unsigned long long dc = wave_sum_u64(pc - pc0), da = wave_sum_u64(pa - pa0);
+            const unsigned long long da = wave_sum_u64(npa);
             if (lane == 0) {
-                atomicAdd(&A.tile_pairs[2 * ti], dc);
+                atomicAdd(&A.tile_pairs[2 * ti], (unsigned long long)(ncand - 1u) * (unsigned)ni);
                 atomicAdd(&A.tile_pairs[2 * ti + 1], da);
             }
         }
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(256, 6) void k_pp_tiled(PPArgs A, const int* __rest
     }
     const float mx[4] = {f2, v0, v1, v2};
     block_max_to<4>(&A.red->f2max_bits, mx);
-    const unsigned long long sm[2] = {pc, pa};
+    const unsigned long long sm[2] = {lane == 0 ? pc : 0ull, pa};
     block_sum_to<2>(&A.red->p_cand, sm);
 }
 
