@@ -80,14 +80,14 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
         out = kept[blockIdx.x];
         if (kept[blockIdx.x + 1] == out) return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
+    const int v0 = (int)blockIdx.x * kSlotChunk;
     const int dmax = (A.nlayer - 2) / 2;
     const float rf = (float)A.ratio_cs, irf = 1.0f / rf;
     const double rd = 1.0 / 65536.0 * (double)A.ratio_cs, ird = 1.0 / rd;
     unsigned bad = 0;
     int mine = 0;  // kept slots of the wavefront's windows
     constexpr int kIt = kSlotChunk / kSlotThreads;
-    walk_slots(A.start, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+    walk_slots(A.start, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
         uint32_t kk[kIt], ss[kIt];
         int16_t code[kIt][3];
         uint64_t km[kIt];
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
             if (v < e) {
                 int s0, s1;
                 const CellPos c = cell_pos(G, cell_of(v, s0, s1));
-                const int64_t sh = row_shift(A.start, A.idx_b_r, c.row, G.nte.d);
+                const int64_t sh = row_shift(A.start, A.idx_b_r, c.row, G.nte.d) + v0;
                 if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > A.n_used) {
                     bad |= 1u;
                 } else {
@@ -186,13 +186,13 @@ __global__ __launch_bounds__(kSlotThreads) void k_slot_positions(
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1u);
         return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
+    const int v0 = (int)blockIdx.x * kSlotChunk;
     unsigned bad = 0;
-    walk_slots(start, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+    walk_slots(start, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));
-            const int64_t sh = row_shift(start, idx_b_r, c.row, G.nte.d);
+            const int64_t sh = row_shift(start, idx_b_r, c.row, G.nte.d) + v0;
             if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > n_used) {
                 bad = 1u;
                 continue;

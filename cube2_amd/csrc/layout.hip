@@ -126,8 +126,8 @@ __global__ __launch_bounds__(kSlotThreads) void k_layout_fill(
     const int16_t* __restrict__ code_s, const float* __restrict__ vel_s, int16_t* __restrict__ xp,
     float* __restrict__ vp) {
     __shared__ int win[kSlotWin + 1];
-    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
-    walk_slots(slot, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+    const int v0 = (int)blockIdx.x * kSlotChunk;
+    walk_slots(slot, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kSlotThreads) void k_layout_fill(
             const int nc = (int)G.nc.d;
             const int g = (image_coord(G, tz, c.k) * nc + image_coord(G, ty, c.j)) * nc +
                           image_coord(G, tx, c.i);
-            const int64_t p = (int64_t)gstart[g] + (v - s0), d = v;
+            const int64_t p = (int64_t)gstart[g] + (v - s0), d = (int64_t)v0 + v;
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 xp[3 * d + k] = code_s[3 * p + k];
@@ -160,6 +160,10 @@ int layout_build(const double* d_pos, const float* d_vel, int64_t n, int* d_rhoc
     hipStream_t s = C.stream;
     const int64_t nbin = (int64_t)g.nc * g.nc * g.nc;
     const int64_t ncells = (int64_t)g.ntile * g.nte * g.nte * g.nte;
+    if (ncells >= ((int64_t)1 << 31)) {
+        set_error("layout: more than 2^31 cells with the halos");
+        return CUBE2_ERR_CAPACITY;
+    }
     const int64_t nrows = (int64_t)g.ntile * g.nte * g.nte;
     const size_t nn = (size_t)std::max<int64_t>(n, 1);
     C2_TRY(g_lay.gid.reserve(nn * 4));
@@ -251,10 +255,10 @@ __global__ __launch_bounds__(kSlotThreads) void k_halo_vp(SlotGeom G,
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1);
         return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk, v1 = min(total, v0 + kSlotChunk);
+    const int v0 = (int)blockIdx.x * kSlotChunk;
     const int nte = (int)G.nte.d;
     int bad = 0;
-    walk_slots(start, G.ncells, v0, v1, win, [&](int b, int e, auto cell_of) {
+    walk_slots(start, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(kSlotThreads) void k_halo_vp(SlotGeom G,
             const uint32_t ts = (uint32_t)((st[2] * (int)G.nnt.d + st[1]) * (int)G.nnt.d + st[0]);
             const uint32_t rs = (ts * nte + sc[2]) * nte + sc[1], qs = rs * nte + sc[0];
             const int u0 = start[qs], u1 = start[qs + 1];
-            const int64_t h0 = row_shift(start, idx_b_r, c.row, nte);
+            const int64_t h0 = row_shift(start, idx_b_r, c.row, nte) + v0;
             const int64_t h1 = row_shift(start, idx_b_r, rs, nte);
             if (v < s0 || v >= s1 || u1 - u0 != s1 - s0 || s0 + h0 < 0 || u0 + h1 < 0 || s1 + h0 > n_used ||
                 u1 + h1 > n_used) {

@@ -93,20 +93,21 @@ __device__ inline uint32_t block_last_le(const int* __restrict__ start, uint32_t
     return lo;
 }
 
-// Block-wide walk of slots [v0, v1) of the running slot count `start`
-// [ncells + 1] (win: kSlotWin + 1 ints of LDS).  For each window of cells,
-// body(begin, end, cell_of) with the slots [begin, end) it covers; cell_of(v,
-// s0, s1) gives slot v's cell and the cell's slot range.  body is called
-// block-uniformly and may synchronise.
+// Block-wide walk of the n <= kSlotChunk slots from v0 on of the running slot
+// count `start` [ncells + 1] (win: kSlotWin + 1 ints of LDS).  For each window
+// of cells, body(begin, end, cell_of) with the slots [begin, end) it covers,
+// counted from v0 (the last block's v0 + kSlotChunk may pass 2^31); cell_of(v,
+// s0, s1) gives slot v's cell and the cell's slot range, counted alike (a range
+// may begin before v0).  body is called block-uniformly and may synchronise.
 template <class Body>
-__device__ inline void walk_slots(const int* __restrict__ start, uint32_t ncells, int v0, int v1,
+__device__ inline void walk_slots(const int* __restrict__ start, uint32_t ncells, int v0, int n,
                                   int* win, Body&& body) {
-    for (int v = v0; v < v1;) {
-        const uint32_t q0 = block_last_le(start, ncells, v);
+    for (int v = 0; v < n;) {
+        const uint32_t q0 = block_last_le(start, ncells, v0 + v);
         const int nw = (int)min((uint32_t)kSlotWin, ncells - q0);
-        for (int a = threadIdx.x; a <= nw; a += kSlotThreads) win[a] = start[q0 + a];
+        for (int a = threadIdx.x; a <= nw; a += kSlotThreads) win[a] = start[q0 + a] - v0;
         __syncthreads();
-        const int end = min(v1, max(win[nw], v + 1));
+        const int end = min(n, max(win[nw], v + 1));
         body(v, end, [&](int s, int& s0, int& s1) {
             int lo = 0, hi = nw;
             while (hi - lo > 1) {
@@ -122,6 +123,9 @@ __device__ inline void walk_slots(const int* __restrict__ start, uint32_t ncells
         v = end;
     }
 }
+
+// Slots of the block at v0 of `total`.
+__device__ inline int block_slots(int total, int v0) { return min(kSlotChunk, max(total - v0, 0)); }
 
 // Running slot counts of the cells (scan.hip: negative counts as 0) and,
 // per row, what to add to a running count to get a slot: idx_b_r of the row
