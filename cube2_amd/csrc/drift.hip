@@ -17,7 +17,7 @@
 //   counts   run boundaries of the sorted cells give the new rhoc (halo
 //            cells 0), a row scan gives idx_b_r;
 //   gather   codes and velocities of the kept slots in sorted order.
-// At 256^3 (90 M slots, 16.7 M kept) the two key passes take 0.67 and 0.30 ms
+// At 256^3 (90 M slots, 16.7 M kept) the two key passes take 0.64 and 0.31 ms
 // (18 bytes a slot: 2.4 TB/s) and the sort 0.9 ms; a wavefront per cell that
 // wrote and sorted every slot took 5.9 and 3.3 ms.
 #include <algorithm>
@@ -41,7 +41,7 @@ static DriftState g_dr;
 
 struct DriftArgs {
     SlotGeom G;
-    const int* start;  // running slot counts of the extended cells
+    const long long* start;  // running slot counts of the extended cells
     const int64_t* idx_b_r;
     const int16_t* xp;
     const float* vp;
@@ -67,8 +67,8 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
     __shared__ int wsum[kSlotThreads / 64];
     const SlotGeom& G = A.G;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int total = A.start[G.ncells];
-    if (total < 0 || total > A.n_used) {
+    const int64_t total = A.start[G.ncells];
+    if (total > A.n_used) {
         if (!kEmit && threadIdx.x == 0) {
             kept[blockIdx.x] = 0;
             if (blockIdx.x == 0) atomicOr(err, 1u);
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
         out = kept[blockIdx.x];
         if (kept[blockIdx.x + 1] == out) return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk;
+    const int64_t v0 = (int64_t)blockIdx.x * kSlotChunk;
     const int dmax = (A.nlayer - 2) / 2;
     const float rf = (float)A.ratio_cs, irf = 1.0f / rf;
     const double rd = 1.0 / 65536.0 * (double)A.ratio_cs, ird = 1.0 / rd;
@@ -99,11 +99,10 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
             if (v < e) {
                 int s0, s1;
                 const CellPos c = cell_pos(G, cell_of(v, s0, s1));
-                const int64_t sh = row_shift(A.start, A.idx_b_r, c.row, G.nte.d) + v0;
-                if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > A.n_used) {
+                const int64_t ip = v + v0 + row_shift(A.start, A.idx_b_r, c.row, G.nte.d);
+                if (ip < 0 || ip >= A.n_used) {
                     bad |= 1u;
                 } else {
-                    const int64_t ip = v + sh;
                     const int src[3] = {c.i, c.j, c.k};
                     int ig[3];
                     float f[3];
@@ -175,29 +174,27 @@ __global__ __launch_bounds__(kSlotThreads) void k_drift_keys(
 
 // Positions (standard cells, FP64, wrapped into [0, ng)) of every slot of
 // the image: a block per kSlotChunk slots (16.7 M slots without halo copies:
-// 0.18 ms; a wavefront per cell 1.85 ms).
+// 0.19 ms; a wavefront per cell 1.85 ms).
 __global__ __launch_bounds__(kSlotThreads) void k_slot_positions(
-    SlotGeom G, const int* __restrict__ start, const int64_t* __restrict__ idx_b_r,
+    SlotGeom G, const long long* __restrict__ start, const int64_t* __restrict__ idx_b_r,
     const int16_t* __restrict__ xp, int64_t n_used, int ratio_cs, double* __restrict__ pos,
     unsigned* __restrict__ err) {
     __shared__ int win[kSlotWin + 1];
-    const int total = start[G.ncells];
-    if (total < 0 || total > n_used) {
+    const int64_t total = start[G.ncells];
+    if (total > n_used) {
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1u);
         return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk;
     unsigned bad = 0;
-    walk_slots(start, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
+    walk_all_slots(start, G.ncells, total, win, [&](int64_t v0, int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));
-            const int64_t sh = row_shift(start, idx_b_r, c.row, G.nte.d) + v0;
-            if (v < s0 || v >= s1 || s0 + sh < 0 || s1 + sh > n_used) {
+            const int64_t ip = v + v0 + row_shift(start, idx_b_r, c.row, G.nte.d);
+            if (ip < 0 || ip >= n_used) {
                 bad = 1u;
                 continue;
             }
-            const int64_t ip = v + sh;
             int tx, ty, tz;
             tile_pos(G, c.tile, tx, ty, tz);
             const int gc[3] = {image_coord(G, tx, c.i), image_coord(G, ty, c.j),
@@ -292,13 +289,13 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
     C2_TRY(ensure_init());
     hipStream_t s = C.stream;
     const int64_t ncells = (int64_t)g.nte * g.nte * g.nte * g.ntile;
-    if (ncells >= ((int64_t)1 << 31) || n_used >= ((int64_t)1 << 31) - kSlotChunk) {
-        set_error("drift: image too large for 32-bit slots");
+    if (ncells >= ((int64_t)1 << 31)) {
+        set_error("drift: image too large for 32-bit cells");
         return CUBE2_ERR_CAPACITY;
     }
     const int64_t nrows = (int64_t)g.ntile * g.nte * g.nte;
     const int64_t nblk = std::max<int64_t>(1, (n_used + kSlotChunk - 1) / kSlotChunk);
-    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(int)));
+    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(long long)));
     C2_TRY(g_dr.kept.reserve((size_t)(nblk + 1) * sizeof(int)));
     C2_TRY(g_dr.bounds.reserve((size_t)(2 * ncell_phys) * sizeof(int)));
     C2_TRY(g_dr.rows.reserve((size_t)(nrows + 1) * sizeof(int)));
@@ -311,7 +308,7 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
     C2_TRY(fill_zero(err, sizeof(unsigned), s));
     DriftArgs A;
     A.G = make_slotgeom(g);
-    A.start = g_dr.start.as<int>();
+    A.start = g_dr.start.as<long long>();
     A.idx_b_r = d_idx_b_r;
     A.xp = d_xp;
     A.vp = d_vp;
@@ -324,7 +321,7 @@ int drift(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d_xp, cons
     int* h = g_dr.h_red.as<int>();
     {
         Stage st("drift_keys", (double)n_used * (6 + 12));
-        C2_TRY(exclusive_scan_counts(d_rhoc, g_dr.start.as<int>(), ncells, g_dr.scan_tmp, s));
+        C2_TRY(exclusive_scan_counts(d_rhoc, g_dr.start.as<long long>(), ncells, g_dr.scan_tmp, s));
         auto kern = pow2 ? k_drift_keys<false, true> : k_drift_keys<false, false>;
         kern<<<(unsigned)nblk, kSlotThreads, 0, s>>>(A, kept, nullptr, nullptr, nullptr, nullptr, err);
         C2_HIP(hipGetLastError());
@@ -407,18 +404,18 @@ int slot_positions(const int* d_rhoc, const int64_t* d_idx_b_r, const int16_t* d
     C2_TRY(ensure_init());
     hipStream_t s = C.stream;
     const int64_t ncells = (int64_t)g.nte * g.nte * g.nte * g.ntile;
-    if (ncells >= ((int64_t)1 << 31) || n_used >= ((int64_t)1 << 31) - kSlotChunk) {
-        set_error("positions: image too large for 32-bit slots");
+    if (ncells >= ((int64_t)1 << 31)) {
+        set_error("positions: image too large for 32-bit cells");
         return CUBE2_ERR_CAPACITY;
     }
     C2_TRY(g_dr.red.reserve(sizeof(unsigned)));
     C2_TRY(g_dr.h_red.reserve(2 * sizeof(int)));
-    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(int)));
+    C2_TRY(g_dr.start.reserve((size_t)(ncells + 1) * sizeof(long long)));
     unsigned* err = g_dr.red.as<unsigned>();
     C2_TRY(fill_zero(err, sizeof(unsigned), s));
-    int* start = g_dr.start.as<int>();
+    long long* start = g_dr.start.as<long long>();
     C2_TRY(exclusive_scan_counts(d_rhoc, start, ncells, g_dr.scan_tmp, s));
-    k_slot_positions<<<ceil_div((size_t)std::max<int64_t>(n_used, 1), kSlotChunk), kSlotThreads, 0, s>>>(
+    k_slot_positions<<<slot_blocks(n_used), kSlotThreads, 0, s>>>(
         make_slotgeom(g), start, d_idx_b_r, d_xp, n_used, g.p.ratio_cs, d_pos, err);
     C2_HIP(hipGetLastError());
     int* h = g_dr.h_red.as<int>();

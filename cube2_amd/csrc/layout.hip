@@ -86,20 +86,17 @@ __device__ inline int ext_global(int64_t q, int nt, int ncb, int nte, int nnt, i
 }
 
 __global__ void k_layout_rhoc(const int* __restrict__ gstart, int64_t ncells, int nt, int ncb,
-                              int nte, int nnt, int nc, int* __restrict__ rhoc,
-                              int* __restrict__ slot) {
+                              int nte, int nnt, int nc, int* __restrict__ rhoc) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= ncells) return;
     const int g = ext_global(q, nt, ncb, nte, nnt, nc);
-    const int c = gstart[g + 1] - gstart[g];
-    rhoc[q] = c;
-    slot[q] = c;  // scanned into slot starts
+    rhoc[q] = gstart[g + 1] - gstart[g];
 }
 
-__global__ void k_layout_rows(const int* __restrict__ slot, int64_t nrows, int nte,
+__global__ void k_layout_rows(const long long* __restrict__ slot, int64_t nrows, int nte,
                               int64_t* __restrict__ idx_b_r) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nrows) idx_b_r[r] = (int64_t)slot[(r + 1) * nte];  // exclusive start of the next row
+    if (r < nrows) idx_b_r[r] = slot[(r + 1) * nte];  // exclusive start of the next row
 }
 
 // Codes and velocities in sorted (cell) order, so that the fill below copies
@@ -122,11 +119,11 @@ __global__ void k_layout_gather(const uint32_t* __restrict__ src, int64_t n,
 // 256^3 in 0.85 ms, and 0.25 ms for the gather before it; a wavefront per
 // cell that gathered every copy took 5.6 ms.
 __global__ __launch_bounds__(kSlotThreads) void k_layout_fill(
-    SlotGeom G, const int* __restrict__ gstart, const int* __restrict__ slot, int total,
+    SlotGeom G, const int* __restrict__ gstart, const long long* __restrict__ slot, int64_t total,
     const int16_t* __restrict__ code_s, const float* __restrict__ vel_s, int16_t* __restrict__ xp,
     float* __restrict__ vp) {
     __shared__ int win[kSlotWin + 1];
-    const int v0 = (int)blockIdx.x * kSlotChunk;
+    const int64_t v0 = (int64_t)blockIdx.x * kSlotChunk;
     walk_slots(slot, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
@@ -136,7 +133,7 @@ __global__ __launch_bounds__(kSlotThreads) void k_layout_fill(
             const int nc = (int)G.nc.d;
             const int g = (image_coord(G, tz, c.k) * nc + image_coord(G, ty, c.j)) * nc +
                           image_coord(G, tx, c.i);
-            const int64_t p = (int64_t)gstart[g] + (v - s0), d = (int64_t)v0 + v;
+            const int64_t p = (int64_t)gstart[g] + (v - s0), d = v0 + v;
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 xp[3 * d + k] = code_s[3 * p + k];
@@ -174,7 +171,7 @@ int layout_build(const double* d_pos, const float* d_vel, int64_t n, int* d_rhoc
     C2_TRY(g_lay.code_sorted.reserve(nn * 6));
     C2_TRY(g_lay.vel_sorted.reserve(nn * 12));
     C2_TRY(g_lay.cnt.reserve((nbin + 1) * sizeof(int)));
-    C2_TRY(g_lay.slot.reserve((ncells + 1) * sizeof(int)));
+    C2_TRY(g_lay.slot.reserve((ncells + 1) * sizeof(long long)));
     C2_TRY(g_lay.scan_tmp.reserve(scan_tmp_ints(std::max(nbin, ncells)) * sizeof(int)));
     int end_bit = 1;
     while (((int64_t)1 << end_bit) < nbin) end_bit++;
@@ -195,29 +192,29 @@ int layout_build(const double* d_pos, const float* d_vel, int64_t n, int* d_rhoc
                                     end_bit, g_lay.sort_tmp, g_lay.scan_tmp, s));
     }
     int* cnt = g_lay.cnt.as<int>();
-    int* slot = g_lay.slot.as<int>();
+    long long* slot = g_lay.slot.as<long long>();
     {
         Stage st("layout_cells", (double)n * 8 + (double)ncells * 16);
         k_layout_starts<<<ceil_div(nbin + 1, 256), 256, 0, s>>>(g_lay.gid_sorted.as<uint32_t>(), n,
                                                                 nbin, cnt);  // total at [nbin]
         C2_HIP(hipGetLastError());
         k_layout_rhoc<<<ceil_div(ncells, 256), 256, 0, s>>>(cnt, ncells, g.nt, g.ncb, g.nte,
-                                                            g.p.nnt, g.nc, d_rhoc, slot);
+                                                            g.p.nnt, g.nc, d_rhoc);
         C2_HIP(hipGetLastError());
-        C2_TRY(exclusive_scan(slot, ncells, g_lay.scan_tmp, s));
+        C2_TRY(exclusive_scan_counts(d_rhoc, slot, ncells, g_lay.scan_tmp, s));
         k_layout_rows<<<ceil_div(nrows, 256), 256, 0, s>>>(slot, nrows, g.nte, d_idx_b_r);
         C2_HIP(hipGetLastError());
     }
-    int total = 0;
-    C2_HIP(hipMemcpyAsync(&total, slot + ncells, sizeof(int), hipMemcpyDeviceToHost, s));
+    long long total = 0;
+    C2_HIP(hipMemcpyAsync(&total, slot + ncells, sizeof(total), hipMemcpyDeviceToHost, s));
     C2_HIP(hipStreamSynchronize(s));
     *n_used = total;
-    if (total < 0) {
+    if (total >= (1ll << 31)) {
         set_error("layout: more than 2^31 particle slots");
         return CUBE2_ERR_CAPACITY;
     }
     if (total > cap || !d_xp || !d_vp) {
-        set_error("layout: %d slots needed, capacity %lld", total, (long long)cap);
+        set_error("layout: %lld slots needed, capacity %lld", total, (long long)cap);
         return CUBE2_ERR_CAPACITY;
     }
     {
@@ -242,23 +239,22 @@ int layout_build(const double* d_pos, const float* d_vel, int64_t n, int* d_rhoc
 // :23-345): the velocities of every halo cell's slots from the periodic
 // source cell's slots, which hold the same particles in the same order.  A
 // block per kSlotChunk slots; those of physical cells are left alone.  90 M
-// slots at 256^3: 0.75 ms (a wavefront per cell: 4.25 ms).
+// slots at 256^3: 0.71 ms (a wavefront per cell: 4.25 ms).
 // err: 1 a halo cell and its source differ, or slots outside [0, n_used).
-__global__ __launch_bounds__(kSlotThreads) void k_halo_vp(SlotGeom G,
-                                                          const int* __restrict__ start,
+__global__ __launch_bounds__(kSlotThreads) void k_halo_vp(SlotGeom G, const int* __restrict__ rhoc,
+                                                          const long long* __restrict__ start,
                                                           const int64_t* __restrict__ idx_b_r,
                                                           float* __restrict__ vp, int64_t n_used,
                                                           int* __restrict__ err) {
     __shared__ int win[kSlotWin + 1];
-    const int total = start[G.ncells];
-    if (total < 0 || total > n_used) {
+    const int64_t total = start[G.ncells];
+    if (total > n_used) {
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1);
         return;
     }
-    const int v0 = (int)blockIdx.x * kSlotChunk;
     const int nte = (int)G.nte.d;
     int bad = 0;
-    walk_slots(start, G.ncells, v0, block_slots(total, v0), win, [&](int b, int e, auto cell_of) {
+    walk_all_slots(start, G.ncells, total, win, [&](int64_t v0, int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));
@@ -278,15 +274,16 @@ __global__ __launch_bounds__(kSlotThreads) void k_halo_vp(SlotGeom G,
             }
             const uint32_t ts = (uint32_t)((st[2] * (int)G.nnt.d + st[1]) * (int)G.nnt.d + st[0]);
             const uint32_t rs = (ts * nte + sc[2]) * nte + sc[1], qs = rs * nte + sc[0];
-            const int u0 = start[qs], u1 = start[qs + 1];
+            const int64_t u0 = start[qs];
+            const int64_t np = s1 < INT_MAX ? (int64_t)s1 - s0 : rhoc[c.row * nte + c.i];
             const int64_t h0 = row_shift(start, idx_b_r, c.row, nte) + v0;
             const int64_t h1 = row_shift(start, idx_b_r, rs, nte);
-            if (v < s0 || v >= s1 || u1 - u0 != s1 - s0 || s0 + h0 < 0 || u0 + h1 < 0 || s1 + h0 > n_used ||
-                u1 + h1 > n_used) {
+            const int64_t d0 = v + h0, d1 = u0 + (v - s0) + h1;
+            if (start[qs + 1] - u0 != np || d0 < 0 || d1 < 0 || d0 >= n_used ||
+                d1 >= n_used) {
                 bad = 1;
                 continue;
             }
-            const int64_t d0 = v + h0, d1 = u0 + (v - s0) + h1;
             const float a0 = vp[3 * d1], a1 = vp[3 * d1 + 1], a2 = vp[3 * d1 + 2];
             vp[3 * d0] = a0;
             vp[3 * d0 + 1] = a1;
@@ -310,17 +307,17 @@ int halo_velocities(const int* d_rhoc, const int64_t* d_idx_b_r, float* d_vp, in
     int* err = g_lay.red.as<int>();
     C2_TRY(fill_zero(err, sizeof(int), s));
     const int64_t ncells = (int64_t)g.ntile * g.nte * g.nte * g.nte;
-    if (n_used >= ((int64_t)1 << 31) - kSlotChunk || ncells >= ((int64_t)1 << 31)) {
-        set_error("halo velocities: more than 2^31 particle slots or cells");
+    if (ncells >= ((int64_t)1 << 31)) {
+        set_error("halo velocities: more than 2^31 cells");
         return CUBE2_ERR_CAPACITY;
     }
-    C2_TRY(g_lay.slot.reserve((ncells + 1) * sizeof(int)));
+    C2_TRY(g_lay.slot.reserve((ncells + 1) * sizeof(long long)));
     {
         Stage st("halo_vp", (double)n_used * 24);
-        int* start = g_lay.slot.as<int>();
+        long long* start = g_lay.slot.as<long long>();
         C2_TRY(exclusive_scan_counts(d_rhoc, start, ncells, g_lay.scan_tmp, s));
-        k_halo_vp<<<ceil_div((size_t)std::max<int64_t>(n_used, 1), kSlotChunk), kSlotThreads, 0, s>>>(
-            make_slotgeom(g), start, d_idx_b_r, d_vp, n_used, err);
+        k_halo_vp<<<slot_blocks(n_used), kSlotThreads, 0, s>>>(
+            make_slotgeom(g), d_rhoc, start, d_idx_b_r, d_vp, n_used, err);
         C2_HIP(hipGetLastError());
     }
     int h = 0;

@@ -1,5 +1,6 @@
-// Device-wide exclusive prefix sum of int32 counts (cell lists).
-#include <climits>
+// Device-wide exclusive prefix sum of int32 counts (cell lists), in 32 or 64
+// bits.
+#include <limits>
 
 #include "common.h"
 #include "scan.h"
@@ -10,27 +11,29 @@ constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
-__device__ inline int wave_inclusive_scan(int x) {
+template <class T>
+__device__ inline T wave_inclusive_scan(T x) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
+        T y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
     return x;
 }
 
 // Block-wide exclusive scan of one value per thread; returns the block total.
-__device__ inline int block_exclusive_scan(int v, int* total) {
-    __shared__ int wsum[kScanThreads / 64];
+template <class T>
+__device__ inline T block_exclusive_scan(T v, T* total) {
+    __shared__ T wsum[kScanThreads / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int inc = wave_inclusive_scan(v);
+    T inc = wave_inclusive_scan(v);
     if (lane == 63) wsum[wave] = inc;
     __syncthreads();
-    int off = 0, tot = 0;
+    T off = 0, tot = 0;
 #pragma unroll
     for (int w = 0; w < kScanThreads / 64; w++) {
-        int s = wsum[w];
+        T s = wsum[w];
         if (w < wave) off += s;
         tot += s;
     }
@@ -39,15 +42,17 @@ __device__ inline int block_exclusive_scan(int v, int* total) {
     return off + inc - v;
 }
 
-// lo: values below it count as lo (0 for counts from a caller, INT_MIN for none)
-__global__ __launch_bounds__(kScanThreads) void k_block_sums(const int* __restrict__ d, int64_t n,
-                                                             int lo, int* __restrict__ sums) {
+// lo: values below it count as lo (0 for counts from a caller, the type's lowest
+// for none)
+template <class S, class T>
+__global__ __launch_bounds__(kScanThreads) void k_block_sums(const S* __restrict__ d, int64_t n,
+                                                             S lo, T* __restrict__ sums) {
     int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    int s = 0;
+    T s = 0;
 #pragma unroll
     for (int q = 0; q < kScanItems; q++)
         if (base + q < n) s += max(d[base + q], lo);
-    int tot;
+    T tot;
     (void)block_exclusive_scan(s, &tot);
     if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
@@ -55,20 +60,21 @@ __global__ __launch_bounds__(kScanThreads) void k_block_sums(const int* __restri
 // Exclusive scan of each tile of src into d (may be src), offset by
 // offs[blockIdx.x] (nullptr: 0); writes the grand total to d[n] from the last
 // block.
-__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const int* src, int* d, int64_t n,
-                                                             int lo, const int* __restrict__ offs) {
+template <class S, class T>
+__global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const S* src, T* d, int64_t n, S lo,
+                                                             const T* __restrict__ offs) {
     int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    int v[kScanItems];
-    int s = 0;
+    T v[kScanItems];
+    T s = 0;
 #pragma unroll
     for (int q = 0; q < kScanItems; q++) {
         v[q] = base + q < n ? max(src[base + q], lo) : 0;
         s += v[q];
     }
-    int tot;
-    int pre = block_exclusive_scan(s, &tot);
-    int o = offs ? offs[blockIdx.x] : 0;
-    int run = o + pre;
+    T tot;
+    T excl = block_exclusive_scan(s, &tot);
+    const T o = offs ? offs[blockIdx.x] : 0;
+    T run = o + excl;
 #pragma unroll
     for (int q = 0; q < kScanItems; q++) {
         if (base + q < n) d[base + q] = run;
@@ -81,22 +87,23 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_tiles(const int* src, int
 // of about 6 us instead of three of 3 to 4 us each and the gaps between them
 // (a kick of 3600 particles has two such scans).
 constexpr int64_t kScanOneMax = 32768;
-__global__ __launch_bounds__(1024) void k_scan_one(const int* src, int* d, int n, int lo) {
-    __shared__ int wsum[1024 / 64];
+template <class S, class T>
+__global__ __launch_bounds__(1024) void k_scan_one(const S* src, T* d, int n, S lo) {
+    __shared__ T wsum[1024 / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int carry = 0;
+    T carry = 0;
     for (int b = 0; b < n; b += 1024 * kScanItems) {
         const int base = b + (int)threadIdx.x * kScanItems;
-        int v[kScanItems], s = 0;
+        T v[kScanItems], s = 0;
 #pragma unroll
         for (int q = 0; q < kScanItems; q++) {
             v[q] = base + q < n ? max(src[base + q], lo) : 0;
             s += v[q];
         }
-        const int inc = wave_inclusive_scan(s);
+        const T inc = wave_inclusive_scan(s);
         if (lane == 63) wsum[wave] = inc;
         __syncthreads();
-        int run = carry + inc - s;
+        T run = carry + inc - s;
 #pragma unroll
         for (int w = 0; w < 1024 / 64; w++) {
             run += w < wave ? wsum[w] : 0;
@@ -112,23 +119,24 @@ __global__ __launch_bounds__(1024) void k_scan_one(const int* src, int* d, int n
     if (threadIdx.x == 0) d[n] = carry;
 }
 
-static int scan_rec(const int* src, int* d, int64_t n, int lo, int* tmp, hipStream_t s) {
+template <class S, class T>
+static int scan_rec(const S* src, T* d, int64_t n, S lo, T* tmp, hipStream_t s) {
     const int64_t nb = (n + kScanTile - 1) / kScanTile;
     if (nb <= 1) {
-        k_scan_tiles<<<1, kScanThreads, 0, s>>>(src, d, n, lo, nullptr);
+        k_scan_tiles<S, T><<<1, kScanThreads, 0, s>>>(src, d, n, lo, nullptr);
         C2_HIP(hipGetLastError());
         return CUBE2_OK;
     }
     if (n <= kScanOneMax) {
-        k_scan_one<<<1, 1024, 0, s>>>(src, d, (int)n, lo);
+        k_scan_one<S, T><<<1, 1024, 0, s>>>(src, d, (int)n, lo);
         C2_HIP(hipGetLastError());
         return CUBE2_OK;
     }
-    int* sums = tmp;
-    k_block_sums<<<(unsigned)nb, kScanThreads, 0, s>>>(src, n, lo, sums);
+    T* sums = tmp;
+    k_block_sums<S, T><<<(unsigned)nb, kScanThreads, 0, s>>>(src, n, lo, sums);
     C2_HIP(hipGetLastError());
-    C2_TRY(scan_rec(sums, sums, nb, INT_MIN, tmp + nb + 1, s));
-    k_scan_tiles<<<(unsigned)nb, kScanThreads, 0, s>>>(src, d, n, lo, sums);
+    C2_TRY((scan_rec<T, T>(sums, sums, nb, std::numeric_limits<T>::lowest(), tmp + nb + 1, s)));
+    k_scan_tiles<S, T><<<(unsigned)nb, kScanThreads, 0, s>>>(src, d, n, lo, sums);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }
@@ -161,13 +169,13 @@ int fill_zero(void* d, size_t bytes, hipStream_t s) {
 int exclusive_scan(int* d, int64_t n, DevBuf& tmp, hipStream_t s) {
     if (n <= 0) return fill_zero(d, sizeof(int), s);
     C2_TRY(tmp.reserve(scan_tmp_ints(n) * sizeof(int)));
-    return scan_rec(d, d, n, INT_MIN, tmp.as<int>(), s);
+    return scan_rec<int, int>(d, d, n, std::numeric_limits<int>::lowest(), tmp.as<int>(), s);
 }
 
-int exclusive_scan_counts(const int* counts, int* d, int64_t n, DevBuf& tmp, hipStream_t s) {
-    if (n <= 0) return fill_zero(d, sizeof(int), s);
-    C2_TRY(tmp.reserve(scan_tmp_ints(n) * sizeof(int)));
-    return scan_rec(counts, d, n, 0, tmp.as<int>(), s);
+int exclusive_scan_counts(const int* counts, long long* d, int64_t n, DevBuf& tmp, hipStream_t s) {
+    if (n <= 0) return fill_zero(d, sizeof(long long), s);
+    C2_TRY(tmp.reserve(scan_tmp_ints(n) * sizeof(long long)));
+    return scan_rec<int, long long>(counts, d, n, 0, tmp.as<long long>(), s);
 }
 
 }  // namespace cube2

@@ -7,13 +7,16 @@
 // the kernel).  Instead a block takes a fixed number of consecutive slots
 // and finds the cells they lie in from the exclusive scan of the cell counts.
 #pragma once
+#include <algorithm>
+#include <climits>
+
 #include "common.h"
 
 namespace cube2 {
 
 constexpr int kSlotThreads = 256;
 constexpr int kSlotChunk = 1024;  // slots a block takes at a time
-constexpr int kSlotWin = 1024;    // cell starts staged in LDS at a time
+constexpr int kSlotWin = 1024;    // cell starts staged in LDS at a time, at most
 
 // n / d for n < 2^31 by a multiply (Granlund and Montgomery's round-up
 // method: m = floor(2^32 (2^l - d) / d) + 1, l = ceil(log2 d)).
@@ -81,7 +84,7 @@ __device__ inline int image_coord(const SlotGeom& G, int tile_c, int c) {
 // Block-wide: the last q in [0, n) with start[q] <= v, for start ascending
 // with start[0] <= v (the cell that holds v, empty cells before it skipped):
 // 256 probes a round.
-__device__ inline uint32_t block_last_le(const int* __restrict__ start, uint32_t n, int v) {
+__device__ inline uint32_t block_last_le(const long long* __restrict__ start, uint32_t n, int64_t v) {
     uint32_t lo = 0, hi = n;
     while (hi - lo > 1) {
         const uint32_t step = (hi - lo + kSlotThreads - 1) / kSlotThreads;
@@ -96,16 +99,21 @@ __device__ inline uint32_t block_last_le(const int* __restrict__ start, uint32_t
 // Block-wide walk of the n <= kSlotChunk slots from v0 on of the running slot
 // count `start` [ncells + 1] (win: kSlotWin + 1 ints of LDS).  For each window
 // of cells, body(begin, end, cell_of) with the slots [begin, end) it covers,
-// counted from v0 (the last block's v0 + kSlotChunk may pass 2^31); cell_of(v,
-// s0, s1) gives slot v's cell and the cell's slot range, counted alike (a range
-// may begin before v0).  body is called block-uniformly and may synchronise.
+// counted from v0 in 32 bits (an image may have 2^31 slots and more);
+// cell_of(v, s0, s1) gives slot v's cell and the cell's slot range, counted
+// alike: a range may begin before v0 (by less than 2^31, the largest count),
+// and one that ends 2^31 or more past v0 is cut there.  body is called
+// block-uniformly and may synchronise.
 template <class Body>
-__device__ inline void walk_slots(const int* __restrict__ start, uint32_t ncells, int v0, int n,
-                                  int* win, Body&& body) {
+__device__ inline void walk_slots(const long long* __restrict__ start, uint32_t ncells, int64_t v0,
+                                  int n, int* win, Body&& body) {
     for (int v = 0; v < n;) {
         const uint32_t q0 = block_last_le(start, ncells, v0 + v);
-        const int nw = (int)min((uint32_t)kSlotWin, ncells - q0);
-        for (int a = threadIdx.x; a <= nw; a += kSlotThreads) win[a] = start[q0 + a] - v0;
+        // (as few as reach the end, where a cell holds several slots)
+        int nw = (int)min((uint32_t)kSlotThreads, ncells - q0);
+        if (start[q0 + nw] < v0 + n) nw = (int)min((uint32_t)kSlotWin, ncells - q0);
+        for (int a = threadIdx.x; a <= nw; a += kSlotThreads)
+            win[a] = (int)min(start[q0 + a] - (long long)v0, (long long)INT_MAX);
         __syncthreads();
         const int end = min(n, max(win[nw], v + 1));
         body(v, end, [&](int s, int& s0, int& s1) {
@@ -124,16 +132,33 @@ __device__ inline void walk_slots(const int* __restrict__ start, uint32_t ncells
     }
 }
 
-// Slots of the block at v0 of `total`.
-__device__ inline int block_slots(int total, int v0) { return min(kSlotChunk, max(total - v0, 0)); }
+// Blocks of walk_all_slots over about n slots.
+inline unsigned slot_blocks(int64_t n) {
+    return std::min(ceil_div((size_t)std::max<int64_t>(n, 1), kSlotChunk), 1u << 20);
+}
+
+// Slots of the chunk at v0 of `total`.
+__device__ inline int block_slots(int64_t total, int64_t v0) {
+    return (int)min((long long)kSlotChunk, max((long long)(total - v0), 0ll));
+}
+
+// walk_slots over all `total` slots: body(v0, begin, end, cell_of) with slots
+// counted from v0.
+template <class Body>
+__device__ inline void walk_all_slots(const long long* __restrict__ start, uint32_t ncells,
+                                      int64_t total, int* win, Body&& body) {
+    for (int64_t v0 = (int64_t)blockIdx.x * kSlotChunk; v0 < total; v0 += (int64_t)gridDim.x * kSlotChunk)
+        walk_slots(start, ncells, v0, block_slots(total, v0), win,
+                   [&](int b, int e, auto cell_of) { body(v0, b, e, cell_of); });
+}
 
 // Running slot counts of the cells (scan.hip: negative counts as 0) and,
 // per row, what to add to a running count to get a slot: idx_b_r of the row
 // less the running count at its end (0 where idx_b_r is the running total,
 // as spine_image leaves it).
-__device__ inline int64_t row_shift(const int* __restrict__ start, const int64_t* __restrict__ idx_b_r,
+__device__ inline int64_t row_shift(const long long* __restrict__ start, const int64_t* __restrict__ idx_b_r,
                                     uint32_t row, uint32_t nte) {
-    return idx_b_r[row] - (int64_t)start[(size_t)(row + 1) * nte];
+    return idx_b_r[row] - start[(size_t)(row + 1) * nte];
 }
 
 }  // namespace cube2

@@ -98,7 +98,7 @@ def build_layout_device(pos, vel, geom: Geometry):
         rc = _lib.lib().cube2_layout_build_dev(
             d_pos.data_ptr(), None if d_vel is None else d_vel.data_ptr(), n, rhoc.data_ptr(),
             idx.data_ptr(), xp.data_ptr(), vp.data_ptr(), m, C.byref(n_used))
-        if rc != _lib.ERR_CAPACITY or n_used.value <= m:
+        if rc != _lib.ERR_CAPACITY or not m < n_used.value < 2 ** 31:
             break
         m = n_used.value
     _lib.check(rc)
