@@ -180,13 +180,9 @@ __global__ __launch_bounds__(kSlotThreads) void k_slot_positions(
     const int16_t* __restrict__ xp, int64_t n_used, int ratio_cs, double* __restrict__ pos,
     unsigned* __restrict__ err) {
     __shared__ int win[kSlotWin + 1];
-    const int64_t total = start[G.ncells];
-    if (total > n_used) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, 1u);
-        return;
-    }
     unsigned bad = 0;
-    walk_all_slots(start, G.ncells, total, win, [&](int64_t v0, int b, int e, auto cell_of) {
+    // (more than n_used slots where rows share theirs)
+    walk_all_slots(start, G.ncells, start[G.ncells], win, [&](int64_t v0, int b, int e, auto cell_of) {
         for (int v = b + (int)threadIdx.x; v < e; v += kSlotThreads) {
             int s0, s1;
             const CellPos c = cell_pos(G, cell_of(v, s0, s1));

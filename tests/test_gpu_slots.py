@@ -94,3 +94,36 @@ def test_rows_that_start_past_gaps():
     cell = np.floor(lay.decoded_positions() / g.ratio_cs)
     frac = (lay.xp.view(np.uint16).astype(np.float64) + 0.5) / 65536.0
     assert np.array_equal(pos, (np.mod(cell, g.nc) + frac) * g.ratio_cs)
+
+
+def test_rows_that_share_their_slots():
+    """The halo rows of one periodic tile hold what its physical rows hold, so
+    idx_b_r may name the same slots for both: positions and halo velocities of
+    an image without the halo rows' copies."""
+    import torch
+    from cube2_amd.drift import refresh_halo_velocities, slot_positions_device
+    from cube2_amd.geometry import Geometry
+    from cube2_amd.layout import build_layout
+    g = Geometry(ng=32, nnt=1, nns=1, ratio_cs=4, ngb=8, app=0.05)
+    rng = np.random.default_rng(23)
+    lay = build_layout(rng.uniform(0, 32, (2500, 3)), rng.normal(0, 1, (2500, 3)).astype(np.float32), g)
+    rows = lay.rhoc[0].sum(2).astype(np.int64)                   # [k][j]
+    src = (np.arange(g.nte) - g.ncb) % g.nt + g.ncb              # a row's physical twin
+    phys = np.zeros_like(rows, bool)
+    phys[g.ncb:g.ncb + g.nt, g.ncb:g.ncb + g.nt] = True
+    end = np.where(phys, rows, 0).reshape(-1).cumsum().reshape(rows.shape)[src][:, src]
+    full = lay.idx_b_r[0] - rows                                 # a row's first slot in the whole layout
+    of = np.concatenate([np.arange(full[k, j], full[k, j] + rows[k, j])
+                         for k, j in np.argwhere(phys)])         # its slots, kept once
+    n = of.size
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    rhoc, idx, xp = d(lay.rhoc), d(end[None]), d(lay.xp[of])
+    assert n < lay.n_used and int(idx.max()) == n
+    own = lay.physical_mask()[of]
+    vp = d(np.where(own[:, None], lay.vp[of], np.float32(7)))
+    refresh_halo_velocities(rhoc, idx, vp, n, g)
+    assert np.array_equal(vp.cpu().numpy(), lay.vp[of])
+    pos = slot_positions_device(rhoc, idx, xp, n, g).cpu().numpy()
+    cell = np.floor(lay.decoded_positions() / g.ratio_cs)
+    frac = (lay.xp.view(np.uint16).astype(np.float64) + 0.5) / 65536.0
+    assert np.array_equal(pos, ((np.mod(cell, g.nc) + frac) * g.ratio_cs)[of])
