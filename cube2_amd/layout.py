@@ -90,11 +90,18 @@ def build_layout_device(pos, vel, geom: Geometry):
     n_used = C.c_int64(0)
     # one call where the slots fit an eighth over the mean density's (the
     # sort and the cell counts run once); a second, sized by the first, where
-    # clumps in the halos need more
+    # clumps in the halos need more or there is no memory for the guess
     m = n * geom.nte ** 3 // geom.nt ** 3 * 9 // 8 + 4096
-    for _ in range(2):
-        xp = torch.empty((m, 3), dtype=torch.int16, device=dev)
-        vp = torch.empty((m, 3), dtype=torch.float32, device=dev)
+    for attempt in range(2):
+        xp = vp = None
+        try:
+            xp = torch.empty((m, 3), dtype=torch.int16, device=dev)
+            vp = torch.empty((m, 3), dtype=torch.float32, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            if attempt:
+                raise
+            m = 0
+            xp, vp = torch.empty(0, device=dev), torch.empty(0, device=dev)
         rc = _lib.lib().cube2_layout_build_dev(
             d_pos.data_ptr(), None if d_vel is None else d_vel.data_ptr(), n, rhoc.data_ptr(),
             idx.data_ptr(), xp.data_ptr(), vp.data_ptr(), m, C.byref(n_used))

@@ -57,3 +57,32 @@ def test_layout_empty(lib):
     from cube2_amd.geometry import Geometry
     g = Geometry(ng=64, nnt=2, nns=2, ratio_cs=4, ngb=8, app=0.05)
     assert _compare(np.zeros((0, 3)), None, g) == 0
+
+
+def test_layout_that_fits_only_its_own_size():
+    """Where there is memory for the slots there are, but not for those that the
+    mean density would have, the layout is built all the same: the particles of
+    one cell that the tiles hold 8 times, 16 times on average."""
+    import torch
+    from cube2_amd.geometry import Geometry
+    from cube2_amd.layout import build_layout_device
+    g = Geometry(ng=64, nnt=2, nns=1, ratio_cs=4, ngb=24, app=0.05)
+    n = 1 << 20
+    copies = [sum(((t * g.nt + e - g.ncb) % g.nc) == c for t in range(g.nnt) for e in range(g.nte))
+              for c in range(g.nc)]
+    c = int(np.argmin(copies))
+    slots = n * copies[c] ** 3
+    guess = n * g.nte ** 3 // g.nt ** 3
+    assert copies[c] == 2 and guess > 15 * n
+    pos = torch.full((n, 3), (c + 0.5) * g.ratio_cs, dtype=torch.float64, device="cuda")
+    torch.cuda.empty_cache()
+    limit = torch.cuda.memory_reserved() + slots * 18 + (64 << 20)
+    assert torch.cuda.memory_reserved() + guess * 18 > limit
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        rhoc, idx, xp, vp, k = build_layout_device(pos, None, g)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert k == slots == xp.shape[0] and int(rhoc.sum()) == slots
+    code = np.array(g.ratio_cs // 2 * 65536 // g.ratio_cs).astype(np.uint16).view(np.int16)
+    assert int(xp.min()) == int(xp.max()) == int(code) and float(vp.abs().max()) == 0.0
