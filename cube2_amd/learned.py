@@ -145,6 +145,17 @@ class LearnedPP:
     def step(self, grads, lr: float = 1e-3, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8):
         L = _lib.lib()
         self.t += 1
+        if len(grads) != 4:  # some layers' gradients move those layers
+            for l, (dW, db) in enumerate(grads):
+                dW, db = dW.contiguous(), db.contiguous()
+                _lib.check(L.cube2_cnn_adam_dev(_p(self.W[l]), _p(dW), _p(self.mW[l]),
+                                                _p(self.vW[l]), _p(self.Wb[l]), self.W[l].numel(),
+                                                lr, b1, b2, eps, self.t))
+                _lib.check(L.cube2_cnn_adam_dev(_p(self.b[l]), _p(db), _p(self.mb[l]),
+                                                _p(self.vb[l]), None, self.b[l].numel(),
+                                                lr, b1, b2, eps, self.t))
+            self._refresh(bf16=False)
+            return
         gs = [dW.contiguous() for dW, _ in grads] + [db.contiguous() for _, db in grads]
         _lib.check(L.cube2_cnn_net_adam_dev(_ps(self.W + self.b), _ps(gs), _ps(self.mW + self.mb),
                                             _ps(self.vW + self.vb), _ps(self.Wb), _ps(self.Wp),
