@@ -128,7 +128,9 @@ __global__ __launch_bounds__(kDwThreads) void k_bwd_dw(const float* __restrict__
                     // row r16 = (dx, c), dx = 3 repeats 2, unused
                     const int ch = CIN == 32 ? (a >> 1) * CIN + (a & 1) * 16 + r16
                                              : min(r16 >> 2, 2) * CIN + (r16 & 3);
-                    const v8bf am = xt[ch * RX + row];
+                    v8bf am = xt[ch * RX + row];
+                    // (a row past the outputs: dY is zero, an infinite X times it is not)
+                    if (g * 4 + 4 > P && g * 4 + kq >= P) am = v8bf{};
 #pragma unroll
                     for (int o = 0; o < S::kOT; o++)
                         acc[a][o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm[o], acc[a][o], 0, 0, 0);
@@ -168,11 +170,45 @@ __global__ __launch_bounds__(kDwThreads) void k_bwd_dw(const float* __restrict__
 // a sum would flip roundings).  Rows of LDS are padded by 8 bytes (conflict-
 // free 8-byte reads).  Bound by the dependent MFMA and add chain of a tap.
 template <int COUT>
+struct DxShape {
+    static constexpr int KP = COUT == 32 ? 32 : 16, KH = KP / 16, ST = KP + 4;  // (BF16 elements)
+};
+
+// A tile of 16 positions, its lane's p, tap by tap within the outputs.
+template <int COUT>
+__device__ inline void dx_tile_bounded(const uint16_t* wl, const uint16_t* yl, int p, int kq, int D,
+                                       float* __restrict__ dX) {
+    using S = DxShape<COUT>;
+    const int P = D - 2, E = P + 4, r16 = threadIdx.x & 15;
+    const int pc = min(p, D * D * D - 1), z = pc / (D * D), y = pc / D % D, x = pc % D;
+    v4f s[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+    for (int t = 0; t < 27; t++) {
+        const int oz = z - t / 9, oy = y - t / 3 % 3, ox = x - t % 3;
+        const bool in = (unsigned)oz < (unsigned)P && (unsigned)oy < (unsigned)P && (unsigned)ox < (unsigned)P;
+        const uint16_t* cell = yl + (((oz + 2) * E + oy + 2) * E + ox + 2) * S::ST + kq * 4;
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            v4f d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int h = 0; h < S::KH; h++)
+                d = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    *reinterpret_cast<const v4s*>(wl + (t * 32 + ct * 16 + r16) * S::ST + h * 16 + kq * 4),
+                    *reinterpret_cast<const v4s*>(cell + h * 16), d, 0, 0, 0);
+            if (in) s[ct] += d;
+        }
+    }
+    if (p >= D * D * D) return;
+#pragma unroll
+    for (int ct = 0; ct < 2; ct++) *reinterpret_cast<v4f*>(dX + (int64_t)p * 32 + 4 * kq + ct * 16) = s[ct];
+}
+
+template <int COUT>
 __global__ __launch_bounds__(kDxThreads) void k_bwd_dx(const float* __restrict__ Y,
                                                        const float* __restrict__ dY,
                                                        const uint16_t* __restrict__ Wb, int B,
                                                        int D, int relu, float* __restrict__ dX) {
-    constexpr int KP = COUT == 32 ? 32 : 16, KH = KP / 16, ST = KP + 4;  // (BF16 elements)
+    constexpr int KP = DxShape<COUT>::KP, KH = DxShape<COUT>::KH, ST = DxShape<COUT>::ST;
     extern __shared__ __align__(16) uint16_t dx_lds[];
     uint16_t* wl = dx_lds;                // [27 * 32][ST]
     uint16_t* yl = dx_lds + 27 * 32 * ST;  // [(P + 4)^3][ST]
@@ -231,6 +267,20 @@ __global__ __launch_bounds__(kDxThreads) void k_bwd_dx(const float* __restrict__
                         }
                     }
                 }
+            }
+            // A zero of the border times an infinite weight is no zero: where a sum
+            // is not finite, the tiles again with each tap only where it reaches an
+            // output.
+            float any = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int k = 0; k < 8; k++) any += s[q][k >> 2][k & 3];
+            if (__ballot(!(fabsf(any) < INFINITY))) {
+#pragma unroll 1
+                for (int q = 0; q < 4; q++)
+                    dx_tile_bounded<COUT>(wl, yl, (t0 + q) * 16 + r16, kq, D, dX + (int64_t)b * D * D * D * 32);
+                continue;
             }
 #pragma unroll
             for (int q = 0; q < 4; q++) {

@@ -71,3 +71,48 @@ def test_larger_patches_are_refused_by_the_one_call_backward():
                                                ps(net.mW), ps(net.mb))
     assert rc == _lib.ERR_CAPACITY
     assert len(net.backward(dout)) == 4      # the general path
+
+
+@pytest.mark.parametrize("D,l", [(10, 1), (10, 3), (9, 0), (9, 1), (9, 2), (9, 3)])
+def test_patch_backward_keeps_infinities_where_they_belong(monkeypatch, D, l):
+    """An infinite activation in the last row of layer l's input reaches the
+    weight gradients of the taps that read it and no others, as with im2col:
+    the rows that pad the positions to fours are no terms of the sum."""
+    import torch
+    from cube2_amd import learned
+    net, x, dout = _net_and_input(3, D, 40 + l)
+    net.forward(x)
+    d = D - 2 * l
+    net.acts[l] = net.acts[l].clone()
+    net.acts[l][1, 1, d - 1, 2, 3] = float("inf")
+    got = net.backward(dout)
+    monkeypatch.setattr(learned, "PATCH", 0)
+    want = net.backward(dout)
+    for k, ((gw, gb), (ww, wb)) in enumerate(zip(got, want)):
+        for a, b in ((gw, ww), (gb, wb)):
+            ok = torch.isfinite(b)
+            assert torch.equal(torch.isfinite(a), ok), (k, int(ok.sum()), int(torch.isfinite(a).sum()))
+            assert float((a - b)[ok].double().norm()) <= 3e-5 * float(b[ok].double().norm())
+    assert not torch.isfinite(want[l][0]).all() and torch.isfinite(want[l][0]).any()
+
+
+@pytest.mark.parametrize("D,l", [(10, 3), (10, 1), (9, 2)])
+def test_patch_backward_keeps_infinite_weights_off_the_border(monkeypatch, D, l):
+    """An infinite weight of a tap that no output uses at the only position where
+    its input channel is active: the gradients stay finite, as with im2col."""
+    import torch
+    from cube2_amd import learned
+    net, x, dout = _net_and_input(3, D, 50 + l)
+    net.forward(x)
+    c, cout = 5, (4, 32, 32, 32, 3)[l + 1]
+    net.acts[l] = net.acts[l].clone()
+    net.acts[l][..., c] = 0.0
+    net.acts[l][:, -1, -1, -1, c] = 1.0
+    net.Wb[l].view(27, 32, cout)[0, c, 1] = 0x7f80  # (tap 0 reaches the inputs 0 .. P - 1 alone)
+    got = net.backward(dout)
+    monkeypatch.setattr(learned, "PATCH", 0)
+    want = net.backward(dout)
+    for k, ((gw, gb), (ww, wb)) in enumerate(zip(got, want)):
+        for a, b in ((gw, ww), (gb, wb)):
+            assert torch.isfinite(b).all() and torch.isfinite(a).all(), k
+            assert float((a - b).double().norm()) <= 3e-5 * float(b.double().norm())
