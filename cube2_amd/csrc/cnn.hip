@@ -246,7 +246,10 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ out,
 // 72^3 outputs divide by 8, training patches have 8^3, 6^3, 4^3 and 2^3.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+// The same in memory, at any address of their elements (one 16-byte access
+// wherever it begins): activations are a caller's, views among them.
+typedef v8bf v8bf_at __attribute__((aligned(2)));
+typedef float v4f_at __attribute__((ext_vector_type(4), aligned(4)));
 
 struct ConvTile {
     int tx;   // consecutive x of a tile (16, 8, 4); 16 / tx grids side by side
@@ -255,11 +258,11 @@ struct ConvTile {
 };
 
 // 16 bytes of BF16 channels from 8 values of the input.
-__device__ inline v8bf load_bf16x8(const uint16_t* p) { return *reinterpret_cast<const v8bf*>(p); }
+__device__ inline v8bf load_bf16x8(const uint16_t* p) { return *reinterpret_cast<const v8bf_at*>(p); }
 __device__ inline v8bf load_bf16x8(const float* p) {
-    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-    return v8bf{(__bf16)a.x, (__bf16)a.y, (__bf16)a.z, (__bf16)a.w,
-                (__bf16)b.x, (__bf16)b.y, (__bf16)b.z, (__bf16)b.w};
+    const v4f a = reinterpret_cast<const v4f_at*>(p)[0], b = reinterpret_cast<const v4f_at*>(p)[1];
+    return v8bf{(__bf16)a[0], (__bf16)a[1], (__bf16)a[2], (__bf16)a[3],
+                (__bf16)b[0], (__bf16)b[1], (__bf16)b[2], (__bf16)b[3]};
 }
 
 // The output channel in MFMA row r (0..15) of row tile ct.  BF16 outputs: a
@@ -271,13 +274,13 @@ __device__ inline int conv_channel(int ct, int r) {
 
 // Stores a lane's two result tiles at its position's channels.
 __device__ inline void store32(uint16_t* row, int kq, const v4f& u, const v4f& v) {
-    *reinterpret_cast<v8bf*>(row + 8 * kq) =
+    *reinterpret_cast<v8bf_at*>(row + 8 * kq) =
         v8bf{(__bf16)u[0], (__bf16)u[1], (__bf16)u[2], (__bf16)u[3],
              (__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
 }
 __device__ inline void store32(float* row, int kq, const v4f& u, const v4f& v) {
-    *reinterpret_cast<v4f*>(row + 4 * kq) = u;
-    *reinterpret_cast<v4f*>(row + 16 + 4 * kq) = v;
+    *reinterpret_cast<v4f_at*>(row + 4 * kq) = u;
+    *reinterpret_cast<v4f_at*>(row + 16 + 4 * kq) = v;
 }
 
 // 32 input channels.  A wavefront owns 4 rows of tiles (4 y of tx x) and
@@ -542,8 +545,8 @@ __global__ __launch_bounds__(256, 4) void k_conv3_c4(const float* __restrict__ X
         const int y0 = (int)(q % nyc) * kC4Rows;
         q /= nyc;
         const int gz = (int)(q % P), b0 = (int)(q / P) * ng;
-        const float4* Xi = reinterpret_cast<const float4*>(X) + ((int64_t)b0 * D + gz) * D * D;
-        float4 v[kC4Items];
+        const v4f_at* Xi = reinterpret_cast<const v4f_at*>(X) + ((int64_t)b0 * D + gz) * D * D;
+        v4f v[kC4Items];
 #pragma unroll
         for (int k = 0; k < kC4Items; k++) {
             const int dz = cell[k] >> 20, y = min(y0 + (cell[k] >> 16 & 15), D - 1),
@@ -553,7 +556,7 @@ __global__ __launch_bounds__(256, 4) void k_conv3_c4(const float* __restrict__ X
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int k = 0; k < kC4Items; k++)
-            xl[k * 64 + lane] = v4bf{(__bf16)v[k].x, (__bf16)v[k].y, (__bf16)v[k].z, (__bf16)v[k].w};
+            xl[k * 64 + lane] = v4bf{(__bf16)v[k][0], (__bf16)v[k][1], (__bf16)v[k][2], (__bf16)v[k][3]};
         __builtin_amdgcn_wave_barrier();
         const int gx = x0 + xs, gb = b0 + gi, ny = min(kC4Rows, P - y0);
         TOut* out = Y + ((((int64_t)gb * P + gz) * P + y0) * P + gx) * 32;
