@@ -401,6 +401,8 @@ __global__ __launch_bounds__(256) void k_pp_ptotal(const int* __restrict__ rhoc,
 // subtiles of range occ_range (the network's).  A pairs-once pass (newton)
 // marks both by a negative range (w = -range): to other i they are one-sided
 // sources; every reader of w then takes |w| as the range and w != 0 as active.
+// The marked ones' rpos, which nothing reads after this, is cleared: k_pp_sparse's
+// low words.
 // ntile > 0 (pairs once): flags[a] = the parts the chunk is split into, one
 // per `part` candidates j, but at most one per particle, so that the list
 // of all parts fits the capacity.
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(256) void k_pp_ptotal(const int* __restrict__ rhoc,
 // is a serial chain of its candidates (pair kernel with 2048, 256, 64 of them:
 // 3600 particles 95, 96, 57 us, 64^3 lattice 115, 114, 117).
 constexpr int kPartCand = 2048, kPartFew = 64, kPartCount = 16, kFewSlots = 1 << 20;
-__global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
+__global__ void k_chunk_flags(float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
                               const int* __restrict__ cell_start, const int* __restrict__ n_sorted,
                               const int* __restrict__ err, int cap, int dense_lg, int small, int occ,
@@ -436,7 +438,10 @@ __global__ void k_chunk_flags(const float4* __restrict__ rpos, const uint32_t* _
             if (dense && a == c0) dense_list[atomicAdd(ndense, 1)] = (int)c;
             if (cn <= small || (cn < occ && p.w == occ_range)) {
                 f = 0;
-                if (newton) p.w = -p.w;
+                if (newton) {
+                    p.w = -p.w;
+                    rpos[a] = make_float4(0.f, 0.f, 0.f, 0.f);
+                }
             }
             if (f && ntile && cn >= kPartCount) {
                 const PPTile T = tiles[pp_find_tile(tiles, ntile, c)];
@@ -960,8 +965,8 @@ __global__ void k_react_zero(unsigned long long* __restrict__ react, int* __rest
 // kernel's FP32 operation order, and f2max = max |a m^2|^2.
 __global__ __launch_bounds__(256) void k_pp_newton_terms(
     const float4* __restrict__ pos4, const uint32_t* __restrict__ slot,
-    const unsigned long long* __restrict__ react, const int* __restrict__ n_sorted, int cap,
-    const float* __restrict__ scal, double inv_scale, float net_range, float* __restrict__ term,
+    const unsigned long long* __restrict__ react, const int4* __restrict__ low,
+    const int* __restrict__ n_sorted, int cap, const float* __restrict__ scal, double inv_scale, float net_range, float* __restrict__ term,
     PPRed* red) {
 #pragma clang fp contract(off)
     float f2 = 0.0f;
@@ -970,10 +975,13 @@ __global__ __launch_bounds__(256) void k_pp_newton_terms(
     for (int a = blockIdx.x * blockDim.x + threadIdx.x; a < n; a += gridDim.x * blockDim.x) {
         const float w = pos4[a].w;
         if (w == 0.0f || w == -net_range) continue;  // halo sources; the network's (learned kick)
+        const int4 lo = w < 0.0f ? low[a] : make_int4(0, 0, 0, 0);
+        const int l[3] = {lo.x, lo.y, lo.z};
         float acc[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const float v = (float)((double)(long long)react[c * (size_t)cap + a] * inv_scale);
+            const double u = (double)(long long)react[c * (size_t)cap + a] + l[c] * (1.0 / kLowScale);
+            const float v = (float)(u * inv_scale);
             acc[c] = v * mass * mass;
         }
         f2 = fmaxf(f2, acc[0] * acc[0] + acc[1] * acc[1] + acc[2] * acc[2]);
@@ -1059,6 +1067,7 @@ static PPArgs pair_args(const PPPlan& P, float* d_vp, const float* d_scal, const
     if (P.newton) {
         A.term = g_pp.term.as<float>();
         A.react = g_pp.react.as<unsigned long long>();
+        A.low = g_pp.raw_pos4.as<int4>();
         A.react_scale = P.react_scale;
         A.order = pp_heavy_lg() ? g_pp.order.as<int>() : nullptr;
         A.taken = reinterpret_cast<int*>(A.react + P.cap * 3);
@@ -1069,7 +1078,7 @@ static PPArgs pair_args(const PPPlan& P, float* d_vp, const float* d_scal, const
 // Velocity terms of a pairs-once pass, once every chunk has added to react.
 static int newton_terms(const PPPlan& P, const PPArgs& A, hipStream_t s) {
     Stage st("pp_terms", (double)P.n_used * (16 + 24 + 4 + 12));
-    k_pp_newton_terms<<<std::min(ceil_div(P.cap, 1024), 4096u), 256, 0, s>>>(A.pos4, A.slot, A.react, A.n_sorted, (int)P.cap, A.scal,
+    k_pp_newton_terms<<<std::min(ceil_div(P.cap, 1024), 4096u), 256, 0, s>>>(A.pos4, A.slot, A.react, A.low, A.n_sorted, (int)P.cap, A.scal,
                                             1.0 / (double)P.react_scale, A.learned_range, A.term,
                                             A.red);
     C2_HIP(hipGetLastError());

@@ -78,11 +78,18 @@ struct PPArgs {
     // sums kept as signed 64-bit fixed point (value * react_scale) at
     // react[c * cap + sorted index]; k_pp_newton_terms turns them into term
     unsigned long long* react;
+    // the small cells' sums (k_pp_sparse): what is left of them, in units of
+    // 1 / (react_scale * kLowScale), x, y, z by sorted index
+    int4* low;
     const int* order;  // the parts in another order than the list's, or null
     int* taken;  // per run of the part list (kPartRuns, kRunPad apart): parts taken
     float react_scale;
     int ntt;  // coarse cells per subtile side
 };
+
+// (16 partial sums, each off by half a unit of react_scale at most, stay in 32
+// bits)
+constexpr double kLowScale = 1 << 24;
 
 int launch_pp_pairs(const PPArgs& a, int mode, hipStream_t s);
 

@@ -15,10 +15,13 @@
 // j's cell lies in i's stencil, for the count of candidates, is one packed
 // comparison of cell coordinates.  Accepted pairs are queued in LDS and their
 // forces evaluated 64 at a time, summed per i as 64-bit fixed point (integer
-// LDS atomics; float ones cost ~190 cycles an instruction on gfx950).  These
-// particles evaluate all their pairs themselves and nothing else adds to
-// them (k_chunk_flags marks them), so their sums are stored, not added, unless
-// their j are split.
+// LDS atomics; float ones cost ~190 cycles an instruction on gfx950) at a scale
+// for the 512 pairs of 8 such steps, and in FP64 over the steps: the pass's
+// scale, for as many pairs as there are slots, rounds each pair to 2^-12 where
+// the softening is small.  These particles evaluate all their pairs themselves
+// and nothing else adds to them (k_chunk_flags marks them), so their sums are
+// stored, not added, unless their j are split; what the pass's scale cannot hold
+// of them goes to `low`.
 // Bound by VALU issue: the region's tests.  The particles beside a clump cost
 // the most by far, one batch of them up to 1 ms, and the kernel waits for the
 // last: k_sparse_items shares a coarse cell among wavefronts and lists the
@@ -43,7 +46,7 @@ struct SparseLDS {
     float4 q[kQ];             // accepted pairs (dx, dy, dz, r^2)
     unsigned char qi[kQ];     // and their i slot
     unsigned long long acc[64][3];
-    float4 jb[128];           // a batch of j (w: packed cell), then far-away ones
+    float4 jb[64];            // a batch of j (w: packed cell), far-away ones past it
     int list[128];            // sorted indices of small cells' particles
     unsigned lcell[128];      // their cells (packed, in the coarse cell) and
     unsigned short lblk[128]; // blocks
@@ -66,9 +69,23 @@ __device__ inline void sparse_flush(SparseLDS& L, int lane, int begin, int count
     wave_lds_sync();
 }
 
+// The sums of the last steps, of the lane's i slot, into FP64.
+__device__ inline void sparse_drain(SparseLDS& L, int lane, double (&sum)[3], double inv_scale) {
+    wave_lds_sync();
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        sum[c] += (double)(long long)L.acc[lane][c] * inv_scale;
+        L.acc[lane][c] = 0ull;
+    }
+    wave_lds_sync();
+}
+
 // n / d as the high word of n * recip(d), exact for n d < 2^32.
 __device__ inline unsigned recip_u32(unsigned d) { return 0xffffffffu / d + 1u; }
 __device__ inline int quot(int n, unsigned recip) { return (int)__umulhi((unsigned)n, recip); }
+
+// Pairs between two drains (a multiple of 64).
+constexpr int kDrainPairs = 512;
 
 // Mean particles of a block (below): small blocks walk less that only one of
 // their particles needs, large ones read rows less often (at 256^3 with one
@@ -141,7 +158,8 @@ __global__ __launch_bounds__(256) void k_sparse_items(const int* __restrict__ rh
 
 template <int kMode>
 __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __restrict__ items, int cap,
-                                                      const int* __restrict__ count, int nt, int small) {
+                                                      const int* __restrict__ count, int nt, int small,
+                                                      float scale, double inv_scale) {
     __shared__ SparseLDS lds[4];
     const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     SparseLDS& L = lds[wave];
@@ -256,6 +274,7 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __re
             const float pix = vi ? p.x : -kFar, piy = vi ? p.y : -kFar, piz = vi ? p.z : -kFar;
             for (int q = lane; q < 64 * 3; q += 64) (&L.acc[0][0])[q] = 0ull;
             int qhead = 0, qtail = 0;
+            double sum[3] = {0.0, 0.0, 0.0};  // of i slot `lane`
             for (int rg = 0; rg < nrows; rg += 64) {
                 int js = 0, cnt = 0;
                 const int r = rg + lane;
@@ -297,10 +316,9 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __re
                 for (int vb = v0; vb < M; vb += 64) {
                     const int nb = min(64, M - vb);
                     qc.w = __uint_as_float(rc + jc);
-                    L.jb[lane] = qc;
-                    wave_lds_sync();
                     // past the batch: far away and in no stencil
-                    L.jb[nb + lane] = make_float4(kFar, kFar, kFar, __uint_as_float(511u * kOnes));
+                    if (lane >= nb) qc = make_float4(kFar, kFar, kFar, __uint_as_float(511u * kOnes));
+                    L.jb[lane] = qc;
                     wave_lds_sync();
                     if (vb + 64 < M) qc = fetch(vb + 64);
                     // lane's pair with the j at slot u: its vector, r^2, whether
@@ -326,11 +344,12 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __re
                         qtail += __popcll(m);
                         if (qtail - qhead >= 64) {
                             wave_lds_sync();
-                            sparse_flush<kMode>(L, lane, qhead, 64, Ka, Kr, A.react_scale);
+                            sparse_flush<kMode>(L, lane, qhead, 64, Ka, Kr, scale);
                             qhead += 64;
+                            if (qhead % kDrainPairs == 0) sparse_drain(L, lane, sum, inv_scale);
                         }
                     };
-                    if (J <= 16) {  // (4 J slots past the batch's last are set)
+                    if (J <= 16) {  // (4 J divides 64: no slot past them)
                         for (int u = 0; u < nb; u += 4 * J) {
                             float4 qj[4], e[4];
                             bool ok[4];
@@ -352,16 +371,28 @@ __global__ __launch_bounds__(256, 5) void k_pp_sparse(PPArgs A, const int2* __re
                 }
             }
             wave_lds_sync();
-            if (qtail > qhead) sparse_flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr, A.react_scale);
+            if (qtail > qhead) sparse_flush<kMode>(L, lane, qhead, qtail - qhead, Ka, Kr, scale);
+            sparse_drain(L, lane, sum, inv_scale);
             pa += (unsigned)qtail;
             if (sp == 0) pc -= (unsigned)ni;  // the particles themselves
-            if (vi && jslot == 0)
+            if (vi && jslot == 0) {  // (lane = islot)
+                int4 lo;
+                int* const l = &lo.x;
 #pragma unroll
                 for (int c = 0; c < 3; c++) {
                     unsigned long long* d = A.react + c * (size_t)A.cap + ia;
-                    if (splits > 1) atomicAdd(d, L.acc[islot][c]);
-                    else *d = L.acc[islot][c];
+                    const double v = sum[c] * (double)A.react_scale, hi = rint(v);
+                    l[c] = (int)rint((v - hi) * kLowScale);
+                    if (splits > 1) {
+                        atomicAdd(d, (unsigned long long)(long long)hi);
+                        atomicAdd(&A.low[ia].x + c, l[c]);
+                    } else {
+                        *d = (unsigned long long)(long long)hi;
+                    }
                 }
+                lo.w = 0;
+                if (splits == 1) A.low[ia] = lo;
+            }
             wave_lds_sync();  // acc, the queue and the list are reused
         }
         if (A.tile_pairs && lane == 0) {  // per-tile counts (on request only)
@@ -380,6 +411,12 @@ bool pp_sparse_fits(int rcp, float range, int ratio_cs) {
     return R < 512.0 && rcp + 3.0 * R < 512.0;
 }
 
+// Scale of the LDS sums: a component of a pair's force is below 10 / app^2 (as
+// in pp_prepare) and kDrainPairs of them stay below 2^62.
+float pp_sparse_scale(double app) {
+    return std::ldexp(1.0f, (int)std::floor(62.0 - std::log2(10.0 / (app * app) * kDrainPairs)));
+}
+
 // A coarse cell has up to kParts items and kParts more per kItemCount particles
 // around it; a slot is around 27 coarse cells.
 size_t pp_sparse_items(int64_t ncoarse, int64_t n_used) {
@@ -388,6 +425,8 @@ size_t pp_sparse_items(int64_t ncoarse, int64_t n_used) {
 
 int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoarse, int2* items,
                      size_t cap, int small, int mode, hipStream_t s) {
+    const float scale = pp_sparse_scale(ctx().g.p.app);
+    const double inv = 1.0 / (double)scale;
     if (ncoarse <= 0) return CUBE2_OK;
     Stage st("pp_pairs_sparse");
     int dev = 0, ncu = 0;
@@ -401,8 +440,8 @@ int launch_pp_sparse(const PPArgs& a, const int* rhoc, int nt, int ncb, int ncoa
     k_sparse_items<<<ceil_div((size_t)ncoarse, 256), 256, 0, s>>>(rhoc, nt, ncb, ncoarse, a.tiles, &a.red->err,
                                                                   (int)cap, items, count);
     C2_HIP(hipGetLastError());
-    if (mode == CUBE2_PP_REF) k_pp_sparse<kModeRef><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small);
-    else k_pp_sparse<kModeFast><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small);
+    if (mode == CUBE2_PP_REF) k_pp_sparse<kModeRef><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small, scale, inv);
+    else k_pp_sparse<kModeFast><<<blocks, 256, 0, s>>>(a, items, (int)cap, count, nt, small, scale, inv);
     C2_HIP(hipGetLastError());
     return CUBE2_OK;
 }

@@ -125,7 +125,8 @@ int cube2_set_pp_mode(int mode);
  *   PP_DIRECT_LG      1..7, chunks of > 2^(v-1) particles (lanes for >= 2^v
  *                     i slots) sum directly, smaller ones queue pairs (2);
  *                     where PP_NEWTON evaluates pairs once, cells of at most
- *                     2^(v-1) particles are taken by coarse cells instead;
+ *                     2^(v-1) particles (63 for 7) are taken by coarse cells
+ *                     instead;
  *   FFT_MIN_LGC       1..6, minimum log2 column-tile width of the y/z FFT
  *                     passes (built-in: ~2048 LDS elements per tile);
  *   INTERP_SEG        1..32, particles per wavefront work item of the mesh
@@ -150,7 +151,8 @@ int cube2_set_pp_mode(int mode);
  *                     evaluate each pair of two active particles of one
  *                     range once and add its force to both, summing in
  *                     64-bit fixed point at 2^k, k = min(40, floor(62 -
- *                     log2(10 cap / app^2))), cap the particle capacity
+ *                     log2(10 cap / app^2))), cap the particle capacity (the
+ *                     cells taken by coarse cells at 2^(k + 24))
  *                     (built-in; used when app > 0 and k >= 12, else as 2);
  *                     2: every ordered pair is evaluated by its i.
  * A change makes the next recorded kick record again. */
