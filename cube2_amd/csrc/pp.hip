@@ -747,6 +747,14 @@ __global__ void k_pp_check_total(const int* __restrict__ total, int64_t cap, PPR
     if (threadIdx.x == 0 && (int64_t)*total > cap) red->err |= 4;
 }
 
+// The learned kick evaluates pairs once from this k of the fixed-point scale
+// 2^k on: there the RMS error against a direct FP64 sum, of particles of forces
+// of order 1 to 10 in cells of 3 and more, is that of the ordered pass's FP32
+// sums (levels 3, 4 and 2; in units of 1e-6, k = 23, 22, 22: 6.44 to 6.44, 11.31
+// to 11.31, 9.28 to 9.39; 21, 20, 20: 6.46, 11.35, 9.52; 17, 16, 16: 10.4, 18.1,
+// 35.7).  256^3 particles with their halos at app 0.05: 23.
+constexpr int kLearnedLg = 22;
+
 int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* ratio_sf,
                int64_t n_used, PPPlan& P, bool split, bool learned) {
     ensure_params();
@@ -832,12 +840,14 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
     // below 2^62 for 2^k <= 2^62 / (10 / app^2 * cap); at 256^3 (app 0.06)
     // k = 24, a resolution of 6e-8 against forces of order 1 to 1e3.
     P.newton = false;
+    int react_lg = 0;
     if (pp_newton_on() && pp_newton_mode(P.mode) && g.p.app > 0.0) {
         const double bound = 10.0 / (g.p.app * g.p.app) * (double)P.cap;
         const int k = std::min(40, (int)std::floor(62.0 - std::log2(bound)));
         if (k >= 12) {
             P.newton = true;
             P.react_scale = std::ldexp(1.0f, k);
+            react_lg = k;
         }
     }
     // Small cells apart where a tile's grid is finer than its sparse subtiles
@@ -859,9 +869,10 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
         if (fine && fits) P.small = std::min((1 << pp_direct_lg()) / 2, 63);
         P.newton = !fine || fits;
         // learned: the network's cells hold more than `small` and are not
-        // subsorted, so that k_chunk_flags can mark them
+        // subsorted, so that k_chunk_flags can mark them; and its sums, FP32
+        // ones in the ordered pass, are no coarser (kLearnedLg)
         const int occ = learned_model_occupancy();
-        if (learned && (occ <= P.small || occ > 64)) {
+        if (learned && (occ <= P.small || occ > 64 || react_lg < kLearnedLg)) {
             P.newton = false;
             P.small = 0;
         }
