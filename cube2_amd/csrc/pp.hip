@@ -411,7 +411,10 @@ __global__ __launch_bounds__(256) void k_pp_ptotal(const int* __restrict__ rhoc,
 // of fewer than 16 particles have no chunk worth splitting)
 // Below kFewSlots slots there are few chunks for all the wavefronts, and a part
 // is a serial chain of its candidates (pair kernel with 2048, 256, 64 of them:
-// 3600 particles 95, 96, 57 us, 64^3 lattice 115, 114, 117).
+// 3600 particles 95, 96, 57 us, 64^3 lattice 115, 114, 117).  Each part rounds
+// its i's sums to the pass's fixed point, so that so many parts need a fine one
+// (kFineLg; error of forces of order 1 at 2^-13: 8.4e-5 in a part, 1.1e-4 in
+// parts of 64).
 constexpr int kPartCand = 2048, kPartFew = 64, kPartCount = 16, kFewSlots = 1 << 20;
 __global__ void k_chunk_flags(float4* __restrict__ rpos, const uint32_t* __restrict__ rslot,
                               const uint32_t* __restrict__ cellid,
@@ -747,13 +750,13 @@ __global__ void k_pp_check_total(const int* __restrict__ total, int64_t cap, PPR
     if (threadIdx.x == 0 && (int64_t)*total > cap) red->err |= 4;
 }
 
-// The learned kick evaluates pairs once from this k of the fixed-point scale
-// 2^k on: there the RMS error against a direct FP64 sum, of particles of forces
+// A fixed-point scale 2^k is fine from this k on (the learned kick evaluates pairs
+// once, chunks of small calls are split into short parts): there the RMS error against a direct FP64 sum, of particles of forces
 // of order 1 to 10 in cells of 3 and more, is that of the ordered pass's FP32
 // sums (levels 3, 4 and 2; in units of 1e-6, k = 23, 22, 22: 6.44 to 6.44, 11.31
 // to 11.31, 9.28 to 9.39; 21, 20, 20: 6.46, 11.35, 9.52; 17, 16, 16: 10.4, 18.1,
 // 35.7).  256^3 particles with their halos at app 0.05: 23.
-constexpr int kLearnedLg = 22;
+constexpr int kFineLg = 22;
 
 int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* ratio_sf,
                int64_t n_used, PPPlan& P, bool split, bool learned) {
@@ -870,9 +873,9 @@ int pp_prepare(const int* ires, const int* ixyz3, const float* apm3, const int* 
         P.newton = !fine || fits;
         // learned: the network's cells hold more than `small` and are not
         // subsorted, so that k_chunk_flags can mark them; and its sums, FP32
-        // ones in the ordered pass, are no coarser (kLearnedLg)
+        // ones in the ordered pass, are no coarser (kFineLg)
         const int occ = learned_model_occupancy();
-        if (learned && (occ <= P.small || occ > 64 || react_lg < kLearnedLg)) {
+        if (learned && (occ <= P.small || occ > 64 || react_lg < kFineLg)) {
             P.newton = false;
             P.small = 0;
         }
@@ -1175,7 +1178,7 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
                 n_sorted, &red->err, (int)P.cap, pp_dense_lg(P.newton),
                 P.small, A.learned_occ, A.learned_range, P.newton, A.tiles,
                 P.newton ? P.ntile : 0, g.p.ratio_cs,
-                P.n_used < kFewSlots ? kPartFew : kPartCand, flags, g_pp.dense.as<int>(),
+                P.n_used < kFewSlots && P.react_scale >= (float)(1 << kFineLg) ? kPartFew : kPartCand, flags, g_pp.dense.as<int>(),
                 &red->ndense, g_pp.pos4.as<float4>(), g_pp.slot.as<uint32_t>());
             C2_HIP(hipGetLastError());
             C2_TRY(exclusive_scan(flags, (int64_t)P.cap, g_pp.scan_tmp, s));
