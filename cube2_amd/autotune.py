@@ -13,16 +13,20 @@ import time
 
 from . import _lib
 
+# (which pair kernel runs comes before its grids: of the block counts, those up to
+# 8 per CU are the pairs-once kernel's, which takes parts from counters, the
+# others the ordered kernel's, whose blocks beyond the resident ones even out
+# its chunks' costs)
 CANDIDATES = {
-    "pp_blocks_per_cu": [0, 24, 48, 128],
-    "pp_overlap_blocks": [0, 32, 96],
+    "pp_newton": [0, 2],
+    "pp_blocks_per_cu": [0, 4, 8, 24, 48, 128],
+    "pp_overlap_blocks": [0, 2, 4, 6, 32, 96],
     "pp_dense_lg": [0, 4, 6],
     "pp_direct_lg": [0, 3, 1],
     "fft_min_lgc": [0, 3, 4],
     "interp_seg": [0, 2, 8],
     "pp_order": [0, 20],
     "pp_jbatch": [0, 2],
-    "pp_newton": [0, 2],
 }
 
 
