@@ -47,16 +47,6 @@ struct LearnedBufs {
 };
 static LearnedBufs g_lb;
 
-__device__ inline int find_tile_l(const PPTile* __restrict__ T, int ntile, uint32_t c) {
-    int lo = 0, hi = ntile - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (T[mid].cell_off <= (long long)c) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // Fine-cell input of the jobs [j0, j0 + nj): count and offset sums, from
 // every sorted particle (physical and halo copies) of each job's tile that
 // falls inside its grid of DI^3 cells (fine cell o - kLMargin + index).
@@ -111,7 +101,7 @@ __device__ inline int learned_job_of(const PPArgs& A, const LearnedArgs& L, int 
     if (fabsf(p.w) != L.range) return -1;  // (w < 0: pairs-once small cell)
     const uint32_t cid = A.cellid[a];
     if (A.cell_start[cid + 1] - A.cell_start[cid] >= L.occupancy) return -1;
-    const int t = find_tile_l(A.tiles, A.ntile, cid);
+    const int t = pp_find_tile(A.tiles, A.ntile, cid);
     const int sx = min((int)floorf(p.x / L.sub_std), L.nns - 1);
     const int sy = min((int)floorf(p.y / L.sub_std), L.nns - 1);
     const int sz = min((int)floorf(p.z / L.sub_std), L.nns - 1);

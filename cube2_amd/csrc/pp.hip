@@ -520,13 +520,7 @@ __global__ __launch_bounds__(kOrderBins) void k_chunk_cost(PPArgs A, const int* 
         const int ni = min(cend - cbeg >= 64 ? 1 << dense_lg : 64, cend - a0);
         int I = 1;
         while (I < ni) I <<= 1;
-        int lo = 0, hi = A.ntile - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (A.tiles[mid].cell_off <= (long long)cid) lo = mid;
-            else hi = mid - 1;
-        }
-        const int rcp = A.tiles[lo].rcp;
+        const int rcp = A.tiles[pp_find_tile(A.tiles, A.ntile, cid)].rcp;
         const int W = 2 * (int)ceilf(fabsf(A.pos4[a0].w) * (float)rcp / (float)A.ratio_cs) + 1;
         const float cost = (float)(I + 1) * (float)(cend - cbeg) * (float)(W * W * W);
         const int k = min(kOrderBins - 1, (int)(8.0f * log2f(cost + 1.0f)));
@@ -607,13 +601,7 @@ __global__ __launch_bounds__(256) void k_pp_subsort(
     for (int qc = blockIdx.x * kWaves + wave; qc < ndense; qc += gridDim.x * kWaves) {
     const uint32_t cid = (uint32_t)dense_list[qc];
     const int c0 = cell_start[cid], c1 = cell_start[cid + 1];
-    int lo = 0, hi = ntile - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (tiles[mid].cell_off <= (long long)cid) lo = mid;
-        else hi = mid - 1;
-    }
-    const PPTile T = tiles[lo];
+    const PPTile T = tiles[pp_find_tile(tiles, ntile, cid)];
     const long long key = (long long)cid - T.cell_off;
     const int S = T.S;
     const int kx = (int)(key % S), ky = (int)((key / S) % S), kz = (int)(key / ((long long)S * S));
@@ -1187,7 +1175,7 @@ int pp_enqueue(const PPPlan& P, const int* d_rhoc, const int64_t* d_idx, const i
         }
         {
             Stage st("pp_subsort", (double)P.n_used * 24);
-            // one wavefront per chunk (only first chunks of dense cells work)
+            // (wavefronts stride over the dense cells)
             k_pp_subsort<<<(unsigned)std::max(1, pp_tiled_grid(false)), 256, 0, s>>>(
                 g_pp.raw_pos4.as<float4>(), g_pp.raw_slot.as<uint32_t>(), A.cell_start, A.tiles,
                 P.ntile, g_pp.dense.as<int>(), &red->ndense, g.p.ratio_cs, g_pp.pos4.as<float4>(),

@@ -1,5 +1,5 @@
-// The pair force laws of the PP pair kernels (pp_tiled.hip, pp_sparse.hip):
-// the arithmetic of each mode is described at the head of pp_tiled.hip.
+// The pair force laws of the PP pair kernels (pp_tiled.hip, pp_newton.hip,
+// pp_sparse.hip): the arithmetic of each mode is described at the head of pp_tiled.hip.
 #pragma once
 #include "common.h"
 #include "pp_kernels.h"
@@ -20,31 +20,11 @@ __device__ inline double recip_refine(double x, double y0) {
     return fma(fma(e, e, e), y0, y0);
 }
 
-// FP64 reciprocal of a float: v_rcp_f64 and one cubic refinement.  The
-// self-test checks |1 - x*y| <= 2^-51 for every float x with exponent in
-// [-40, 40].
-__device__ inline double recip64(double x) { return recip_refine(x, __builtin_amdgcn_rcp(x)); }
-
 __device__ inline float div_by(float a, double y) { return (float)((double)a * y); }
 
-// RN(sqrt(x)) for normal positive finite x (pair distances: r^2 >= 2^-28,
-// the positions being multiples of ratio_cs * 2^-16 apart).  v_sqrt_f32 is
-// within one ulp; of s and its neighbours s-, s+ the rounding test keeps s-
-// if x <= s- * s and s+ if x > s * s+ (FMA residuals, exact in sign: the
-// residuals are integer multiples of ulp^2 and midpoints squared are not).
-// No scaling or special-value fix-ups, which only zero, infinities, NaNs and
-// tiny inputs need.  The self-test checks it against IEEE sqrtf for every
-// float with exponent in [-40, 40].
-__device__ inline float sqrt_rn(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float lo = __int_as_float(__float_as_int(s) - 1);
-    const float hi = __int_as_float(__float_as_int(s) + 1);
-    float r = fmaf(-lo, s, x) <= 0.0f ? lo : s;
-    r = fmaf(-hi, s, x) > 0.0f ? hi : r;
-    return r;
-}
-
-// RN(sqrt(x)) and an FP64 reciprocal of it from one v_rsq_f32.  With y =
+// RN(sqrt(x)) and an FP64 reciprocal of it from one v_rsq_f32, for normal
+// positive finite x (pair distances: the positions are multiples of ratio_cs *
+// 2^-16 apart).  With y =
 // rsq(x), g = x y is within a few ulps of sqrt(x), its residual d = x - g^2 is
 // exact in an FMA, and g + d y/2 differs from sqrt(x) by about 2^-45, so that
 // its rounding could only err where sqrt(x) lies that close to a midpoint;

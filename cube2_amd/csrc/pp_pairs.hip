@@ -16,16 +16,6 @@
 
 namespace cube2 {
 
-__device__ inline int find_tile(const PPTile* __restrict__ T, int ntile, uint32_t c) {
-    int lo = 0, hi = ntile - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (T[mid].cell_off <= (long long)c) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // basic_functions.f08:95-109, term for term (no contraction).
 __device__ inline float fra_exact(float r, float apm) {
 #pragma clang fp contract(off)
@@ -102,7 +92,7 @@ __global__ __launch_bounds__(256) void k_pp_pairs(PPArgs A) {
     if (a < n) p = A.pos4[a];
     if (p.w > 0.0f) {
         const uint32_t cid = A.cellid[a];
-        const PPTile T = A.tiles[find_tile(A.tiles, A.ntile, cid)];
+        const PPTile T = A.tiles[pp_find_tile(A.tiles, A.ntile, cid)];
         const long long key = (long long)cid - T.cell_off;
         const int S = T.S;
         const int x = (int)(key % S), y = (int)((key / S) % S), z = (int)(key / ((long long)S * S));
@@ -168,7 +158,7 @@ __global__ __launch_bounds__(256) void k_pp_pairs(PPArgs A) {
         pc -= 1;  // the particle itself
         pp_update(A, a, ax, ay, az, f2, v0, v1, v2);
         if (A.tile_pairs) {  // per-tile counts (on request only)
-            const int ti = find_tile(A.tiles, A.ntile, cid);
+            const int ti = pp_find_tile(A.tiles, A.ntile, cid);
             atomicAdd(&A.tile_pairs[2 * ti], pc);
             atomicAdd(&A.tile_pairs[2 * ti + 1], pa);
         }

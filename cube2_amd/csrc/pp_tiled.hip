@@ -77,16 +77,6 @@ __device__ inline void flush(WaveLDS<kMode, kJB>& L, int lane, int begin, int co
     wave_lds_sync();
 }
 
-__device__ inline int find_tile2(const PPTile* __restrict__ T, int ntile, uint32_t c) {
-    int lo = 0, hi = ntile - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (T[mid].cell_off <= (long long)c) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
 // Wavefront w of the grid takes chunks w, w + W, w + 2W, ... (W = waves in
 // the grid); the chunk count is read on the device.  Chunk-level values are
 // kept wavefront-uniform (scalar registers), and the register budget is
@@ -127,7 +117,7 @@ __global__ __launch_bounds__(256, kMode >= kModePrecise ? 5 : 6) void k_pp_tiled
         const bool vi = islot < ni;
         const int ia = a0 + (vi ? islot : 0);
         const float4 p = A.pos4[ia];
-        const int ti = uni(find_tile2(A.tiles, A.ntile, cid));
+        const int ti = uni(pp_find_tile(A.tiles, A.ntile, cid));
         const PPTile T = A.tiles[ti];
         unsigned ncand = 0;  // (wavefront-uniform)
         const int S = T.S;
@@ -501,6 +491,9 @@ int pair_forces_debug(int mode, const float* pairs, int n, float app, float* for
     return CUBE2_OK;
 }
 
+// FP64 reciprocal of a float that is no root: v_rcp_f64 and one cubic refinement.
+__device__ inline double recip64(double x) { return recip_refine(x, __builtin_amdgcn_rcp(x)); }
+
 // --- arithmetic self-test: the reciprocal-based quotients of the
 // reference-arithmetic kernel against IEEE float division.
 // seed != 0: n seeded random operands (a, b with exponents in [-40, 40],
@@ -508,7 +501,8 @@ int pair_forces_debug(int mode, const float* pairs, int n, float app, float* for
 // [-40, 40] (n = 81 * 2^23) as b and r, with a = l = 1.  Checked: a/b,
 // 12/b, |1 - b*recip64(b)| <= 2^-51, 1/RN(r*r) refined from (1/r)^2, and
 // 12/e2 for ep = RN(2r/l), e2 = RN(ep*ep) refined from (l/2)^2 (1/r)^2, and
-// sqrt_rn(b) and sqrt_recip(b) against IEEE sqrtf, and the latter's reciprocal.
+// sqrt_recip(b) against IEEE sqrtf, its reciprocal, and the pair law's quotients by
+// it: a/root and 1/RN(root*root).
 __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
@@ -532,10 +526,12 @@ __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
         r = mk((int)(nxt() % 41) - 20, nxt());
         l = mk((int)(nxt() % 41) - 20, nxt());
     }
-    float ieee, ieee12, ieee_rr, ieee_t12, p, ep, e2, ieee_sqrt;
+    float ieee, ieee12, ieee_rr, ieee_t12, p, ep, e2, ieee_sqrt, ieee_q, ieee_q2;
     {
 #pragma clang fp contract(off)
         ieee_sqrt = sqrtf(b);
+        ieee_q = a / ieee_sqrt;
+        ieee_q2 = 1.0f / (ieee_sqrt * ieee_sqrt);
         ieee = a / b;
         ieee12 = 12.0f / b;
         p = r * r;
@@ -551,7 +547,10 @@ __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
     double inv_s;
     const float root = sqrt_recip(b, inv_s);
     const bool root_ok = __float_as_uint(root) == __float_as_uint(ieee_sqrt) &&
-                         fabs(fma(-(double)root, inv_s, 1.0)) <= 0x1p-51;
+                         fabs(fma(-(double)root, inv_s, 1.0)) <= 0x1p-51 &&
+                         __float_as_uint(div_by(a, inv_s)) == __float_as_uint(ieee_q) &&
+                         __float_as_uint((float)recip_refine((double)(root * root), inv_s * inv_s)) ==
+                             __float_as_uint(ieee_q2);
     const double inv_r = recip64((double)r);
     const float rr = (float)recip_refine((double)p, inv_r * inv_r);
     const float ep2 = div_by(2.0f * r, 1.0 / (double)l);
@@ -560,8 +559,7 @@ __global__ void k_selftest_div(uint64_t seed, int n, unsigned long long* bad) {
     if (__float_as_uint(ieee) != __float_as_uint(mine) ||
         __float_as_uint(ieee12) != __float_as_uint(twelve) || !resid ||
         __float_as_uint(ieee_rr) != __float_as_uint(rr) || __float_as_uint(ep) != __float_as_uint(ep2) ||
-        __float_as_uint(ieee_t12) != __float_as_uint(t12) ||
-        __float_as_uint(ieee_sqrt) != __float_as_uint(sqrt_rn(b)) || !root_ok)
+        __float_as_uint(ieee_t12) != __float_as_uint(t12) || !root_ok)
         atomicAdd(bad, 1ull);
 }
 
