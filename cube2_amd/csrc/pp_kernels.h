@@ -107,7 +107,8 @@ __device__ inline int pp_find_tile(const PPTile* __restrict__ T, int ntile, uint
 // Pairs-once pair kernel (pp_newton.hip) over the parts of the chunks:
 // chunks[k] is the chunk of part k, first[a] the first part of chunk a;
 // first[cap] is their number; they are taken in the order of the list or of
-// a.order.  help: a second launch that joins the first.  Cells of at most `small` particles are k_pp_sparse's (0: none).
+// a.order.  help: a second launch that joins the first.  Cells of at most
+// `small` particles are k_pp_sparse's (0: none).
 int launch_pp_newton(const PPArgs& a, const int* chunks, const int* first, int grid, int small,
                      int mode, bool help, hipStream_t s);
 

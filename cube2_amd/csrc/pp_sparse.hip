@@ -22,7 +22,9 @@
 // and nothing else adds to them (k_chunk_flags marks them), so their sums are
 // stored, not added, unless their j are split; what the pass's scale cannot hold
 // of them goes to `low`.
-// Bound by VALU issue: the region's tests.  The particles beside a clump cost
+// Bound by the chains of row and batch loads of each region: 0.16 VALU and 0.14
+// scalar instructions per SIMD cycle, half of the wavefronts' time waiting, 1.3
+// TB/s (7.3-8.0 ms alone at 256^3).  The particles beside a clump cost
 // the most by far, one batch of them up to 1 ms, and the kernel waits for the
 // last: k_sparse_items shares a coarse cell among wavefronts and lists the
 // costly ones first.  REF, clustered, ms at 256^3 / 128^3 / 120^3 in level-6

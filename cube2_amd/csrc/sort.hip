@@ -1,19 +1,19 @@
 // Stable LSD radix sort of 32-bit (key, value) pairs: ceil(end_bit / 11)
 // passes of equal digit widths (at most 11 bits, 2048 digits).
 //
-// A pass splits the n pairs into contiguous segments, one per block.  k_sort_hist counts each segment's digits in LDS and stores the
-// counts digit-major ([digit][block]), so that one exclusive scan of them
-// gives every (digit, block) its first output position: all pairs of a
-// smaller digit first, and within a digit the segments in order.  The
-// scatter (k_sort_scatter) walks its segment 256 pairs at a time in input
-// order; a pair's place is its (digit, block) base, the pairs of its digit in
-// the earlier wavefronts of the step, and its rank among its own
-// wavefront's lanes of that digit, found with one ballot per digit bit.
-// Equal digits thus keep their input order (stability), which makes the
-// passes compose into a sort by the whole key.  Only the first lane of each
-// digit's group in a wavefront touches the LDS counts, so nearly sorted
-// input (the drift's) does not serialise on one address, and a step costs
-// the same whatever the digit width.
+// A pass splits the n pairs into contiguous segments, one per block.
+// k_sort_hist counts each segment's digits in LDS and stores the counts
+// digit-major ([digit][block]), so that one exclusive scan of them gives every
+// (digit, block) its first output position: all pairs of a smaller digit first,
+// and within a digit the segments in order.  The scatter (k_sort_scatter) walks
+// its segment 256 pairs at a time in input order; a pair's place is its (digit,
+// block) base, the pairs of its digit in the earlier wavefronts of the step,
+// and its rank among its own wavefront's lanes of that digit, found with one
+// ballot per digit bit.  Equal digits thus keep their input order (stability),
+// which makes the passes compose into a sort by the whole key.  Only the first
+// lane of each digit's group in a wavefront touches the LDS counts, so nearly
+// sorted input (the drift's) does not serialise on one address, and a step
+// costs the same whatever the digit width.
 #include "sort.h"
 
 #include <algorithm>
