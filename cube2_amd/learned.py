@@ -107,8 +107,9 @@ class LearnedPP:
         B, D = dout.shape[0], self.acts[0].shape[1]
         if D <= PATCH and B:  # training patches: no im2col
             grads = [(torch.empty_like(w), torch.empty_like(b)) for w, b in zip(self.W, self.b)]
-            # (its size checked by the reshape) held until the call returns
-            dout = dout.reshape(B * (D - 8) ** 3, CHANNELS[4]).contiguous()
+            if dout.numel() != B * (D - 8) ** 3 * CHANNELS[4]:
+                raise RuntimeError(f"gradient of shape {tuple(dout.shape)} for {B} patches of {D}^3")
+            dout = dout.contiguous()  # held until the call returns
             _lib.check(L.cube2_cnn_net_backward_dev(_ps(self.acts), _ps(self.Wb), _p(dout), B, D,
                                                     _ps([g[0] for g in grads]),
                                                     _ps([g[1] for g in grads])))
