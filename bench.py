@@ -660,7 +660,9 @@ def main(argv=None) -> int:
         achieved = flops / (pp_ms * 1e-3) / 1e12
         roof = dict(kernel=name, bound="valu", achieved=round(achieved, 3),
                     peak=FP32_PEAK_TFLOPS, unit="TFLOP/s",
-                    frac=round(achieved / FP32_PEAK_TFLOPS, 4), traffic=profiled_traffic(name),
+                    frac=round(achieved / FP32_PEAK_TFLOPS, 4),
+                    # (measured on the pairs-once kernels, whose pass the small cells' stage tells)
+                    traffic=profiled_traffic(name) if "pp_pairs_sparse" in stats else None,
                     avg_launch_ms=round(per_launch_ms, 3))
     else:
         achieved = st["bytes"] / (st["ms"] * 1e-3) / 1e9
